@@ -90,16 +90,18 @@ struct GemmArgs {
 
 constexpr int kMaxKB = 256;                 // reduction length limit: 256 * 128 = 32768
 
-template <int MT, int NW, int STAGES, int WSTAGES, int WTILE = 2048, int TPS = 16>
+// SAC: there are activation scales (their pieces of the small-tile kernels' LDS are what lets two or three workgroups
+// share a compute unit, so the 16-bit modes do not carry them there)
+template <int MT, int NW, int STAGES, int WSTAGES, int WTILE = 2048, int TPS = 16, bool SAC = true>
 struct GemmSmem {
   static constexpr int BM = 16 * MT;
   alignas(1024) uint8_t wt[WSTAGES][TPS * WTILE];   // weight tiles: [tile][row][swizzled 16-byte chunk], read by their owner
   alignas(1024) uint8_t tok[STAGES][BM * 128];   // token tiles, XOR-swizzled 16-byte chunks
-  alignas(1024) float sac[2][MT * 256];          // activation scales, 16 steps at a time: [m-tile][4-step part][row][4]
+  alignas(1024) float sac[2][SAC ? MT * 256 : 4];   // activation scales, 16 steps at a time: [m-tile][4-step part][row][4]
   int arow[BM];                                  // source row in aq / as for each tile row
   int oslot[BM];                                 // second GEMM: output row of each tile row
   float amax[NW][BM];                            // GATED epilogue: per-wavefront partial amax
-  float2 fsc[4][BM];                             // large tiles: scale products of four steps, one pair per tile row
+  float2 fsc[4][SAC ? BM : 1];                   // large tiles: scale products of four steps, one pair per tile row
   float sb[2][kMaxKB + 4];                       // weight-block scales of the strip for every 128-step, then zeros
 };
 
@@ -174,7 +176,8 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   constexpr int NT = 64 * NW;                         // threads
   constexpr int WT = TPS / NW;                        // weight tiles per wavefront
   constexpr int STAGES = WREG ? 4 : DEPTH + 1;        // token tiles staged in LDS
-  using Smem = GemmSmem<MT, NW, STAGES, WREG ? 1 : STAGES, WREG ? 64 : 2048, TPS>;
+  constexpr int WLDS = DQ ? 1024 : 2048;              // bytes of a weight tile's step in LDS (DQ: one half of a block)
+  using Smem = GemmSmem<MT, NW, STAGES, WREG ? 1 : STAGES, WREG ? 64 : WLDS, TPS, WREG || !BF16>;
   static_assert(sizeof(Smem) <= 160 * 1024, "one workgroup's LDS");
   __shared__ Smem sm;
 
@@ -331,7 +334,8 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   for (int u = 0; u < NTOK; u++) {
     const int t = min(wave * NTOK + u, NROW8 - 1);
     const int row = 8 * t + (lane >> 3);
-    const int c = (lane & 7) ^ (lane >> 3);
+    int c = (lane & 7) ^ (lane >> 3);
+    if (DQ) c = c < 4 ? 2 * c : 2 * c - 7;             // (see tok_chunk0)
     // row-groups past the tile's last row are never read by a matrix instruction that matters:
     // every lane fetches the same 16 bytes there, which costs one cache line instead of eight
     tok_src[u] = 8 * t < rows ? (uint32_t)sm.arow[row] * (uint32_t)a.Kd + c * 16 : (uint32_t)sm.arow[0] * (uint32_t)a.Kd;
@@ -350,8 +354,8 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     sac_src[u] = (uint32_t)sm.arow[mt * 16 + li] * (uint32_t)a.as_pitch * 4u + lg * 16;   // bytes
     sac_m0[u] = mt * 1024;
   }
-  const uint32_t wt_base = __builtin_amdgcn_readfirstlane(lds_offset(&sm.wt[0][0])) + wave * (WT * 2048);
-  constexpr uint32_t kWtStage = TPS * 2048;
+  const uint32_t wt_base = __builtin_amdgcn_readfirstlane(lds_offset(&sm.wt[0][0])) + wave * (WT * WLDS);
+  constexpr uint32_t kWtStage = TPS * WLDS;
   const uint32_t tok_base = __builtin_amdgcn_readfirstlane(lds_offset(&sm.tok[0][0]));
   const uint32_t sac_base = __builtin_amdgcn_readfirstlane(lds_offset(&sm.sac[0][0]));
   constexpr uint32_t kTokStage = BM * 128, kSacBuf = MT * 1024;
@@ -375,13 +379,23 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   constexpr int LPT = DQ ? 1 : 2;                      // load instructions per weight tile and step (1 KB each)
   constexpr int WSTEP = 1024 * LPT;                    // bytes of a tile's step in memory
   constexpr int L_STEP = NTOK + LPT * WT;              // loads per wavefront and step (scale chunks come on top)
-  v4i wlo[WREG ? DEPTH : 1][WT], whi[WREG ? DEPTH : 1][WT];   // WREG: weight fragments ride in a register ring
+  // WREG: weight fragments ride in a register ring of R steps.  DQ: a step of codes is half as many bytes, so the ring
+  // is twice as long for as much in flight (the half tile's four weight tiles per wavefront leave no registers for that)
+  constexpr int R = DQ && NW == 8 ? 2 * DEPTH : DEPTH;
+  v4i wlo[WREG ? R : 1][WT], whi[WREG ? R : 1][WT];
+  if constexpr (WREG && DQ) {
+#pragma unroll
+    for (int d = 0; d < R; d++)
+#pragma unroll
+      for (int j = 0; j < WT; j++) wlo[d][j] = (v4i){0, 0, 0, 0};
+  }
   auto request_weights_reg = [&](int kb, v4i(&lo)[WT], v4i(&hi)[WT]) {
 #pragma unroll
     for (int j = 0; j < WT; j++) {
       const uint8_t *base = wtile[j] + (size_t)kb * WSTEP;
       if constexpr (DQ)
-        asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(lo[j]) : "v"(woff), "s"(base) : "memory");
+        // tied to the slot's register: a free choice per request made the compiler move slots while loads are in flight
+        asm volatile("global_load_dwordx4 %0, %1, %2" : "+v"(lo[j]) : "v"(woff), "s"(base) : "memory");
       else
         asm volatile("global_load_dwordx4 %0, %2, %3\n\tglobal_load_dwordx4 %1, %2, %3 offset:1024"
                      : "=&v"(lo[j]), "=&v"(hi[j]) : "v"(woff), "s"(base) : "memory");
@@ -420,7 +434,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
 #pragma unroll
         for (int j = 0; j < WT; j++) {
           const uint8_t *base = wtile[j] + (size_t)kb * WSTEP;
-          const uint32_t m0 = wt_base + stage * kWtStage + j * 2048;
+          const uint32_t m0 = wt_base + stage * kWtStage + j * WLDS;
           if constexpr (DQ)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(m0), "v"(woff), "s"(base) : "memory", "m0");
           else
@@ -432,7 +446,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
 #pragma unroll
         for (int j = 0; j < WT; j++) {
           const uint8_t *base = wtile[j] + (size_t)kb * WSTEP;
-          const uint32_t m0 = wt_base + stage * kWtStage + j * 2048;
+          const uint32_t m0 = wt_base + stage * kWtStage + j * WLDS;
           if constexpr (DQ)
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(m0), "v"(woff), "s"(base) : "memory", "m0");
           else
@@ -446,9 +460,11 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
 
   // Which two 16-byte chunks of a token row's 128-byte step a lane reads (positions XOR-swizzled by the row).  FP8 and
   // bf16 operands: chunks g and g + 4, conflict-free for 128-bit LDS reads, and the weights are stored to match.  DQ:
-  // the lane's 16 weight codes are reduction elements 16g..16g+15 of the step, bytes 32g..32g+31 of the token row.
-  auto tok_chunk0 = [](int g, int i) { return ((DQ ? 2 * g : g) ^ (i & 7)) << 4; };
-  auto tok_chunk1 = [](int g, int i) { return ((DQ ? 2 * g + 1 : g + 4) ^ (i & 7)) << 4; };
+  // the lane's 16 weight codes are reduction elements 16g..16g+15 of the step, bytes 32g..32g+31 of the token row; its
+  // chunks 2g and 2g + 1 are laid down where the other modes keep g and g + 4 (the request fetches them in that order):
+  // read in place they met in the same banks two by two.
+  auto tok_chunk0 = [](int g, int i) { return (g ^ (i & 7)) << 4; };
+  auto tok_chunk1 = [](int g, int i) { return ((g + 4) ^ (i & 7)) << 4; };
   // m-tiles are processed in groups of up to four; a group is skipped when it holds no row.  A
   // group first issues all of its LDS reads (one exposed LDS latency per group, not per tile),
   // then its matrix instructions back to back, each tile's scale multiply-adds trailing the
@@ -456,17 +472,17 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   constexpr int MG = MT < 4 ? MT : (MT % 4 == 0 && MT <= 8 ? 4 : (DEPTH >= 3 ? 2 : 3));
   auto compute = [&](int stage, int kb, const v4i(&lo)[WT], const v4i(&hi)[WT]) {
     v8i wc[WT];
-    const uint8_t *wbase = sm.wt[WREG ? 0 : stage] + wave * (WT * 2048) + lane * 16;
+    const uint8_t *wbase = sm.wt[WREG ? 0 : stage] + wave * (WT * WLDS) + lane * 16;
     const float s0 = BF16 && !DQ ? 0.f : sm.sb[sb_row0][kb], s1 = BF16 && !DQ ? 0.f : sm.sb[sb_row1][kb];
 #pragma unroll
     for (int j = 0; j < WT; j++) {
-      if constexpr (DQ) wc[j] = dequant16(WREG ? lo[j] : *(const v4i *)(wbase + j * 2048), (GATED && j >= WT / 2) ? s1 : s0);
+      if constexpr (DQ) wc[j] = dequant16(WREG ? lo[j] : *(const v4i *)(wbase + j * WLDS), (GATED && j >= WT / 2) ? s1 : s0);
       else if (WREG) wc[j] = concat8(lo[j], hi[j]);
       else wc[j] = concat8(*(const v4i *)(wbase + j * 2048), *(const v4i *)(wbase + j * 2048 + 1024));
     }
     const uint8_t *tbase = sm.tok[stage] + li * 128;
     const int o0 = tok_chunk0(lg, li), o1 = tok_chunk1(lg, li);
-    const float *sap = sm.sac[(kb >> 4) & 1] + ((kb & 12) << 4) + li * 4 + (kb & 3);
+    const float *sap = BF16 ? nullptr : sm.sac[(kb >> 4) & 1] + ((kb & 12) << 4) + li * 4 + (kb & 3);
 #pragma unroll
     for (int mg = 0; mg < MT / MG; mg++) {
       if (mg == 0 || mg * MG < mt_live) {
@@ -558,9 +574,9 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     // an odd count multiplies by the zero weight scale stored behind the table.  The loop body is
     // instantiated per number of live m-tiles, so there is no branch between matrix instructions.
     static_assert(DEPTH == 2, "the register ring holds two steps");
-    constexpr int R = DEPTH;                             // ring slots = steps per pass of the unrolled loop
+    // R ring slots = steps per pass of the unrolled loop
     constexpr int XB = 4;                                // token operand buffers; R * LIVE is a multiple of it
-    constexpr int L_WAIT = NTOK + LPT * WT * (R - 1);    // loads younger than the ones a step boundary needs
+    constexpr int L_WAIT = NTOK + LPT * WT * (R / 2);    // loads younger than the ones a step boundary needs
     const int last = NKB - 1;
     const int o0 = tok_chunk0(lg, li), o1 = tok_chunk1(lg, li);
     auto run = [&](auto live_c) {
@@ -572,12 +588,33 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
       // load's request and its wait (the compiler would copy the registers while the load is in flight)
       request(0, 0);
       request(min(1, last), 1);
-      request_weights_reg(0, wlo[0], whi[0]);
-      request(min(2, last), 2);
+      // DQ: the operands of a step are made from its codes during the step before, a piece with each m-tile, so that
+      // the conversions run beside matrix instructions; codes are asked for a step earlier to match.  A step's codes
+      // sit in ring slot (step % R), its operands in wdq[step % 2].
+      // A wavefront's 64 conversion instructions at the top of the step held up its matrix instructions; with that, the
+      // banks of tok_chunk0 and the longer ring the Mixtral-shaped layer at 333 tokens takes 437 -> 420 us (476 -> 453 on
+      // another card; the conversions and banks alone 451 -> 430), at 1500 tokens 1199 -> 1160, whose first product then
+      // runs at 1.07 PFLOP/s of the 1.24 that a large library product in bf16 reaches here.
+      v8i wdq[DQ ? 2 : 1][WT];
+      if constexpr (DQ) {
 #pragma unroll
-      for (int d = 1; d < R; d++) request_weights_reg(min(d, last), wlo[d], whi[d]);
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L_WAIT) : "memory");
-      arrived_weights(wlo[0], whi[0]);
+        for (int d = 0; d < R; d++) request_weights_reg(min(d, last), wlo[d], whi[d]);
+        request(min(2, last), 2);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NTOK + LPT * WT * (R - 1)) : "memory");
+        arrived_weights(wlo[0], whi[0]);
+#pragma unroll
+        for (int j = 0; j < WT; j++) wdq[0][j] = dequant16(wlo[0][j], sm.sb[(GATED && j >= WT / 2) ? sb_row1 : sb_row0][0]);
+        request_weights_reg(min(R, last), wlo[0], whi[0]);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L_WAIT) : "memory");
+        arrived_weights(wlo[1], whi[1]);
+      } else {
+        request_weights_reg(0, wlo[0], whi[0]);
+        request(min(2, last), 2);
+#pragma unroll
+        for (int d = 1; d < R; d++) request_weights_reg(min(d, last), wlo[d], whi[d]);
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L_WAIT) : "memory");
+        arrived_weights(wlo[0], whi[0]);
+      }
       __syncthreads();
       if (n_chunks > 1) request_scales(1);
       // Scale products: what a lane multiplies a matrix-instruction result with is (activation scale
@@ -626,9 +663,10 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
           v8i wc[WT];
 #pragma unroll
           for (int j = 0; j < WT; j++) {
-            if constexpr (DQ) wc[j] = dequant16(wlo[h][j], sm.sb[(GATED && j >= WT / 2) ? sb_row1 : sb_row0][kb]);
+            if constexpr (DQ) wc[j] = wdq[h & 1][j];
             else wc[j] = concat8(wlo[h][j], whi[h][j]);
           }
+          const float sn0 = DQ ? sm.sb[sb_row0][kb + 1] : 0.f, sn1 = DQ ? sm.sb[sb_row1][kb + 1] : 0.f;   // the next step's
           // one m-tile: LDS reads two m-tiles ahead, its matrix instructions, then the multiply-adds
           // of the m-tile before it (tp), whose products are complete by now
           // m-tiles are walked from the last live one down to 0 so that the m-tile whose products are
@@ -653,6 +691,18 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
             if (q == LIVE / 2) produce_f(kb + 3);
             if constexpr (BF16) {                        // accumulates in place: nothing is pending afterwards
               if (q != 0 || !top_empty) mma_bf16<WT>(acc[LIVE - 1 - q], wc, x[g % XB]);
+              if constexpr (DQ) {
+#pragma unroll
+                for (int c = 0; c < 4 * WT; c++)         // a piece: four codes
+                  if (c * LIVE / (4 * WT) == q) {
+                    const int j = c >> 2, i = c & 3;
+                    const float s = (GATED && j >= WT / 2) ? sn1 : sn0;
+                    const v2f_t a2 = __builtin_amdgcn_cvt_pk_f32_fp8(wlo[(h + 1) % R][j][i], false);
+                    const v2f_t b2 = __builtin_amdgcn_cvt_pk_f32_fp8(wlo[(h + 1) % R][j][i], true);
+                    wdq[(h + 1) & 1][j][2 * i] = (int)pack2_bf16(a2[0] * s, a2[1] * s);
+                    wdq[(h + 1) & 1][j][2 * i + 1] = (int)pack2_bf16(b2[0] * s, b2[1] * s);
+                  }
+              }
               __builtin_amdgcn_sched_barrier(0);
               return;
             }
@@ -684,9 +734,15 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
 #pragma unroll
           for (int q = 1; q < LIVE; q++) tile(q, LIVE - q);
           // top of step kb + 1
-          request_weights_reg(min(kb + R, last), wlo[h], whi[h]);
-          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L_WAIT) : "memory");
-          arrived_weights(wlo[(h + 1) % R], whi[(h + 1) % R]);
+          if constexpr (DQ) {                            // the codes of step kb + 1 have just been converted
+            request_weights_reg(min(kb + R + 1, last), wlo[(h + 1) % R], whi[(h + 1) % R]);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L_WAIT) : "memory");
+            arrived_weights(wlo[(h + 2) % R], whi[(h + 2) % R]);
+          } else {
+            request_weights_reg(min(kb + R, last), wlo[h], whi[h]);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L_WAIT) : "memory");
+            arrived_weights(wlo[(h + 1) % R], whi[(h + 1) % R]);
+          }
           __syncthreads();
           if (((kb + 1) & 15) == 0 && ((kb + 1) >> 4) + 1 < n_chunks) request_scales(((kb + 1) >> 4) + 1);
           __builtin_amdgcn_sched_barrier(0);
@@ -711,7 +767,9 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
       else if (mt_live <= LIVE) run(live_c);
       else self(self, std::integral_constant<int, LIVE + 2>{});
     };
-    pick(pick, std::integral_constant<int, 2>{});
+    // (with the long ring of DQ the body for two m-tiles is left out: the compiler moves a ring slot at the end of that
+    // body's loop while the slot's load is in flight, which the static check of the assembly refuses)
+    pick(pick, std::integral_constant<int, (R > 2 ? 4 : 2)>{});
   }
   __syncthreads();
 
