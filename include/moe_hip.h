@@ -249,11 +249,11 @@ int moe_fused_experts_w8a16(void *stream, const void *x_bf16, int T, int H, cons
  * moe_mm_fp8 replaces at::mm_w8a16_dq_forward -> tpudnnMmW8A16DqAsync
  * (torch_tpu/csrc/ops/my_ops/MmW8A16Dq.cpp:185-228): out [M, N] bf16 = x [M, K] bf16 times the
  * transpose of w [N, K] fp8 with fp32 scales [ceil(N/128), K/128].  K a multiple of 128, N a
- * multiple of 16.  Up to 128 rows a per-wavefront kernel slices the reduction over the chip and a
- * second kernel adds the slices in a fixed order (for the MLP the SwiGLU and re-quantisation ride in that
- * reduction) - for a single product only where that pays (K > 2048 and N < 12288; narrow layers keep it
- * further: N <= 2048 up to 384 rows, N <= 1024 up to 512); otherwise the grouped kernel runs with one expert.  Which of the two ran changes the order of the sums, not
- * the arithmetic: a result is reproducible for a given (M, K, N).
+ * multiple of 16.  Layers of few rows run on per-wavefront kernels that slice the reduction over the chip (the
+ * slices are added in a fixed order; for the MLP the SwiGLU and re-quantisation ride in that reduction), the others
+ * on the grouped kernel with one expert, whose reduction is sliced too where it is long and the output narrow.
+ * Which of them runs is a function of (M, K, N), or (M, H, I), that decides the order of the sums, not the
+ * arithmetic: a result is reproducible for a given shape.
  * moe_mlp_fp8 replaces at::mlp_w8a16_dq_forward -> tpudnnMlpW8A16DqAsync
  * (torch_tpu/csrc/ops/my_ops/MlpW8A16Dq.cpp:189-241): out [M, H] bf16 =
  * (silu(x Wg^T) * (x Wu^T)) Wd^T with w13 [2I, H] = gate rows then up rows, w2 [H, I].

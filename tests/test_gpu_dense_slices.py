@@ -1,0 +1,43 @@
+"""Dense FP8 products whose reduction is cut into slices on the grouped kernel: the last slice shorter than the others,
+ragged row and column tiles, against the quantised operands' product in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# 64-, 128- and 192-row tiles; 144, 128, 37 and 65 steps of 128; N that ends inside a 256-column strip
+@pytest.mark.parametrize("M,K,N", [(129, 18432, 7168), (300, 18432, 7168), (150, 14336, 4096), (520, 16384, 1024),
+                                   (33, 18432, 7168), (64, 16384, 1024), (128, 18432, 272), (32, 18432, 1024),
+                                   (1501, 16384, 1008), (385, 4736, 272), (417, 8320, 16), (700, 16384, 1040)])
+def test_sliced_product(pkg, dev, M, K, N):
+    g = torch.Generator().manual_seed(M + K + N)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
+    w = (torch.randn(N, K, generator=g) * 100).clamp(-448, 448).to(torch.float8_e4m3fn).to(dev)
+    ws = (torch.rand(-(-N // 128), K // 128, generator=g) + 0.5).to(dev)
+    out = pkg.mm_fp8(x, pkg.pack_weights(w), ws)
+    q, s = pkg.act_quant(x)
+    xd = (q.double().view(M, K // 128, 128) * s[:, :K // 128, None].double()).view(M, K)
+    wd = w.double() * ws.double().repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)
+    want = xd @ wd.t()
+    d = (out.double() - want).abs()
+    # bf16 result: half a unit in the last place, 2^-9 of the value; the matrix instruction's internal error (2^-11.8 of
+    # the largest of 128 products, 4.5 times an element's size squared) adds about 1e-3 of the result's spread
+    assert (d <= 2.0 ** -8 * want.abs() + 4e-3 * want.pow(2).mean().sqrt()).all(), d.max().item()
+    assert torch.equal(out.view(torch.int16), pkg.mm_fp8(x, pkg.pack_weights(w), ws).view(torch.int16))
+
+
+@pytest.mark.parametrize("M,H,I", [(33, 1024, 12288), (64, 256, 12416), (65, 512, 8192), (128, 1024, 18432), (257, 512, 9216)])
+def test_gated_mlp_of_few_rows_on_the_grouped_kernels(pkg, dev, M, H, I):
+    """Against the same layer run row block by row block on the per-wavefront kernels (at most 32 rows)."""
+    w13, s13 = (t[0] for t in pkg.synthetic_weights(1, 2 * I, H, dev, 3))
+    w2, s2 = (t[0] for t in pkg.synthetic_weights(1, H, I, dev, 4))
+    x = torch.randn(M, H, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(dev)
+    got = pkg.mlp_fp8(x, w13, s13, w2, s2).float()
+    want = torch.cat([pkg.mlp_fp8(x[i:i + 32].contiguous(), w13, s13, w2, s2) for i in range(0, M, 32)]).float()
+    # the first product's sums are formed in another order: an element of the intermediate on a rounding boundary takes
+    # the neighbouring e4m3 code (up to 1/8 of its value) in about 0.2 % of the elements, sqrt(0.002) / 8 / sqrt(3) = 0.003
+    # of the result's spread, 0.02 at seven standard deviations; bf16 adds 2^-8 of the value
+    d = (got - want).abs()
+    rms = want.pow(2).mean().sqrt()
+    assert (d <= 2.0 ** -7 * want.abs() + 0.02 * rms).all() and d.pow(2).mean().sqrt() <= 0.006 * rms

@@ -42,8 +42,19 @@ int route_from_partials_launch(hipStream_t st, const float *partial, int n_slice
 size_t dense_small_partial_bytes(int M, int K, int N, bool keep_partial);
 int dense_small_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M, int K, const uint8_t *w, const float *ws,
                        int N, uint16_t *out, float *partial, int *n_splits_out);
+int dense_product_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M, int K, const uint8_t *w, const float *ws,
+                         int N, uint16_t *out, float *partial);
 int swiglu_quant_reduce_launch(hipStream_t st, const float *partial, int n_splits, int M, int I, uint8_t *hq, float *hs);
-constexpr int kDenseSmallRows = 128;        // up to this many rows the gated MLP uses the per-wavefront dense kernel
+// The gated MLP of few rows: the per-wavefront dense kernels, unless the layer is wide enough for the grouped kernel's 128 +
+// 128 column strips to fill the chip and the rows are too many for one pass of the small kernel over its weights; the
+// second product's reduction is then sliced (dense_split).  Small / grouped in us, gated width 18432 at 17 / 33 / 64 / 100 /
+// 128 rows 90 / 120 / 142 / 196 / 215 against 87 / 92 / 100 / 118 / 121; 14336: 55 / 61 / 72 / 90 / 102 against 54 / 57 / 63 / 57 /
+// 60; 12288 at 32 / 128 rows 77 / 144 against 81 / 94; 10240 at 64 / 128: 60 / 80 against 57 / 60; 8192: 54 / 67 against 55 / 59;
+// 2048 at 64 / 128: 38 / 46 against 60 / 68.
+static inline bool mlp_uses_small_kernel(int M, int I) {
+  if (M > 128) return false;
+  return M > 64 ? I < 8192 : M <= 32 || I < 12288;
+}
 // A single product of few rows: the per-wavefront kernel slices the reduction over the chip, which is what a narrow
 // layer with a long reduction needs (16384 -> 1024 at 64 rows: 28 us against 67 us for the grouped kernel's 16 strips).
 // A wide layer gives the grouped kernel's 64-column strips enough workgroups by itself, and they stream through the
@@ -52,9 +63,11 @@ constexpr int kDenseSmallRows = 128;        // up to this many rows the gated ML
 // launch latencies, of which the grouped path has one fewer (no slices to add).  A layer of at most 2048 columns keeps
 // the sliced kernel up to 384 rows, one of at most 1024 up to 512: the grouped kernel has a handful of strips there
 // (7168 -> 1536 at 129 / 256 / 384 rows: 24 / 27 / 29 us against 34 / 35 / 36 us; 16384 -> 1024: 27 / 31 / 40 against
-// 67 / 69 / 70 us; 4096 -> 4096 is already the grouped kernel's).
+// 67 / 69 / 70 us; 4096 -> 4096 is already the grouped kernel's).  From 33 rows on a reduction of 16384 or more is the
+// grouped kernel's, in slices (dense_split): 18432 -> 7168 at 64 / 128 rows 55 / 71 -> 40 / 44 us, 16384 -> 1024 at 64 / 128 /
+// 300 / 500 rows 24.7 / 28.7 / 36 / 43.5 -> 23.7 / 27.6 / 31.5 / 33.6 us; at 17 rows nothing is gained.
 static inline bool mm_uses_small_kernel(int M, int K, int N) {
-  if (K <= 2048) return false;
+  if (K <= 2048 || (K >= 16384 && M > 32)) return false;
   if (M <= 128) return N < 12288;
   return (M <= 384 && N <= 2048) || (M <= 512 && N <= 1024);
 }
@@ -553,13 +566,15 @@ static DenseWs dense_layout(void *base, int M, int K, int I, int N = 0) {
     w.hq = (uint8_t *)take((size_t)M * I);
     w.hs = (float *)take((size_t)M * scale_pitch(I / kBlock) * 4);
   }
-  if (N > 0 && (I > 0 ? M <= kDenseSmallRows : mm_uses_small_kernel(M, K, N))) {
+  if (N > 0 && (I > 0 ? mlp_uses_small_kernel(M, I) : mm_uses_small_kernel(M, K, N))) {
     if (I > 0) {      // MLP: K = H, N = H; first product [M, 2I] over H, second [M, H] over I
       w.partial1 = (float *)take(dense_small_partial_bytes(M, K, 2 * I, true));
       w.partial = (float *)take(dense_small_partial_bytes(M, I, N, false));
     } else {
       w.partial = (float *)take(dense_small_partial_bytes(M, K, N, false));
     }
+  } else if (N > 0) {
+    w.partial = (float *)take(dense_split_bytes(M, I > 0 ? I : K, N));
   }
   w.bytes = off;
   return w;
@@ -588,8 +603,7 @@ extern "C" int moe_mm_fp8(void *stream, const void *x_bf16, int M, int K, const 
   if (rc) return rc;
   if (mm_uses_small_kernel(M, K, N))
     return dense_small_launch((hipStream_t)stream, d.xq, d.xs, M, K, w, w_scale, N, (uint16_t *)out_bf16, d.partial, nullptr);
-  return gemm2_launch((hipStream_t)stream, d.xq, d.xs, M, M, N, w, w_scale, K, 1, 1, nullptr, nullptr, nullptr, 0,
-                      (uint16_t *)out_bf16, nullptr, nullptr, 0, nullptr, nullptr, nullptr);
+  return dense_product_launch((hipStream_t)stream, d.xq, d.xs, M, K, w, w_scale, N, (uint16_t *)out_bf16, d.partial);
 }
 
 extern "C" int moe_mm_bf16(void *stream, const void *x_bf16, int M, int K, const void *w_bf16, int N, void *out_bf16) {
@@ -645,7 +659,7 @@ extern "C" int moe_mlp_fp8(void *stream, const void *x_bf16, int M, int H, const
   hipStream_t st = (hipStream_t)stream;
   int rc = moe_act_quant(stream, x_bf16, M, H, d.xq, d.xs);
   if (rc) return rc;
-  if (M <= kDenseSmallRows) {
+  if (mlp_uses_small_kernel(M, I)) {
     int n1 = 0;
     rc = dense_small_launch(st, d.xq, d.xs, M, H, w13, w13_scale, 2 * I, nullptr, d.partial1, &n1);
     if (rc) return rc;
@@ -656,8 +670,7 @@ extern "C" int moe_mlp_fp8(void *stream, const void *x_bf16, int M, int H, const
   rc = gemm1_launch(st, d.xq, d.xs, M, H, w13, w13_scale, I, 1, 1, nullptr, nullptr, nullptr, 0, d.hq, d.hs, nullptr,
                     nullptr, nullptr, nullptr);
   if (rc) return rc;
-  return gemm2_launch(st, d.hq, d.hs, M, M, H, w2, w2_scale, I, 1, 1, nullptr, nullptr, nullptr, 0, (uint16_t *)out_bf16,
-                      nullptr, nullptr, 0, nullptr, nullptr, nullptr);
+  return dense_product_launch(st, d.hq, d.hs, M, I, w2, w2_scale, H, (uint16_t *)out_bf16, d.partial);
 }
 
 // ---- un-quantised experts: bf16 weights, bf16 activations, no scales ----

@@ -250,6 +250,11 @@ size_t dense_small_partial_bytes(int M, int K, int N, bool keep_partial) {
   return (s > 1 || keep_partial) ? (size_t)s * M * N * 4 : 0;
 }
 
+int splitk_reduce_launch(hipStream_t st, const float *partial, int n_splits, size_t mn, uint16_t *out) {
+  splitk_reduce_kernel<<<(unsigned)((mn / 4 + 255) / 256), 256, 0, st>>>(partial, n_splits, mn, out);
+  return (int)hipGetLastError();
+}
+
 // out != nullptr: bf16 result (slices added by a second kernel); out == nullptr: the fp32 slices stay in
 // `partial` for the caller's own reduction, their number is returned through n_splits_out.
 int dense_small_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M, int K, const uint8_t *w, const float *ws,
@@ -281,10 +286,7 @@ int dense_small_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M
   }
 #undef MOE_DENSE_SMALL
   if (n_splits_out) *n_splits_out = a.n_splits;
-  if (a.n_splits > 1 && out != nullptr) {
-    const size_t mn = (size_t)M * N;
-    splitk_reduce_kernel<<<(unsigned)((mn / 4 + 255) / 256), 256, 0, st>>>(partial, a.n_splits, mn, out);
-  }
+  if (a.n_splits > 1 && out != nullptr) return splitk_reduce_launch(st, partial, a.n_splits, (size_t)M * N, out);
   return (int)hipGetLastError();
 }
 

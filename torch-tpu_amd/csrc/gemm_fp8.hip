@@ -50,6 +50,8 @@
 
 namespace moe {
 
+int splitk_reduce_launch(hipStream_t st, const float *partial, int n_splits, size_t mn, uint16_t *out);
+
 struct GemmArgs {
   const uint8_t *aq;            // activations fp8 [rows_a, Kd]
   const float *as;              // activation scales [rows_a, as_pitch] (Kd/128 used columns)
@@ -75,6 +77,10 @@ struct GemmArgs {
   int E;                        // experts (tile_prefix[E] = number of row tiles)
   int fixed_expert;             // >= 0: dense mode, every row belongs to this expert and A row p = p
   int max_mtiles;               // entries allocated in tile_expert (row tiles of the list's height)
+  // SLICED (dense second product, FP8): the reduction cut into n_slices slices of k_steps steps (a multiple of 16: a slice's
+  // activation scales start on a 64-byte boundary), slice s of the product in partial[s][rows_a][N]
+  int k_steps, n_slices;
+  float *partial;
   int split;                    // row tiles of this kernel per row tile of the list (1, or 2: half tiles)
   // optional shared expert riding in the same launch (same N / Kd as the routed experts): its
   // row tiles follow the routed ones; rows are the tokens in order
@@ -167,7 +173,9 @@ __device__ __forceinline__ void mma_bf16(v4f (&acc)[WT], const v8i (&w)[WT], con
 // DQ     BF16 arithmetic on FP8 weights with block scales, de-quantised in registers (a.Kd counts the token row's bytes)
 // BF16   un-quantised mode: both operands are bf16 (a 128-byte step is 64 elements = two
 //        v_mfma_f32_16x16x32_bf16 accumulating in place), no scales, bf16 intermediate
-template <int MT, int NW, int DEPTH, bool GATED, bool WREG, bool BF16 = false, int TPS = 16, bool DQ = false>
+// SLICED a dense second product cut along its reduction: a work item is a slice of a tile's steps, its fp32 sums go to
+//        a.partial (an instantiation of its own, so that the whole products carry nothing of it)
+template <int MT, int NW, int DEPTH, bool GATED, bool WREG, bool BF16 = false, int TPS = 16, bool DQ = false, bool SLICED = false>
 // Four wavefronts with the weights in registers: two such workgroups share a compute unit (256 registers a lane each)
 __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_gemm_kernel(const GemmArgs a) {
   static_assert(!DQ || BF16, "de-quantised weights feed the bf16 matrix instructions");
@@ -197,7 +205,10 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   const int n_mtiles = n_routed + (a.sh_rows + BM - 1) / BM;
   // Each XCD takes an equal share of the shared expert's work items (full tiles: the heaviest, so
   // they go first) and then an equal, contiguous share of the routed ones.
-  const int n_routed_work = n_routed * a.n_strips, n_shared_work = (n_mtiles - n_routed) * a.n_strips;
+  static_assert(!SLICED || (!GATED && !BF16 && TPS == 16), "slices: second product on FP8 operands, wide strips");
+  const int n_slice_work = n_routed * a.n_strips;      // work items of one slice
+  const int n_routed_work = SLICED ? n_slice_work * a.n_slices : n_slice_work;
+  const int n_shared_work = (n_mtiles - n_routed) * a.n_strips;
   const int per_xcd_r = (n_routed_work + 7) >> 3, per_xcd_s = (n_shared_work + 7) >> 3;
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   const int my_shared = min(max(n_shared_work - xcd * per_xcd_s, 0), per_xcd_s);
@@ -209,6 +220,11 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     if (j >= per_xcd_r) return;
     logical = xcd * per_xcd_r + j;
     if (logical >= n_routed_work) return;
+  }
+  int slice = 0;                                       // a slice's items follow one another; no shared expert then
+  if (SLICED) {
+    slice = logical / n_slice_work;
+    logical -= slice * n_slice_work;
   }
   // Inside one expert the (row tile, strip) pairs are walked in blocks of up to kBlockM row tiles x
   // kBlockS strips, so that the ~32 workgroups an XCD runs at a time share a few token tiles and a few
@@ -257,8 +273,10 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     row0 = e_row0 + (mtile - first_mtile) * BM;
     rows = min(BM, e_row0 + e_rows - row0);
   }
-  const uint8_t *const aq = shared ? a.sh_aq : a.aq;
-  const float *const as = shared ? a.sh_as : a.as;
+  // first step of this workgroup's slice of the reduction
+  const int kb_first = SLICED ? slice * a.k_steps : 0;
+  const uint8_t *const aq = (shared ? a.sh_aq : a.aq) + (SLICED ? (size_t)kb_first * 128 : 0);
+  const float *const as = (shared ? a.sh_as : a.as) + (SLICED ? kb_first : 0);
   const uint8_t *const wq = shared ? a.sh_w : a.w;
   const float *const ws = shared ? a.sh_ws : a.ws;
   const int rows_a = shared ? a.sh_rows : a.rows_a;
@@ -266,7 +284,8 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   const int mt_live = (rows + 15) >> 4;               // m-tiles that hold at least one row
   const bool stream_weights = n_mt == 1;              // the expert's rows fit this one row tile
 
-  const int NKB = a.Kd >> 7;
+  const int n_kb = a.Kd >> 7;                         // 128-steps of the whole reduction
+  const int NKB = SLICED ? min(a.k_steps, n_kb - kb_first) : n_kb;
   const int n_wblk = (a.n_rows_w + 127) >> 7;         // weight-scale rows per expert
 
   // ---- per-lane source addresses ------------------------------------------------------------
@@ -280,7 +299,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     if (GATED) wrow = (j < WT / 2 ? 0 : a.N) + strip * 128 + wave * (8 * WT) + (j % (WT / 2)) * 16;
     else wrow = strip * (16 * TPS) + wave * (16 * WT) + j * 16;
     wrow = min(wrow, a.n_rows_w - 16);                 // tiles past the matrix re-read its last rows
-    wtile[j] = wq + ((size_t)e * a.n_rows_w + wrow) * (DQ ? a.Kd >> 1 : a.Kd);
+    wtile[j] = wq + ((size_t)e * a.n_rows_w + wrow) * (DQ ? a.Kd >> 1 : a.Kd) + (SLICED ? (size_t)kb_first * 2048 : 0);
   }
   // Weights are stored tile-blocked: the 2 KB a (16-row tile, 128-byte step) pair needs are contiguous and already
   // in operand order - two 1 KB halves of [lane][16 bytes] - so every load instruction of a wavefront reads 1 KB of
@@ -293,7 +312,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   constexpr int NSB = (2 * kMaxKB + NT - 1) / NT;
   float sbv[NSB];
   // DQ: a step is half a 128-block of the reduction (64 elements), two steps share a block scale
-  const int NKBW = DQ ? NKB >> 1 : NKB;
+  const int NKBW = DQ ? n_kb >> 1 : n_kb;
   if constexpr (!BF16 || DQ) {
     // second GEMM: the 128-row blocks the strip's first and ninth tile lie in (a narrow strip lies in one)
     const int blk0 = GATED ? strip : min(strip * TPS / 8, n_wblk - 1);
@@ -301,7 +320,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
 #pragma unroll
     for (int u = 0; u < NSB; u++) {
       const int i = tid + u * NT, r = i >= NKB, kb = i - r * NKB;
-      sbv[u] = i < 2 * NKB ? ws[((size_t)e * n_wblk + (r ? blk1 : blk0)) * NKBW + (DQ ? kb >> 1 : kb)] : 0.f;
+      sbv[u] = i < 2 * NKB ? ws[((size_t)e * n_wblk + (r ? blk1 : blk0)) * NKBW + (DQ ? kb >> 1 : kb_first + kb)] : 0.f;
     }
   }
   for (int i = tid; i < BM; i += NT) {
@@ -843,6 +862,19 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
         if (i < rows && wave == 0 && lg == 0) (shared ? a.sh_hs : a.hs)[(size_t)(row0 + i) * a.hs_pitch + strip] = sc;
       }
     }
+  } else if constexpr (SLICED) {
+    // a slice of the product: fp32, straight from the registers (16 bytes per lane, 64 per row and tile)
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++) {
+      const int r = mt * 16 + li;
+#pragma unroll
+      for (int j = 0; j < WT; j++) {
+        const int col = strip * (16 * TPS) + (wave * WT + j) * 16 + lg * 4;
+        if (r < rows && col < a.N)
+          *(v4f *)(a.partial + ((size_t)slice * a.rows_a + row0 + r) * a.N + col) = acc[mt][j];
+      }
+    }
+    return;
   } else {
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
@@ -906,10 +938,10 @@ static int launch_gemm(hipStream_t st, GemmArgs &a, int tile_m, int routed_tiles
   // round (a dense 7168 -> 7168 product at 288-384 rows, 140-168 wide items: 64 us in narrow strips, 46 us in wide ones).
   // (a dense layer knows its row tiles; the tile list's entries are an upper bound, a few more than the real ones -
   // Mixtral shape at 48-96 tokens: 9-11 entries for 8 real tiles of 16 strips each - hence the wider margin there)
-  const bool narrow = !GATED && (km <= 32 || (km == 64 && row_tiles * ((a.N + 255) / 256) < (a.fixed_expert >= 0 ? 129 : 193)));
+  const bool narrow = !GATED && !a.partial && (km <= 32 || (km == 64 && row_tiles * ((a.N + 255) / 256) < (a.fixed_expert >= 0 ? 129 : 193)));
   a.n_strips = GATED ? a.N / 128 : narrow ? (a.N + 63) / 64 : (a.N + 255) / 256;
   a.max_mtiles = routed_tiles;
-  long total = row_tiles * a.n_strips;
+  long total = row_tiles * a.n_strips * (a.partial ? a.n_slices : 1);
   total = (total + 7) / 8 * 8 + 16;                  // the per-XCD split rounds two shares up
   if (total <= 0 || total > 0x7fffffffl) return MOE_E_SHAPE;
   a.total_blocks = (int)total;
@@ -926,6 +958,19 @@ static int launch_gemm(hipStream_t st, GemmArgs &a, int tile_m, int routed_tiles
         default: MOE_GEMM_NARROW(4, 2); break;
       }
 #undef MOE_GEMM_NARROW
+      return (int)hipGetLastError();
+    }
+  }
+  if constexpr (!GATED && !BF16) {
+    if (a.partial) {
+#define MOE_GEMM_SLICED(MT, WREG) grouped_gemm_kernel<MT, 8, 2, false, WREG, false, 16, false, true><<<grid, dim3(512), 0, st>>>(a)
+      switch (km) {
+        case 64: MOE_GEMM_SLICED(4, false); break;
+        case 128: MOE_GEMM_SLICED(8, true); break;
+        case 192: MOE_GEMM_SLICED(12, true); break;
+        default: return MOE_E_SHAPE;
+      }
+#undef MOE_GEMM_SLICED
       return (int)hipGetLastError();
     }
   }
@@ -997,6 +1042,24 @@ int gemm2_launch(hipStream_t st, const uint8_t *hq, const float *hs, int rows_a,
   if (numerics == kNumericsW8A16) return launch_gemm<false, true, true>(st, a, tile_m, routed_tiles, mean_rows);
   if (bf16) return launch_gemm<false, true>(st, a, tile_m, routed_tiles, mean_rows);
   return launch_gemm<false>(st, a, tile_m, routed_tiles, mean_rows);
+}
+
+// A dense FP8 product on the grouped kernels: out [M, N] bf16 = xq [M, K] . w [N, K]^T.  `partial` holds the slices when
+// dense_split() cuts the reduction (they are added in slice order by a second kernel).
+int dense_product_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M, int K, const uint8_t *w, const float *ws,
+                         int N, uint16_t *out, float *partial) {
+  const DenseSplit sp = dense_split(M, K, N);
+  if (sp.slices == 1)
+    return gemm2_launch(st, xq, xs, M, M, N, w, ws, K, 1, 1, nullptr, nullptr, nullptr, 0, out, nullptr, nullptr, 0, nullptr,
+                        nullptr, nullptr, kNumericsFp8);
+  GemmArgs a{};
+  a.aq = xq; a.as = xs; a.w = w; a.ws = ws; a.y = out;
+  a.as_pitch = scale_pitch(K / kBlock);
+  a.Kd = K; a.N = N; a.n_rows_w = N; a.rows_a = M; a.topk = 1; a.E = 1; a.fixed_expert = 0;
+  a.k_steps = sp.k_steps; a.n_slices = sp.slices; a.partial = partial;
+  const int rc = launch_gemm<false>(st, a, sp.tile_m, (M + sp.tile_m - 1) / sp.tile_m, (double)M);
+  if (rc) return rc;
+  return splitk_reduce_launch(st, partial, sp.slices, (size_t)M * N, out);
 }
 
 }  // namespace moe

@@ -72,6 +72,47 @@ static inline int choose_dense_tile_m(long rows, int items_per_row_tile, int ste
   return best;
 }
 
+// How a dense product on the grouped kernels is cut along its reduction.  A long reduction over few output strips leaves
+// half of the compute units without work and the others with a chain of steps that each wait for the weight stream
+// (18432 -> 7168 at 300 rows: 140 items of 64 rows x 144 steps, 115 us for 132 MB).  Slices of whole 16-step pieces on the
+// tall tiles, fp32, added in order by a second kernel, when the same kind of model says it pays: rounds of items x
+// (steps x step + start and end), in shader cycles, plus, for slices, 10 000 for the second launch and their bytes (written
+// and read once) at 2000 a cycle.  A step of a 64-row tile counts what it takes with the weights coming from HBM, not L2
+// (1500 wide, 1000 in narrow strips).  Up to 32 rows a product is one stream of weights and stays whole.
+// Measured, whole op, before -> after: 16384 -> 1024 at 520 / 700 / 1500 / 4000 rows 70 / 72 / 83 / 126 -> 34 / 36 / 53 / 105 us;
+// gated MLP 7168 / 18432 at 129 / 300 / 400 rows 165 / 209 / 245 -> 130 / 174 / 219 us (the second product 115 -> 57 + 6 us at 300
+// rows, 2.3 TB/s of weights), 4096 / 14336 at 129 / 300 / 600 rows 99 / 107 / 167 -> 71 / 85 / 146 us.
+struct DenseSplit {
+  int tile_m, slices, k_steps;
+};
+static inline DenseSplit dense_split(long rows, int K, int N) {
+  const int steps = K / 128, strips = (N + 255) / 256;
+  DenseSplit best = {choose_dense_tile_m(rows, strips, steps), 1, steps};
+  const auto rounds = [](long items) { return (double)((items + 255) / 256); };
+  double best_cost;
+  {
+    const long row_tiles = (rows + best.tile_m - 1) / best.tile_m;
+    const bool narrow = best.tile_m == 64 && row_tiles * strips < 129;
+    const double step = best.tile_m > 64 ? 300.0 + 150.0 * (best.tile_m / 16) : narrow ? 1000.0 : 1500.0;
+    best_cost = 0.87 * rounds(row_tiles * strips) * (steps * step + 20000.0);      // a clear win or none
+  }
+  if (rows <= 32 || best.tile_m == 96) return best;
+  for (int tm = rows <= 64 ? 64 : 128; tm <= 192; tm += 64) {
+    const long items = (rows + tm - 1) / tm * (long)strips;
+    for (int len = 16; len < steps; len += 16) {
+      const int slices = (steps + len - 1) / len;
+      const double cost = rounds(items * slices) * (len * (300.0 + 150.0 * (tm / 16)) + 20000.0) + 10000.0 +
+                          8.0 * slices * (double)rows * N / 2000.0;
+      if (cost < best_cost) { best = {tm, slices, len}; best_cost = cost; }
+    }
+  }
+  return best;
+}
+static inline size_t dense_split_bytes(long rows, int K, int N) {
+  const DenseSplit s = dense_split(rows, K, N);
+  return s.slices > 1 ? (size_t)s.slices * rows * N * 4 : 0;
+}
+
 struct PermuteWs {
   int32_t *chunk_counts;   // [n_chunks, E]
   int32_t *tile_prefix;    // [E + 1] first tile of each expert; [E] = number of tiles
