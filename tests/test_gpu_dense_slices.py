@@ -9,6 +9,9 @@ pytestmark = pytest.mark.gpu
 # 64-, 128- and 192-row tiles; 144, 128, 37 and 65 steps of 128; N that ends inside a 256-column strip
 @pytest.mark.parametrize("M,K,N", [(129, 18432, 7168), (300, 18432, 7168), (150, 14336, 4096), (520, 16384, 1024),
                                    (33, 18432, 7168), (64, 16384, 1024), (128, 18432, 272), (32, 18432, 1024),
+                                   # a workgroup per 16 columns: 1, 2 and 4 row tiles, columns past the last eight
+                                   (1, 7168, 1536), (16, 2176, 1040), (32, 7168, 2048), (33, 4096, 2064), (64, 7168, 4096),
+                                   (17, 16384, 16), (31, 2304, 4096), (64, 7168, 4112),
                                    (1501, 16384, 1008), (385, 4736, 272), (417, 8320, 16), (700, 16384, 1040)])
 def test_sliced_product(pkg, dev, M, K, N):
     g = torch.Generator().manual_seed(M + K + N)

@@ -155,6 +155,96 @@ __global__ __launch_bounds__(64 * kDsWaves) void dense_small_kernel(const SmallA
   }
 }
 
+// Narrow layers: one launch for the product and the sum of its slices.  A workgroup of sixteen wavefronts owns one
+// 16-column weight tile for 16 MT token rows and the whole reduction, a sixteenth of it per wavefront; the slices meet in
+// LDS and are added in slice order.  Against items of one wavefront with the slices in memory that saves the launch that
+// adds them (5 us and a gap, more than such a product itself takes); what it gives up is the reuse of a token operand
+// over several weight tiles, so it is for layers whose tiles just about fill the compute units (dense_narrow_mt).
+constexpr int kNarrowWaves = 16, kNarrowMaxWgs = 256;
+template <int MT>
+__global__ __launch_bounds__(64 * kNarrowWaves) void dense_narrow_kernel(const SmallArgs a) {
+  constexpr int U = MT == 1 ? 4 : (MT == 2 ? 2 : 1);     // steps of one load batch: 128 registers a lane
+  __shared__ v4f part[kNarrowWaves][MT][64];
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // workgroup ids go round the eight XCDs: the row chunks of a tile sit eight apart, so that they share its weights in L2
+  const int n_tiles = a.N / 16;
+  const int grp = blockIdx.x / (8 * a.n_mchunks), in = blockIdx.x % (8 * a.n_mchunks);
+  const int nt = grp * 8 + in % 8, mc = in / 8;
+  if (nt >= n_tiles) return;
+  const int kb0 = wave * a.split_len, kb1 = min(kb0 + a.split_len, a.NKB);
+  const uint8_t *wp = a.w + (size_t)(nt * 16) * a.K + lane * 16;
+  const float *wsp = a.ws + (size_t)(nt >> 3) * a.NKB;
+  const uint8_t *xp[MT];
+  const float *sap[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) {
+    const int row = min(mc * 16 * MT + mt * 16 + li, a.M - 1);
+    xp[mt] = a.xq + (size_t)row * a.K + lg * 16;
+    sap[mt] = a.xs + (size_t)row * a.xs_pitch;
+  }
+  v4f acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) acc[mt] = (v4f){0.f, 0.f, 0.f, 0.f};
+  for (int kb = kb0; kb < kb1; kb += U) {
+    v4i wl[U], wh[U], xl[U][MT], xh[U][MT];
+    float f[U][MT];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int kk = min(kb + u, kb1 - 1);               // past the slice: the last step again, times zero
+      const float sb = kb + u < kb1 ? wsp[kk] : 0.f;
+      const v4i *lo = (const v4i *)(wp + (size_t)kk * 2048);
+      wl[u] = lo[0]; wh[u] = lo[64];
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) {
+        xl[u][mt] = *(const v4i *)(xp[mt] + (size_t)kk * 128);
+        xh[u][mt] = *(const v4i *)(xp[mt] + (size_t)kk * 128 + 64);
+        f[u][mt] = sap[mt][kk] * sb;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++)
+#pragma unroll
+      for (int mt = 0; mt < MT; mt++) {
+        const v4f zero = {0.f, 0.f, 0.f, 0.f};
+        const v4f p = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(cat8(wl[u], wh[u]), cat8(xl[u][mt], xh[u][mt]), zero,
+                                                                       0, 0, 0, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[mt][r] = fmaf(p[r], f[u][mt], acc[mt][r]);
+      }
+  }
+#pragma unroll
+  for (int mt = 0; mt < MT; mt++) part[wave][mt][lane] = acc[mt];
+  __syncthreads();
+  if (wave >= MT) return;
+  const int row = mc * 16 * MT + wave * 16 + li;
+  if (row >= a.M) return;
+  v4f s = part[0][wave][lane];
+#pragma unroll
+  for (int k = 1; k < kNarrowWaves; k++) {
+    const v4f t = part[k][wave][lane];
+    s[0] += t[0]; s[1] += t[1]; s[2] += t[2]; s[3] += t[3];
+  }
+  v2i v;
+  v[0] = (int)((uint32_t)f32_to_bf16(s[0]) | ((uint32_t)f32_to_bf16(s[1]) << 16));
+  v[1] = (int)((uint32_t)f32_to_bf16(s[2]) | ((uint32_t)f32_to_bf16(s[3]) << 16));
+  *(v2i *)(a.out + (size_t)row * a.N + nt * 16 + lg * 4) = v;
+}
+
+// m-tiles per workgroup of that kernel, 0: the layer is not one for it.  The smallest count whose workgroups all run at
+// once, one per compute unit (its sixteen wavefronts fill half of one).  Whole op with the quantiser's launch, before ->
+// after: 7168 -> 1536 at 1 / 16 / 32 / 64 rows 10.6 / 13.1 / 15.0 / 19.2 -> 7.2 / 10.9 / 11.0 / 16.1 us, 16384 -> 1024 15.9 / 19.3 /
+// 19.9 -> 9.3 / 17.9 / 18.4, 4096 -> 4096 at 1 / 16 / 17 / 64 rows 10.1 / 12.9 / 12.8 / 19.2 -> 7.4 / 12.1 / 9.5 / 17.2.  With
+// more workgroups than that it loses: 7168 -> 7168 at 32 / 64 rows 20 / 27 -> 30 / 48 us.
+int dense_narrow_mt(int M, int K, int N) {
+  if (M > 64 || K < 2048) return 0;
+  for (int mt = 1; mt <= 4; mt *= 2) {
+    const long chunks = (M + 16 * mt - 1) / (16 * mt);
+    if ((long)(N / 16) * chunks <= kNarrowMaxWgs) return mt;
+  }
+  return 0;
+}
+
 // out[m, n] = bf16(sum over slices in slice order), four columns per lane
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ partial, int n_splits, size_t mn,
                                                            uint16_t *__restrict__ out) {
@@ -246,6 +336,7 @@ void dense_small_plan(int M, int K, int N, int *n_splits, int *split_len, int *r
 
 size_t dense_small_partial_bytes(int M, int K, int N, bool keep_partial) {
   int s, l, r, c, t;
+  if (!keep_partial && dense_narrow_mt(M, K, N)) return 0;
   dense_small_plan(M, K, N, &s, &l, &r, &c, &t);
   return (s > 1 || keep_partial) ? (size_t)s * M * N * 4 : 0;
 }
@@ -265,6 +356,16 @@ int dense_small_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M
   dense_small_plan(M, K, N, &a.n_splits, &a.split_len, &rows, &a.n_mchunks, &ntw);
   a.xq = xq; a.xs = xs; a.xs_pitch = scale_pitch(K / kBlock); a.w = w; a.ws = ws; a.partial = partial; a.out = out;
   a.M = M; a.K = K; a.N = N; a.NKB = K / kBlock;
+  if (const int mt = out ? dense_narrow_mt(M, K, N) : 0) {
+    a.n_mchunks = (M + 16 * mt - 1) / (16 * mt);
+    a.split_len = (a.NKB + kNarrowWaves - 1) / kNarrowWaves;
+    const unsigned wgs = (unsigned)((N / 16 + 7) / 8 * 8 * a.n_mchunks);
+    if (mt == 1) dense_narrow_kernel<1><<<wgs, 64 * kNarrowWaves, 0, st>>>(a);
+    else if (mt == 2) dense_narrow_kernel<2><<<wgs, 64 * kNarrowWaves, 0, st>>>(a);
+    else dense_narrow_kernel<4><<<wgs, 64 * kNarrowWaves, 0, st>>>(a);
+    if (n_splits_out) *n_splits_out = 1;
+    return (int)hipGetLastError();
+  }
   const bool stream_w = a.n_mchunks == 1 && (size_t)N * K >= ((size_t)64 << 20);
   const long items = (long)(N / (16 * ntw)) * a.n_splits * a.n_mchunks;
   const long blocks = (items + kDsWaves - 1) / kDsWaves;
