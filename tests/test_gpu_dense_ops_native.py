@@ -1,0 +1,65 @@
+"""The dense ops' native path against the general one: the same bits for every form both accept, and packed copies that
+follow their weights."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def weights(dev, n, k, seed, dtype=torch.bfloat16):
+    g = torch.Generator().manual_seed(seed)
+    w = (torch.randn(n, k, generator=g) * 100).clamp(-448, 448).to(torch.float8_e4m3fn).to(dev)
+    return w, ((torch.rand(-(-n // 128), -(-k // 128), generator=g) + 0.5) * 0.01).to(dtype).to(dev)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 128, 16), (32, 7168, 1536), (5, 256, 1040), (130, 384, 272)])
+@pytest.mark.parametrize("form", ["plain", "fp32 scales", "strided weight", "strided input", "strided output", "float64 scales"])
+def test_mm_forms(pkg, dev, M, K, N, form):
+    w, s = weights(dev, N, K, M + K, {"fp32 scales": torch.float32, "float64 scales": torch.float64}.get(form, torch.bfloat16))
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(N)).to(torch.bfloat16).to(dev)
+    if form == "strided weight":
+        w = w.t().contiguous().t()
+    if form == "strided input":
+        x = torch.cat([x, x], 1)[:, :K]
+    a, b = torch.zeros(2, M, 2 * N, dtype=torch.bfloat16, device=dev)
+    a, b = (t[:, :N] if form == "strided output" else t[:, :N].contiguous() for t in (a, b))
+    r = torch.ops.my_ops.mm_w8a16_dq_forward(x, w, s, a, 128)
+    assert r.data_ptr() == a.data_ptr()
+    torch.ops.my_ops._mm_general(x, w, s, b, 128)
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16)) and a.abs().max() > 0
+
+
+@pytest.mark.parametrize("M,H,I", [(1, 128, 128), (3, 256, 384), (140, 384, 512)])
+@pytest.mark.parametrize("scale_dtype", [torch.bfloat16, torch.float32])
+def test_mlp_forms(pkg, dev, M, H, I, scale_dtype):
+    (g, gs), (u, us), (d, ds) = (weights(dev, I, H, i, scale_dtype) for i in range(3))
+    x = torch.randn(M, H, generator=torch.Generator().manual_seed(M)).to(torch.bfloat16).to(dev)
+    a, b = torch.zeros(2, M, H, dtype=torch.bfloat16, device=dev)
+    torch.ops.my_ops.mlp_w8a16_dq_forward(x, g, u, d, gs, us, ds, a, 128)
+    torch.ops.my_ops._mlp_general(x, g, u, d, gs, us, ds, b, 128)
+    assert torch.equal(a.view(torch.int16), b.view(torch.int16)) and a.abs().max() > 0
+
+
+def test_packed_copy_follows_its_weight(pkg, dev):
+    x = torch.randn(4, 256, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(dev)
+    w, s = weights(dev, 128, 256, 2)
+    run = lambda: torch.ops.my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty(4, 128, dtype=torch.bfloat16, device=dev), 128)
+    first = run()
+    s.mul_(2)                                             # an in-place write moves the version counter
+    assert torch.equal(run(), first * 2)
+    w.copy_(torch.zeros_like(w))
+    assert run().abs().max() == 0
+    del w
+    w, s = weights(dev, 128, 256, 3)                      # new storages, possibly on the old addresses
+    out = torch.empty(4, 128, dtype=torch.bfloat16, device=dev)
+    torch.ops.my_ops._mm_general(x, w, s, out, 128)
+    assert torch.equal(run(), out)
+
+
+def test_what_was_refused_stays_refused(pkg, dev):
+    x = torch.zeros(4, 256, dtype=torch.bfloat16, device=dev)
+    w, s = weights(dev, 128, 256, 2)
+    out = torch.empty(4, 128, dtype=torch.bfloat16, device=dev)
+    for bad in [(x.float(), w, s, out, 128), (x, w.to(torch.bfloat16), s, out, 128), (x, w, s, out.float(), 128), (x, w, s, out, 0)]:
+        with pytest.raises((RuntimeError, TypeError, ValueError)):
+            torch.ops.my_ops.mm_w8a16_dq_forward(*bad)

@@ -9,7 +9,9 @@
 // packed copy of the reference-layout weights (made once per weight set, found again through the identity of the
 // sources' storages), one workspace per (device, stream).  The rarer forms of the op - bf16 weights, block sizes
 // other than 128, ragged sizes, the W8A16 arithmetic - are handed to `my_ops::_fused_experts_general`, which the
-// Python package defines on the same C ABI.
+// Python package defines on the same C ABI.  The dense ops mm_w8a16_dq_forward and mlp_w8a16_dq_forward are split the
+// same way (`_mm_general`, `_mlp_general`): at decode sizes a call took longer in Python (21 us for the 7168 -> 1536 product
+// at 32 rows) than its two launches take on the GPU (11 us).
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/hip/HIPStream.h>
@@ -43,7 +45,7 @@ void *stream_of(const Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(
 // dead and is dropped the next time the table is walked, so new weights that land on a recycled address never meet
 // an old copy.  An in-place write that does not move the version counter cannot be seen from here
 // (my_ops::_invalidate_weight_cache after such an update).
-// (three dimensions: the callers of identify() have checked that)
+// (two or three dimensions: the callers of identify() have checked that)
 struct SourceId {
   const c10::StorageImpl *storage;
   const void *data;
@@ -66,8 +68,8 @@ SourceId identify(const Tensor &t) {
   s.version = t.is_inference() ? 0u : (uint32_t)t._version();
   s.dtype = t.scalar_type();
   for (int i = 0; i < 3; i++) {
-    s.sizes[i] = t.size(i);
-    s.strides[i] = t.stride(i);
+    s.sizes[i] = i < t.dim() ? t.size(i) : 0;
+    s.strides[i] = i < t.dim() ? t.stride(i) : 0;
   }
   return s;
 }
@@ -120,6 +122,49 @@ const PackedEntry &packed_weights(const Tensor &gate, const Tensor &up, const Te
   e.w2s = ds.transpose(1, 2).to(at::kFloat).contiguous();
   g_packed.push_back(std::move(e));
   return g_packed.back();
+}
+
+// The packed copies of the dense ops' weights, under the same rules: `made` is tile-blocked weights and fp32 scales, one
+// pair (a product) or two (the MLP).
+struct DenseEntry {
+  std::vector<SourceId> ids;
+  std::vector<c10::weak_intrusive_ptr<c10::StorageImpl>> alive;
+  std::vector<Tensor> made;
+};
+std::vector<DenseEntry> g_dense;
+
+template <typename Make>
+const std::vector<Tensor> &dense_packed(std::initializer_list<const Tensor *> src, Make make) {
+  std::vector<SourceId> ids;
+  for (const Tensor *t : src) ids.push_back(identify(*t));
+  for (size_t i = 0; i < g_dense.size();) {
+    bool dead = false;
+    for (auto &w : g_dense[i].alive) dead = dead || w.expired();
+    if (dead) {
+      g_dense[i] = std::move(g_dense.back());
+      g_dense.pop_back();
+      continue;
+    }
+    if (g_dense[i].ids == ids) return g_dense[i].made;
+    i++;
+  }
+  DenseEntry e;
+  for (const Tensor *t : src) e.alive.push_back(t->storage().getWeakStorageImpl());
+  e.ids = std::move(ids);
+  e.made = make();
+  g_dense.push_back(std::move(e));
+  return g_dense.back().made;
+}
+
+// what the common forms of the dense ops ask of their tensors; any other form takes the general road
+bool plain_matrix(const Tensor &t, c10::ScalarType dtype, int64_t rows, int64_t cols, const Tensor &like) {
+  return t.dim() == 2 && t.scalar_type() == dtype && t.size(0) == rows && t.size(1) == cols && t.is_cuda() &&
+         t.device() == like.device() && t.is_contiguous() && (uintptr_t)t.const_data_ptr() % 16 == 0;
+}
+bool plain_weight(const Tensor &w, const Tensor &s, int64_t rows, int64_t cols, const Tensor &like) {
+  return w.dim() == 2 && w.scalar_type() == at::kFloat8_e4m3fn && w.size(0) == rows && w.size(1) == cols && w.is_cuda() &&
+         w.device() == like.device() && !w.is_inference() && s.dim() == 2 && s.size(0) == (rows + 127) / 128 &&
+         s.size(1) == (cols + 127) / 128 && s.is_cuda() && s.device() == like.device() && !s.is_inference();
 }
 
 // one scratch tensor per (device, stream), grown on demand: nothing is allocated once it is large enough
@@ -286,6 +331,59 @@ Tensor fused_moe_fused_experts_v2(const Tensor &output, const Tensor &input, con
                                  save_mid_res);
 }
 
+// torch_tpu/csrc/ops/my_ops/MmW8A16Dq.cpp:185-228: weight [N, K], scale [ceil(N/bs), ceil(K/bs)], output [M, N]
+Tensor mm_w8a16_dq_forward(const Tensor &input, const Tensor &weight, const Tensor &scale, const Tensor &output,
+                           int64_t blocksize) {
+  bool fast = blocksize == 128 && input.dim() == 2 && weight.dim() == 2;
+  const int64_t M = fast ? input.size(0) : 0, N = fast ? weight.size(0) : 0, K = fast ? weight.size(1) : 0;
+  fast = fast && M > 0 && K >= 128 && K % 128 == 0 && K <= 32768 && N >= 16 && N % 16 == 0 && N <= (1 << 20) &&
+         M * K < (1ll << 31) && M * N < (1ll << 31) && N * K < (1ll << 32) && plain_weight(weight, scale, N, K, input) &&
+         plain_matrix(input, at::kBFloat16, M, K, input) && plain_matrix(output, at::kBFloat16, M, N, input);
+  std::unique_lock<std::mutex> lock(g_mutex);
+  if (!fast || g_numerics != 0) {
+    lock.unlock();
+    return call_general("my_ops::_mm_general", {input, weight, scale, output, blocksize});
+  }
+  void *st = stream_of(input);
+  const auto &w = dense_packed({&weight, &scale}, [&]() -> std::vector<Tensor> {
+    return {tile_block(weight.contiguous()), scale.to(at::kFloat).contiguous()};
+  });
+  const size_t need = moe_mm_fp8_workspace_bytes((int)M, (int)K, (int)N);
+  Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
+  check_rc(moe_mm_fp8(st, input.data_ptr(), (int)M, (int)K, (const uint8_t *)w[0].data_ptr(), w[1].data_ptr<float>(), (int)N,
+                      output.data_ptr(), ws.data_ptr(), (size_t)ws.numel()),
+           "mm_w8a16_dq_forward");
+  return output;
+}
+
+// torch_tpu/csrc/ops/my_ops/MlpW8A16Dq.cpp:189-241: gate / up [I, H], down passed transposed as [I, H], scales likewise
+Tensor mlp_w8a16_dq_forward(const Tensor &input, const Tensor &gate, const Tensor &up, const Tensor &down, const Tensor &gs,
+                            const Tensor &us, const Tensor &ds, const Tensor &output, int64_t blocksize) {
+  bool fast = blocksize == 128 && input.dim() == 2 && gate.dim() == 2;
+  const int64_t M = fast ? input.size(0) : 0, I = fast ? gate.size(0) : 0, H = fast ? gate.size(1) : 0;
+  fast = fast && M > 0 && H >= 128 && H % 128 == 0 && H <= 32768 && I >= 128 && I % 128 == 0 && I <= 32768 &&
+         M * H < (1ll << 31) && M * I < (1ll << 31) && plain_weight(gate, gs, I, H, input) &&
+         plain_weight(up, us, I, H, input) && plain_weight(down, ds, I, H, input) && gs.scalar_type() == us.scalar_type() &&
+         plain_matrix(input, at::kBFloat16, M, H, input) && plain_matrix(output, at::kBFloat16, M, H, input);
+  std::unique_lock<std::mutex> lock(g_mutex);
+  if (!fast || g_numerics != 0) {
+    lock.unlock();
+    return call_general("my_ops::_mlp_general", {input, gate, up, down, gs, us, ds, output, blocksize});
+  }
+  void *st = stream_of(input);
+  const auto &w = dense_packed({&gate, &up, &down, &gs, &us, &ds}, [&]() -> std::vector<Tensor> {
+    return {tile_block(at::cat({gate, up}, 0).contiguous()), at::cat({gs, us}, 0).to(at::kFloat).contiguous(),
+            tile_block(down.t().contiguous()), ds.t().to(at::kFloat).contiguous()};
+  });
+  const size_t need = moe_mlp_fp8_workspace_bytes((int)M, (int)H, (int)I);
+  Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
+  check_rc(moe_mlp_fp8(st, input.data_ptr(), (int)M, (int)H, (const uint8_t *)w[0].data_ptr(), w[1].data_ptr<float>(),
+                       (const uint8_t *)w[2].data_ptr(), w[3].data_ptr<float>(), (int)I, output.data_ptr(), ws.data_ptr(),
+                       (size_t)ws.numel()),
+           "mlp_w8a16_dq_forward");
+  return output;
+}
+
 // torch_tpu/csrc/ops/my_ops/NoauxTcTopk.cpp:9-67: group-limited top-k into caller-allocated values / indices
 Tensor noaux_tc_topk(const Tensor &values, const Tensor &indices, const Tensor &scores, int64_t n_groups,
                      int64_t topk_groups, int64_t top_k) {
@@ -377,6 +475,7 @@ void _set_expert_numerics(int64_t mode) {
 void _invalidate_weight_cache() {
   std::lock_guard<std::mutex> lock(g_mutex);
   g_packed.clear();
+  g_dense.clear();
 }
 
 int64_t _packed_weight_sets() {
@@ -389,12 +488,20 @@ TORCH_LIBRARY(my_ops, m) {
   m.def("fused_moe_fused_experts", fused_moe_fused_experts);
   m.def("fused_moe_fused_experts_v2", fused_moe_fused_experts_v2);
   m.def("noaux_tc_topk", noaux_tc_topk);
+  m.def("mm_w8a16_dq_forward(Tensor input, Tensor weight, Tensor scale, Tensor(a!) output, int blocksize) -> Tensor(a!)");
+  m.def("mlp_w8a16_dq_forward(Tensor input, Tensor gate_weight, Tensor up_weight, Tensor down_weight, Tensor gate_scale, "
+        "Tensor up_scale, Tensor down_scale, Tensor(a!) output, int blocksize) -> Tensor(a!)");
   m.def("enable_profile", enable_profile);
   m.def("disable_profile", disable_profile);
   m.def("_profile_report", _profile_report);
   m.def("_set_expert_numerics", _set_expert_numerics);
   m.def("_invalidate_weight_cache", _invalidate_weight_cache);
   m.def("_packed_weight_sets", _packed_weight_sets);
+}
+
+TORCH_LIBRARY_IMPL(my_ops, CompositeExplicitAutograd, m) {
+  m.impl("mm_w8a16_dq_forward", mm_w8a16_dq_forward);
+  m.impl("mlp_w8a16_dq_forward", mlp_w8a16_dq_forward);
 }
 
 }  // namespace at

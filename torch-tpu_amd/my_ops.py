@@ -48,9 +48,10 @@ _lib.define("moe_permute(Tensor ids, int num_experts) -> (Tensor, Tensor, Tensor
 _lib.define("moe_pack_weights(Tensor gate_weights, Tensor up_weights, Tensor down_weights, Tensor gate_scales, "
             "Tensor up_scales, Tensor down_scales) -> (Tensor, Tensor, Tensor, Tensor)")
 
-_lib.define("mlp_w8a16_dq_forward(Tensor input, Tensor gate_weight, Tensor up_weight, Tensor down_weight, "
+# the forms of the dense ops that the C++ ops do not run themselves (same arguments, same result)
+_lib.define("_mlp_general(Tensor input, Tensor gate_weight, Tensor up_weight, Tensor down_weight, "
             "Tensor gate_scale, Tensor up_scale, Tensor down_scale, Tensor(a!) output, int blocksize) -> Tensor(a!)")
-_lib.define("mm_w8a16_dq_forward(Tensor input, Tensor weight, Tensor scale, Tensor(a!) output, int blocksize) "
+_lib.define("_mm_general(Tensor input, Tensor weight, Tensor scale, Tensor(a!) output, int blocksize) "
             "-> Tensor(a!)")
 _lib.define("mlp_w8a8_quant_forward(Tensor input, Tensor gate_weight, Tensor up_weight, Tensor down_weight, "
             "Tensor gate_scale, Tensor up_scale, Tensor down_scale, Tensor(a!) output, int blocksize) -> Tensor(a!)")
@@ -465,9 +466,9 @@ def _mm_w8a16_dq_forward(input, weight, scale, output, blocksize):
 
 
 _lib.impl("_fused_experts_general", _fused_experts, "CompositeExplicitAutograd")
-_lib.impl("mlp_w8a16_dq_forward", _mlp_w8a16_dq_forward, "CompositeExplicitAutograd")
+_lib.impl("_mlp_general", _mlp_w8a16_dq_forward, "CompositeExplicitAutograd")
 _lib.impl("mlp_w8a8_quant_forward", _mlp_w8a8_quant_forward, "CompositeExplicitAutograd")
-_lib.impl("mm_w8a16_dq_forward", _mm_w8a16_dq_forward, "CompositeExplicitAutograd")
+_lib.impl("_mm_general", _mm_w8a16_dq_forward, "CompositeExplicitAutograd")
 _lib.impl("moe_route", _moe_route, "CompositeExplicitAutograd")
 _lib.impl("moe_permute", _moe_permute, "CompositeExplicitAutograd")
 _lib.impl("moe_pack_weights", _moe_pack_weights, "CompositeExplicitAutograd")
