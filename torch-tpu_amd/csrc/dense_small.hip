@@ -5,7 +5,8 @@
 // unit: it owns one 16-row weight tile for a slice of the reduction and up to 64 token rows, keeps
 // everything in registers (no LDS, no barrier, operands loaded straight into matrix-instruction
 // layout), and several wavefronts per SIMD hide each other's load latency.  Slices of the
-// reduction are summed by a second, tiny kernel in a fixed order, so results are reproducible.
+// reduction are summed by a second, tiny kernel in a fixed order, so results are reproducible -
+// or, in a narrow layer of at most 64 rows, inside a workgroup (dense_narrow_kernel).
 #include <type_traits>
 #include "moe_common.h"
 #include "moe_layout.h"
