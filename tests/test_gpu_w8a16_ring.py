@@ -31,3 +31,24 @@ def test_codes_converted_a_step_ahead(pkg, dev, T, H, I, E, K):
     # a neighbouring bf16 (2^-7 of the value) in the intermediate or the result, and its echo in sums that cancel
     assert ((gf - wf).abs() <= 1.6e-2 * wf.abs() + 2e-3 * wf.pow(2).mean().sqrt()).all()
     assert (got.view(torch.int16) == want.view(torch.int16)).float().mean().item() >= 0.97
+
+
+@pytest.mark.parametrize("M,K,N", [(100, 128, 128), (100, 384, 128), (100, 640, 272), (3000, 1408, 4096), (100, 512, 128)])
+def test_an_infinite_activation_in_the_last_step_stays_infinite(pkg, dev, M, K, N):
+    """128- and 192-row tiles, an odd number of 128-blocks (and an even one): no step past the reduction's end touches the
+    last token tile.  Against the de-quantised operands' product in 64 bits: the same elements are +Inf, -Inf and NaN (an
+    infinity against a zero code), every other row is finite."""
+    g = torch.Generator().manual_seed(M + K)
+    w = (torch.randn(N, K, generator=g) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)
+    s = torch.rand(-(-N // 128), K // 128, generator=g) + 0.5
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    cols = {3: K - 1, 40: K - 64, M - 1: K - 33, 17: 5}
+    for row, col in cols.items():
+        x[row, col] = float("inf") if col % 2 else float("-inf")
+    got = pkg.mm_w8a16(x.to(dev), pkg.pack_weights(w.to(dev)), s.to(dev)).float().cpu()
+    rows = list(cols)
+    wd = w.double() * s.double().repeat_interleave(128, 0)[:N].repeat_interleave(128, 1)
+    want = x[rows].double() @ wd.t()
+    assert torch.equal(got[rows].isnan(), want.isnan())
+    assert torch.equal(got[rows].isposinf(), want.isposinf()) and torch.equal(got[rows].isneginf(), want.isneginf())
+    assert got[[i for i in range(M) if i not in cols]].isfinite().all()

@@ -398,13 +398,13 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   constexpr int LPT = DQ ? 1 : 2;                      // load instructions per weight tile and step (1 KB each)
   constexpr int WSTEP = 1024 * LPT;                    // bytes of a tile's step in memory
   constexpr int L_STEP = NTOK + LPT * WT;              // loads per wavefront and step (scale chunks come on top)
-  // WREG: weight fragments ride in a register ring of R steps.  DQ: a step of codes is half as many bytes, so the ring
+  // WREG: weight fragments ride in a register ring of RING steps.  DQ: a step of codes is half as many bytes, so the ring
   // is twice as long for as much in flight (the half tile's four weight tiles per wavefront leave no registers for that)
-  constexpr int R = DQ && NW == 8 ? 2 * DEPTH : DEPTH;
-  v4i wlo[WREG ? R : 1][WT], whi[WREG ? R : 1][WT];
+  constexpr int RING = DQ && NW == 8 ? 2 * DEPTH : DEPTH;
+  v4i wlo[WREG ? RING : 1][WT], whi[WREG ? RING : 1][WT];
   if constexpr (WREG && DQ) {
 #pragma unroll
-    for (int d = 0; d < R; d++)
+    for (int d = 0; d < RING; d++)
 #pragma unroll
       for (int j = 0; j < WT; j++) wlo[d][j] = (v4i){0, 0, 0, 0};
   }
@@ -582,7 +582,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
       stage = stage + 1 == STAGES ? 0 : stage + 1;
     }
   } else {
-    // Large tiles: weights in a register ring of two steps, token tiles three steps ahead through
+    // Large tiles: weights in a register ring of two steps (DQ: four), token tiles three steps ahead through
     // four LDS stages, and ONE software pipeline over all m-tiles of all steps: the LDS reads of
     // m-tile g+2 and the scale multiply-adds of m-tile g-1 are issued around the matrix
     // instructions of m-tile g, across step boundaries.  For that the token tile of step s+1 is
@@ -592,14 +592,14 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     // Requests past the last step re-read it (cheap cache hits) instead of branching; a step past
     // an odd count multiplies by the zero weight scale stored behind the table.  The loop body is
     // instantiated per number of live m-tiles, so there is no branch between matrix instructions.
-    static_assert(DEPTH == 2, "the register ring holds two steps");
-    // R ring slots = steps per pass of the unrolled loop
+    static_assert(DEPTH == 2, "operands two steps ahead");
     constexpr int XB = 4;                                // token operand buffers; R * LIVE is a multiple of it
-    constexpr int L_WAIT = NTOK + LPT * WT * (R / 2);    // loads younger than the ones a step boundary needs
     const int last = NKB - 1;
     const int o0 = tok_chunk0(lg, li), o1 = tok_chunk1(lg, li);
-    auto run = [&](auto live_c) {
+    auto run = [&](auto live_c, auto ring_c) {
       constexpr int LIVE = decltype(live_c)::value;
+      constexpr int R = decltype(ring_c)::value;         // ring slots in use = steps per pass of the unrolled loop
+      constexpr int L_WAIT = NTOK + LPT * WT * (R / 2);  // loads younger than the ones a step boundary needs
       static_assert(LIVE % 2 == 0 && LIVE >= 2 && LIVE <= MT, "live m-tiles come in pairs");
       constexpr int PD = 2;                              // m-tiles between an LDS read and its use
       const bool top_empty = mt_live < LIVE;             // uniform: the top m-tile of the top pair holds no row
@@ -780,15 +780,22 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
         for (int r = 0; r < 4; r++) acc[0][j][r] = fmaf(p[1][j][r], f, acc[0][j][r]);
       }
     };
-    auto pick = [&](auto self, auto live_c) -> void {
+    auto pick = [&](auto self, auto live_c, auto ring_c) -> void {
       constexpr int LIVE = decltype(live_c)::value;
-      if constexpr (LIVE >= MT) run(std::integral_constant<int, MT>{});
-      else if (mt_live <= LIVE) run(live_c);
-      else self(self, std::integral_constant<int, LIVE + 2>{});
+      if constexpr (LIVE >= MT) run(std::integral_constant<int, MT>{}, ring_c);
+      else if (mt_live <= LIVE) run(live_c, ring_c);
+      else self(self, std::integral_constant<int, LIVE + 2>{}, ring_c);
     };
-    // (with the long ring of DQ the body for two m-tiles is left out: the compiler moves a ring slot at the end of that
-    // body's loop while the slot's load is in flight, which the static check of the assembly refuses)
-    pick(pick, std::integral_constant<int, (R > 2 ? 4 : 2)>{});
+    using short_ring = std::integral_constant<int, 2>;
+    // DQ: NKB is even (two steps to a 128-block), so two slots never run past the end.  A pass over four would, whenever the
+    // number of blocks is odd: two steps of zero weights against the last token tile, which cost as much as real ones and
+    // make an infinite activation NaN.  Those reductions use two of the slots (1408 x 1408, 16 experts, 1200 tokens 76.7 ->
+    // 72.2 us, 128 x 128 35.8 -> 31.9 us).
+    // (with four the body for two m-tiles is left out: the compiler moves a ring slot at the end of that body's loop while
+    // the slot's load is in flight, which the static check of the assembly refuses)
+    if constexpr (RING == 2) pick(pick, std::integral_constant<int, 2>{}, short_ring{});
+    else if (NKB % RING) pick(pick, std::integral_constant<int, 4>{}, short_ring{});
+    else pick(pick, std::integral_constant<int, 4>{}, std::integral_constant<int, RING>{});
   }
   __syncthreads();
 
