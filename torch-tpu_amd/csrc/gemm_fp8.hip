@@ -791,11 +791,17 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     // number of blocks is odd: two steps of zero weights against the last token tile, which cost as much as real ones and
     // make an infinite activation NaN.  Those reductions use two of the slots (1408 x 1408, 16 experts, 1200 tokens 76.7 ->
     // 72.2 us, 128 x 128 35.8 -> 31.9 us).
-    // (with four the body for two m-tiles is left out: the compiler moves a ring slot at the end of that body's loop while
-    // the slot's load is in flight, which the static check of the assembly refuses)
-    if constexpr (RING == 2) pick(pick, std::integral_constant<int, 2>{}, short_ring{});
-    else if (NKB % RING) pick(pick, std::integral_constant<int, 4>{}, short_ring{});
-    else pick(pick, std::integral_constant<int, 4>{}, std::integral_constant<int, RING>{});
+    // A tile of at most 32 rows uses two slots as well: with four the body for two m-tiles does not come out right (the
+    // compiler moves a ring slot at the end of its loop while the slot's load is in flight, which the static check of the
+    // assembly refuses), and the body for four does up to twice the matrix instructions (4096 x 4096, 64 experts, 533 tokens
+    // of which 45 experts hold at most 32 rows 840 -> 794 us).
+    if constexpr (RING == 2) {
+      pick(pick, std::integral_constant<int, 2>{}, short_ring{});
+    } else {
+      if (mt_live <= 2) run(std::integral_constant<int, 2>{}, short_ring{});
+      else if (NKB % RING) pick(pick, std::integral_constant<int, 4>{}, short_ring{});
+      else pick(pick, std::integral_constant<int, 4>{}, std::integral_constant<int, RING>{});
+    }
   }
   __syncthreads();
 
