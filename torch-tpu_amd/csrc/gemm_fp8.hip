@@ -790,7 +790,10 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     // DQ: NKB is even (two steps to a 128-block), so two slots never run past the end.  A pass over four would, whenever the
     // number of blocks is odd: two steps of zero weights against the last token tile, which cost as much as real ones and
     // make an infinite activation NaN.  Those reductions use two of the slots (1408 x 1408, 16 experts, 1200 tokens 76.7 ->
-    // 72.2 us, 128 x 128 35.8 -> 31.9 us).
+    // 72.2 us, 128 x 128 35.8 -> 31.9 us).  Short reductions too: what four slots ask for past the end is then a fair share of
+    // all loads (2048 x 768, 32 and 12 steps, 128 experts, 960 tokens 190.4 us with four slots, 185.6 with two; 48 steps of
+    // the 3072 x 1536 shape at 800 tokens 168.6 and 168.8, 64 of the 4096 x 4096 one at 533 tokens 640 and 651).
+    constexpr int kLongRingMinSteps = 40;
     // A tile of at most 32 rows uses two slots as well: with four the body for two m-tiles does not come out right (the
     // compiler moves a ring slot at the end of its loop while the slot's load is in flight, which the static check of the
     // assembly refuses), and the body for four does up to twice the matrix instructions (4096 x 4096, 64 experts, 533 tokens
@@ -799,7 +802,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
       pick(pick, std::integral_constant<int, 2>{}, short_ring{});
     } else {
       if (mt_live <= 2) run(std::integral_constant<int, 2>{}, short_ring{});
-      else if (NKB % RING) pick(pick, std::integral_constant<int, 4>{}, short_ring{});
+      else if (NKB % RING || NKB < kLongRingMinSteps) pick(pick, std::integral_constant<int, 4>{}, short_ring{});
       else pick(pick, std::integral_constant<int, 4>{}, std::integral_constant<int, RING>{});
     }
   }
