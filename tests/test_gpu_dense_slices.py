@@ -44,3 +44,29 @@ def test_gated_mlp_of_few_rows_on_the_grouped_kernels(pkg, dev, M, H, I):
     d = (got - want).abs()
     rms = want.pow(2).mean().sqrt()
     assert (d <= 2.0 ** -7 * want.abs() + 0.02 * rms).all() and d.pow(2).mean().sqrt() <= 0.006 * rms
+
+
+# reductions that end inside a batch of steps: per-wavefront kernels (four and two steps a batch), sliced products on the tall
+# tiles with an odd number of steps in the last slice
+@pytest.mark.parametrize("M,K,N", [(1, 2304, 256), (1, 4096, 256), (1, 14336, 256), (16, 5120, 1024), (32, 2304, 256),
+                                   (64, 18048, 128), (520, 16512, 1024), (150, 18560, 4096)])
+def test_an_infinite_scale_in_the_last_step_adds_no_nan(pkg, dev, M, K, N):
+    """The quantised operands' product, group by group, in 64 bits: an activation group whose scale is infinite gives
+    infinities of the same signs, not the NaN of a step past the end that counts it times zero."""
+    g = torch.Generator().manual_seed(M + K)
+    w = (torch.randn(N, K, generator=g) * 100).clamp(-448, 448).to(torch.float8_e4m3fn).to(dev)
+    ws = (torch.rand(-(-N // 128), K // 128, generator=g) + 0.5).to(dev)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    rows = sorted({0, M // 2, M - 1})
+    cols = [K - 1, K // 2 + 3, 128 * (K // 2048) + 383]
+    for i, col in enumerate(cols):                        # one infinity in a row; with one row, one call for each
+        for row in rows[i:i + 1] if M > 1 else [0]:
+            xi = x.clone()
+            xi[row, col] = float("inf")
+            xi = xi.to(dev)
+            got = pkg.mm_fp8(xi, pkg.pack_weights(w), ws)[row].float()
+            q, s = pkg.act_quant(xi[row:row + 1])
+            p = (q.double().view(K // 128, 1, 128) @ w.double().view(N, K // 128, 128).permute(1, 2, 0)).squeeze(1)
+            want = (p * (s[0, :K // 128, None].double() * ws.double().repeat_interleave(128, 0)[:N].t())).sum(0)
+            assert torch.equal(got.isnan(), want.isnan()), (row, col, got.isnan().sum().item(), want.isnan().sum().item())
+            assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())

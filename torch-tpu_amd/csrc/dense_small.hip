@@ -187,13 +187,14 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void dense_narrow_kernel(const S
   v4f acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; mt++) acc[mt] = (v4f){0.f, 0.f, 0.f, 0.f};
-  for (int kb = kb0; kb < kb1; kb += U) {
+  auto batch = [&](int kb, auto whole_c) {
+    constexpr bool whole = decltype(whole_c)::value;
     v4i wl[U], wh[U], xl[U][MT], xh[U][MT];
     float f[U][MT];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      const int kk = min(kb + u, kb1 - 1);               // past the slice: the last step again, times zero
-      const float sb = kb + u < kb1 ? wsp[kk] : 0.f;
+      const int kk = whole ? kb + u : min(kb + u, kb1 - 1);      // past the slice: the last step again, left out below
+      const float sb = wsp[kk];
       const v4i *lo = (const v4i *)(wp + (size_t)kk * 2048);
       wl[u] = lo[0]; wh[u] = lo[64];
 #pragma unroll
@@ -204,7 +205,8 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void dense_narrow_kernel(const S
       }
     }
 #pragma unroll
-    for (int u = 0; u < U; u++)
+    for (int u = 0; u < U; u++) {
+      if (!whole && kb + u >= kb1) break;                // (counted times zero, an infinite scale would make NaN)
 #pragma unroll
       for (int mt = 0; mt < MT; mt++) {
         const v4f zero = {0.f, 0.f, 0.f, 0.f};
@@ -213,7 +215,11 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void dense_narrow_kernel(const S
 #pragma unroll
         for (int r = 0; r < 4; r++) acc[mt][r] = fmaf(p[r], f[u][mt], acc[mt][r]);
       }
-  }
+    }
+  };
+  int kb = kb0;
+  for (; kb + U <= kb1; kb += U) batch(kb, std::true_type{});
+  if (kb < kb1) batch(kb, std::false_type{});
 #pragma unroll
   for (int mt = 0; mt < MT; mt++) part[wave][mt][lane] = acc[mt];
   __syncthreads();

@@ -644,7 +644,10 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
         if constexpr (BF16) return;
         if (tid < BM) {
           const int kc = min(k, last);                   // past the end: a finite scale times the zero behind the table
-          const float sa = sm.sac[(kc >> 4) & 1][(tid >> 4) * 256 + ((kc & 12) << 4) + (tid & 15) * 4 + (kc & 3)];
+          float sa = sm.sac[(kc >> 4) & 1][(tid >> 4) * 256 + ((kc & 12) << 4) + (tid & 15) * 4 + (kc & 3)];
+          // (an infinite scale would make NaN of the zero.  The whole products leave it at that: the select costs 1 % of a
+          // prefill layer, and a register that the 96-row kernel does not have)
+          if (SLICED && k > last) sa = 0.f;
           sm.fsc[k & 3][tid] = make_float2(sa * sm.sb[0][k], sa * sm.sb[1][k]);
         }
       };
