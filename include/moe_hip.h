@@ -261,6 +261,13 @@ int moe_fused_experts_w8a16(void *stream, const void *x_bf16, int T, int H, cons
  * activations per row and 128 columns, as the expert path does; the matrix products run in FP8.
  */
 size_t moe_mm_fp8_workspace_bytes(int M, int K, int N);
+/* What moe_mm_fp8 runs for a shape: plan[0] one of MOE_PLAN_*, plan[1] token rows of a work item, plan[2] slices of the
+ * reduction, plan[3] 128-steps of a slice (the last one may be shorter).  For tests and tuning; no GPU is touched. */
+#define MOE_PLAN_GROUPED        0   /* the grouped kernel, whole reduction                              */
+#define MOE_PLAN_GROUPED_SLICED 1   /* the grouped kernel, slices added by a second launch              */
+#define MOE_PLAN_WAVEFRONT      2   /* a wavefront per work item, slices added by a second launch       */
+#define MOE_PLAN_NARROW         3   /* a workgroup per 16 columns, the reduction sliced over its wavefronts */
+int moe_mm_fp8_plan(int M, int K, int N, int *plan);
 int moe_mm_fp8(void *stream, const void *x_bf16, int M, int K, const uint8_t *w, const float *w_scale, int N,
                void *out_bf16, void *workspace, size_t workspace_bytes);
 /*

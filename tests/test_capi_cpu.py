@@ -306,3 +306,14 @@ def test_bench_refuses_more_than_one_gpu_and_its_power_roof_is_plain_arithmetic(
     assert abs(roof["floor_ms"] - 1.3 / 1100.0 * 1e3) < 1e-9
     assert bench.power_roof(dict(power, idle_watts=1500.0), 1, 1, 1) is None           # a cap below idle: no roof
     assert bench.power_roof(dict(power, read_probe=None), 1, 1, 1) is None             # counters unreadable
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [
+    # one workgroup per 16 columns while its rows' reduction stays short: 2048 -> 4096 row-steps by tile height
+    (1, 7168, 1536, "narrow"), (32, 7168, 1536, "narrow"), (16, 32768, 2048, "narrow"), (17, 14336, 4096, "narrow"),
+    (32, 8192, 4096, "narrow"), (32, 14336, 4096, "wavefront"), (32, 16384, 3072, "wavefront"), (64, 4096, 4096, "narrow"),
+    (64, 8192, 3072, "wavefront"), (64, 14336, 4096, "wavefront"), (48, 12288, 3072, "wavefront"), (16, 32768, 16, "wavefront"),
+    (1, 32768, 16, "narrow"), (64, 7168, 4112, "wavefront"),
+])
+def test_dense_products_of_few_rows_take_the_kernel_that_measured_faster(pkg, M, K, N, kernel):
+    assert pkg.ops.mm_plan(M, K, N)[0] == kernel

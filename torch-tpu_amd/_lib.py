@@ -5,7 +5,7 @@ module raises, and every op built on it is unavailable.
 """
 import ctypes
 import os
-from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
+from ctypes import POINTER, c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libmoe_hip.so")
@@ -58,6 +58,7 @@ SIGNATURES = {
     "moe_router_logits_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
     "moe_router_logits": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_size_t]),
     "moe_mm_fp8_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
+    "moe_mm_fp8_plan": (c_int, [c_int, c_int, c_int, POINTER(c_int)]),
     "moe_mm_fp8": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_size_t]),
     "moe_mm_bf16": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_void_p]),
     "moe_mm_w8a16": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p]),

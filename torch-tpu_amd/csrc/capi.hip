@@ -40,6 +40,9 @@ int route_from_partials_launch(hipStream_t st, const float *partial, int n_slice
                                int32_t *chunk_counts = nullptr);
 
 size_t dense_small_partial_bytes(int M, int K, int N, bool keep_partial);
+int dense_narrow_mt(int M, int K, int N);
+void dense_small_plan(int M, int K, int N, int *n_splits, int *split_len, int *rows_per_item, int *n_mchunks,
+                      int *tiles_per_item);
 int dense_small_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M, int K, const uint8_t *w, const float *ws,
                        int N, uint16_t *out, float *partial, int *n_splits_out);
 int dense_product_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M, int K, const uint8_t *w, const float *ws,
@@ -584,6 +587,27 @@ static DenseWs dense_layout(void *base, int M, int K, int I, int N = 0) {
 extern "C" size_t moe_mm_fp8_workspace_bytes(int M, int K, int N) {
   if (M < 0 || K < 1 || N < 16 || K % moe::kBlock || N % 16) return 0;
   return moe::dense_layout(nullptr, M, K, 0, N).bytes;
+}
+
+extern "C" int moe_mm_fp8_plan(int M, int K, int N, int *plan) {
+  using namespace moe;
+  if (!plan) return MOE_E_NULL;
+  if (M < 0 || K < 1 || N < 16 || K > 32768 || N > (1 << 20)) return MOE_E_SHAPE;
+  if (K % kBlock || N % 16) return MOE_E_ALIGN;
+  if (!mm_uses_small_kernel(M, K, N)) {
+    const DenseSplit sp = dense_split(M, K, N);
+    plan[0] = sp.slices > 1 ? MOE_PLAN_GROUPED_SLICED : MOE_PLAN_GROUPED;
+    // (an unsliced product of at most 128 rows takes the tile of its row count)
+    plan[1] = sp.slices > 1 || M > 128 ? sp.tile_m : choose_tile_m(M, 1, 1);
+    plan[2] = sp.slices; plan[3] = sp.k_steps;
+  } else if (const int mt = dense_narrow_mt(M, K, N)) {
+    plan[0] = MOE_PLAN_NARROW; plan[1] = 16 * mt; plan[2] = 1; plan[3] = K / kBlock;
+  } else {
+    int chunks, tiles;
+    plan[0] = MOE_PLAN_WAVEFRONT;
+    dense_small_plan(M, K, N, &plan[2], &plan[3], &plan[1], &chunks, &tiles);
+  }
+  return MOE_OK;
 }
 
 extern "C" int moe_mm_fp8(void *stream, const void *x_bf16, int M, int K, const uint8_t *w, const float *w_scale,

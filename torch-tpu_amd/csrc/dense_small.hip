@@ -160,7 +160,8 @@ __global__ __launch_bounds__(64 * kDsWaves) void dense_small_kernel(const SmallA
 // 16-column weight tile for 16 MT token rows and the whole reduction, a sixteenth of it per wavefront; the slices meet in
 // LDS and are added in slice order.  Against items of one wavefront with the slices in memory that saves the launch that
 // adds them (5 us and a gap, more than such a product itself takes); what it gives up is the reuse of a token operand
-// over several weight tiles, so it is for layers whose tiles just about fill the compute units (dense_narrow_mt).
+// over several weight tiles, so it is for layers whose tiles just about fill the compute units and whose reduction is not too
+// long for its rows (dense_narrow_mt).
 constexpr int kNarrowWaves = 16, kNarrowMaxWgs = 256;
 template <int MT>
 __global__ __launch_bounds__(64 * kNarrowWaves) void dense_narrow_kernel(const SmallArgs a) {
@@ -239,15 +240,23 @@ __global__ __launch_bounds__(64 * kNarrowWaves) void dense_narrow_kernel(const S
 }
 
 // m-tiles per workgroup of that kernel, 0: the layer is not one for it.  The smallest count whose workgroups all run at
-// once, one per compute unit (its sixteen wavefronts fill half of one).  Whole op with the quantiser's launch, before ->
-// after: 7168 -> 1536 at 1 / 16 / 32 / 64 rows 10.6 / 13.1 / 15.0 / 19.2 -> 7.2 / 10.9 / 11.0 / 16.1 us, 16384 -> 1024 15.9 / 19.3 /
-// 19.9 -> 9.3 / 17.9 / 18.4, 4096 -> 4096 at 1 / 16 / 17 / 64 rows 10.1 / 12.9 / 12.8 / 19.2 -> 7.4 / 12.1 / 9.5 / 17.2.  With
-// more workgroups than that it loses: 7168 -> 7168 at 32 / 64 rows 20 / 27 -> 30 / 48 us.
+// once, one per compute unit (its sixteen wavefronts fill half of one), as long as the token operand stays small: a
+// workgroup fetches its rows' whole reduction, a line per row and half step, for one weight tile, where the sliced kernel
+// shares it among four tiles or spreads it over many units - so the limit is on rows x steps of a workgroup.  Whole op with
+// the quantiser's launch, sliced -> narrow in us, one m-tile: 7168 -> 1536 at 1 / 16 / 32 rows 10.8 / 13.5 / 14.8 -> 6.8 / 9.6 /
+// 9.7, 16384 -> 1024 15.5 / 19.5 / 19.9 -> 9.0 / 15.0 / 15.3, 12288 -> 2048 at 16 rows 15.8 -> 13.4; only a layer of a few
+// tiles gives the sliced kernel a short enough sum to win from 2048 on (32768 -> 16 at 16 rows 23.6 -> 27).  Two: 4096 -> 4096
+// at 17 / 32 rows 12.8 / 13.7 -> 9.3 / 10.8, 8192 -> 4096 at 32 rows 18.4 -> 16.2, 16384 -> 3072 at 32 rows 21.6 -> 26.1.  Four:
+// 4096 -> 4096 at 64 rows 18.9 -> 17.2, 8192 -> 3072 at 64 rows 22.2 -> 28.1, 14336 -> 4096 at 64 rows 29.2 -> 45.  With more
+// workgroups than units it loses: 7168 -> 7168 at 32 / 64 rows 20 / 27 -> 30 / 48 us.
 int dense_narrow_mt(int M, int K, int N) {
   if (M > 64 || K < 2048) return 0;
   for (int mt = 1; mt <= 4; mt *= 2) {
     const long chunks = (M + 16 * mt - 1) / (16 * mt);
-    if ((long)(N / 16) * chunks <= kNarrowMaxWgs) return mt;
+    if ((long)(N / 16) * chunks > kNarrowMaxWgs) continue;
+    const int row_steps = (M < 16 * mt ? M : 16 * mt) * (K / kBlock);
+    const bool fits = mt == 1 ? N >= 128 || row_steps <= 2048 : row_steps <= (mt == 2 ? 3100 : 2400);
+    return fits ? mt : 0;
   }
   return 0;
 }

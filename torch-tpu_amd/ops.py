@@ -8,6 +8,8 @@ non-zero return, as the reference's ops raise through TORCH_CHECK
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from ._lib import MoeHipError, check, lib
@@ -337,6 +339,14 @@ def fused_experts_bf16_workspace_bytes(T, H, I, E, K) -> int:
 
 def mm_workspace_bytes(M, K, N) -> int:
     return lib.moe_mm_fp8_workspace_bytes(M, K, N)
+
+
+def mm_plan(M, K, N):
+    """What mm_fp8 runs for a shape -> (kernel, token rows of a work item, slices of the reduction, 128-steps of a slice);
+    kernel: "grouped" | "sliced" | "wavefront" | "narrow"."""
+    plan = (ctypes.c_int * 4)()
+    check(lib.moe_mm_fp8_plan(M, K, N, plan), "mm_plan")
+    return ("grouped", "sliced", "wavefront", "narrow")[plan[0]], plan[1], plan[2], plan[3]
 
 
 def mlp_workspace_bytes(M, H, I) -> int:
