@@ -314,6 +314,11 @@ def test_bench_refuses_more_than_one_gpu_and_its_power_roof_is_plain_arithmetic(
     (32, 8192, 4096, "narrow"), (32, 14336, 4096, "wavefront"), (32, 16384, 3072, "wavefront"), (64, 4096, 4096, "narrow"),
     (64, 8192, 3072, "wavefront"), (64, 14336, 4096, "wavefront"), (48, 12288, 3072, "wavefront"), (16, 32768, 16, "wavefront"),
     (1, 32768, 16, "narrow"), (64, 7168, 4112, "wavefront"),
+    # a reduction of 16384 or more from 33 rows on: sliced on the grouped kernel, but for the narrow kernel's layers and for a
+    # single strip of columns
+    (33, 16384, 1024, "narrow"), (64, 24576, 1024, "narrow"), (64, 32768, 1024, "sliced"), (33, 16384, 4096, "sliced"),
+    (65, 16384, 1024, "sliced"), (100, 16384, 256, "wavefront"), (500, 16384, 256, "wavefront"), (513, 16384, 256, "sliced"),
+    (100, 18432, 256, "wavefront"), (100, 24576, 256, "sliced"), (32, 18432, 7168, "wavefront"), (33, 18432, 7168, "sliced"),
 ])
 def test_dense_products_of_few_rows_take_the_kernel_that_measured_faster(pkg, M, K, N, kernel):
     assert pkg.ops.mm_plan(M, K, N)[0] == kernel
