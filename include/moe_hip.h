@@ -259,6 +259,8 @@ int moe_fused_experts_w8a16(void *stream, const void *x_bf16, int T, int H, cons
  * (silu(x Wg^T) * (x Wu^T)) Wd^T with w13 [2I, H] = gate rows then up rows, w2 [H, I].
  * Unlike the reference (bf16 activations against de-quantised weights) both quantise the
  * activations per row and 128 columns, as the expert path does; the matrix products run in FP8.
+ * Workspace: what the *_workspace_bytes functions return for M rows serves every batch of at most M rows (the slices that
+ * a middle-sized batch needs are more than those of a large one), 256-byte aligned.
  */
 size_t moe_mm_fp8_workspace_bytes(int M, int K, int N);
 /* What moe_mm_fp8 runs for a shape: plan[0] one of MOE_PLAN_*, plan[1] token rows of a work item, plan[2] slices of the

@@ -322,3 +322,22 @@ def test_bench_refuses_more_than_one_gpu_and_its_power_roof_is_plain_arithmetic(
 ])
 def test_dense_products_of_few_rows_take_the_kernel_that_measured_faster(pkg, M, K, N, kernel):
     assert pkg.ops.mm_plan(M, K, N)[0] == kernel
+
+
+@pytest.mark.parametrize("K,N", [(7168, 1536), (14336, 4096), (16384, 256), (16384, 1024), (18432, 7168), (2304, 4096),
+                                 (12288, 12288), (17280, 128), (2048, 7168), (32768, 28672)])
+def test_dense_workspace_of_a_batch_serves_every_smaller_one(pkg, K, N):
+    """The size never falls with the rows; it holds the quantised operand and the slices that the plan of any smaller batch
+    cuts, in a product alone and as the second product of a gated MLP."""
+    lib = pkg._lib.lib
+    up = lambda n: (n + 255) // 256 * 256
+    rows = sorted({*range(0, 140), *range(144, 1500, 13), *range(1500, 20000, 611), 128, 384, 512, 513, 1 << 20})
+    mm = [lib.moe_mm_fp8_workspace_bytes(m, K, N) for m in rows]
+    mlp = [lib.moe_mlp_fp8_workspace_bytes(m, N, K) for m in rows] if N % 128 == 0 else [0]
+    assert all(a <= b for a, b in zip(mm, mm[1:])) and all(a <= b for a, b in zip(mlp, mlp[1:]))
+    most = 0
+    for m, size in zip(rows[1:], mm[1:]):
+        kernel, _, slices, _ = pkg.ops.mm_plan(m, K, N)
+        if slices > 1:
+            most = max(most, up(slices * m * N * 4))
+        assert size >= up(m * K) + up(m * lib.moe_scale_pitch(K // 128) * 4) + most, (m, kernel, slices)

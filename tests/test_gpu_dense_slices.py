@@ -70,3 +70,19 @@ def test_an_infinite_scale_in_the_last_step_adds_no_nan(pkg, dev, M, K, N):
             want = (p * (s[0, :K // 128, None].double() * ws.double().repeat_interleave(128, 0)[:N].t())).sum(0)
             assert torch.equal(got.isnan(), want.isnan()), (row, col, got.isnan().sum().item(), want.isnan().sum().item())
             assert torch.equal(got.isposinf(), want.isposinf()) and torch.equal(got.isneginf(), want.isneginf())
+
+
+def test_one_workspace_made_for_the_largest_batch_serves_the_smaller_ones(pkg, dev):
+    K, N, I, H = 14336, 4096, 16384, 1024
+    w, ws = (t[0] for t in pkg.synthetic_weights(1, N, K, dev, 5))
+    w13, s13 = (t[0] for t in pkg.synthetic_weights(1, 2 * I, H, dev, 6))
+    w2, s2 = (t[0] for t in pkg.synthetic_weights(1, H, I, dev, 7))
+    rows = (2048, 1, 30, 33, 64, 100, 128, 129, 300, 700, 768, 1100)
+    buf = [torch.empty(n, dtype=torch.uint8, device=dev) for n in (pkg.ops.mm_workspace_bytes(rows[0], K, N),
+                                                                   pkg.ops.mlp_workspace_bytes(rows[0], H, I))]
+    for M in rows:
+        g = torch.Generator().manual_seed(M)
+        x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
+        assert torch.equal(pkg.mm_fp8(x, w, ws, workspace=buf[0]), pkg.mm_fp8(x, w, ws)), M
+        x = torch.randn(M, H, generator=g).to(torch.bfloat16).to(dev)
+        assert torch.equal(pkg.mlp_fp8(x, w13, s13, w2, s2, workspace=buf[1]), pkg.mlp_fp8(x, w13, s13, w2, s2)), M

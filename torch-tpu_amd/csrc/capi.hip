@@ -1,6 +1,7 @@
 // The whole-path entry point and the library's housekeeping calls.
 #include <atomic>
 #include <mutex>
+#include <algorithm>
 #include "moe_common.h"
 #include "moe_layout.h"
 #include "act_quant.h"
@@ -560,7 +561,42 @@ struct DenseWs {
   float *partial1;    // MLP: slices of the first product
   size_t bytes;
 };
-static DenseWs dense_layout(void *base, int M, int K, int I, int N = 0) {
+// Bytes of the slices for M rows: of the only or second product, and of an MLP's first (MLP: K = H, N = H; first product
+// [M, 2I] over H, second [M, H] over I).
+static void dense_partial_bytes(int M, int K, int I, int N, size_t *first, size_t *last) {
+  *first = 0;
+  if (I > 0 ? mlp_uses_small_kernel(M, I) : mm_uses_small_kernel(M, K, N)) {
+    if (I > 0) *first = dense_small_partial_bytes(M, K, 2 * I, true);
+    *last = dense_small_partial_bytes(M, I > 0 ? I : K, N, false);
+  } else {
+    *last = dense_split_bytes(M, I > 0 ? I : K, N);
+  }
+}
+
+// The most that the slices take for any number of rows up to M: their number falls and rises with the rows (a batch that
+// fills the compute units is not sliced), and a buffer made for the largest batch has to serve the smaller ones.  Up to 64
+// rows every count is looked at.  Above, the kernels and the slices' number are the same for 16 rows in a row on the
+// per-wavefront kernels (up to 512 rows); on the grouped ones a model decides whose tile counts change at multiples of 32
+// and in which more rows only speak for fewer slices, so the first row's slices and the last row bound what lies between.
+static size_t dense_partials_bound(int M, int K, int I, int N) {
+  size_t most = 0;
+  const auto see = [&](int rows, int plan_rows) {
+    size_t first, last;
+    dense_partial_bytes(plan_rows, K, I, N, &first, &last);
+    const auto scaled = [&](size_t n) { return align_up(n / plan_rows * rows, 256); };       // (whole slices of rows)
+    const size_t sum = scaled(first) + scaled(last);
+    if (sum > most) most = sum;
+  };
+  for (int m = 1; m <= M && m <= 64; m++) see(m, m);
+  const int end = (int)std::min<long>(M, dense_split_max_rows(I > 0 ? I : K, N));
+  for (int lo = 65, step; lo <= end; lo += step) {
+    step = lo <= 512 ? 16 : 32;
+    see(std::min(lo + step - 1, end), lo);
+  }
+  return most;
+}
+
+static DenseWs dense_layout(void *base, int M, int K, int I, int N) {
   DenseWs w{};
   size_t off = 0;
   auto take = [&](size_t n) {
@@ -574,24 +610,26 @@ static DenseWs dense_layout(void *base, int M, int K, int I, int N = 0) {
     w.hq = (uint8_t *)take((size_t)M * I);
     w.hs = (float *)take((size_t)M * scale_pitch(I / kBlock) * 4);
   }
-  if (N > 0 && (I > 0 ? mlp_uses_small_kernel(M, I) : mm_uses_small_kernel(M, K, N))) {
-    if (I > 0) {      // MLP: K = H, N = H; first product [M, 2I] over H, second [M, H] over I
-      w.partial1 = (float *)take(dense_small_partial_bytes(M, K, 2 * I, true));
-      w.partial = (float *)take(dense_small_partial_bytes(M, I, N, false));
-    } else {
-      w.partial = (float *)take(dense_small_partial_bytes(M, K, N, false));
-    }
-  } else if (N > 0) {
-    w.partial = (float *)take(dense_split_bytes(M, I > 0 ? I : K, N));
-  }
+  size_t first = 0, last = 0;
+  if (M > 0) dense_partial_bytes(M, K, I, N, &first, &last);
+  if (first) w.partial1 = (float *)take(first);
+  if (last) w.partial = (float *)take(last);
   w.bytes = off;
   return w;
+}
+
+// What a caller is told to bring for up to M rows (a call asks for no more than its own layout)
+static size_t dense_workspace_bytes(int M, int K, int I, int N) {
+  DenseWs w = dense_layout(nullptr, M, K, I, N);
+  size_t first = 0, last = 0;
+  if (M > 0) dense_partial_bytes(M, K, I, N, &first, &last);
+  return w.bytes - align_up(first, 256) - align_up(last, 256) + dense_partials_bound(M, K, I, N);
 }
 }  // namespace moe
 
 extern "C" size_t moe_mm_fp8_workspace_bytes(int M, int K, int N) {
   if (M < 0 || K < 1 || N < 16 || K % moe::kBlock || N % 16) return 0;
-  return moe::dense_layout(nullptr, M, K, 0, N).bytes;
+  return moe::dense_workspace_bytes(M, K, 0, N);
 }
 
 extern "C" int moe_mm_fp8_plan(int M, int K, int N, int *plan) {
@@ -667,7 +705,7 @@ extern "C" int moe_mm_w8a16(void *stream, const void *x_bf16, int M, int K, cons
 
 extern "C" size_t moe_mlp_fp8_workspace_bytes(int M, int H, int I) {
   if (M < 0 || H < 1 || I < 1) return 0;
-  return moe::dense_layout(nullptr, M, H, I, H).bytes;
+  return moe::dense_workspace_bytes(M, H, I, H);
 }
 
 extern "C" int moe_mlp_fp8(void *stream, const void *x_bf16, int M, int H, const uint8_t *w13, const float *w13_scale,

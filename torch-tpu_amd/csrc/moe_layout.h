@@ -108,6 +108,13 @@ static inline DenseSplit dense_split(long rows, int K, int N) {
   }
   return best;
 }
+// No product of more rows is sliced: with q rounds of whole items of a tall tile the slices cost at least q (steps x step +
+// 40 000) cycles and the whole product at most 0.87 / 0.97 (q + 1)(steps x step + 20 000) - the tile that is chosen is at
+// most 1 / 0.97 dearer than any other, and not the 64-row one from four rounds on - which is less from q = 9 on.  (At least
+// 512: up to there the per-wavefront kernels have slices of their own.)
+static inline long dense_split_max_rows(int K, int N) {
+  return K / 128 > 16 ? 512 + 192 * (9 * 256 / ((N + 255) / 256) + 1l) : 512;
+}
 static inline size_t dense_split_bytes(long rows, int K, int N) {
   const DenseSplit s = dense_split(rows, K, N);
   return s.slices > 1 ? (size_t)s.slices * rows * N * 4 : 0;

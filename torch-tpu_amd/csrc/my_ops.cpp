@@ -130,11 +130,13 @@ struct DenseEntry {
   std::vector<SourceId> ids;
   std::vector<c10::weak_intrusive_ptr<c10::StorageImpl>> alive;
   std::vector<Tensor> made;
+  int64_t rows = 0;             // the largest batch seen and the workspace that covers it and every smaller one
+  size_t workspace_bytes = 0;
 };
 std::vector<DenseEntry> g_dense;
 
 template <typename Make>
-const std::vector<Tensor> &dense_packed(std::initializer_list<const Tensor *> src, Make make) {
+DenseEntry &dense_packed(std::initializer_list<const Tensor *> src, Make make) {
   std::vector<SourceId> ids;
   for (const Tensor *t : src) ids.push_back(identify(*t));
   for (size_t i = 0; i < g_dense.size();) {
@@ -145,7 +147,7 @@ const std::vector<Tensor> &dense_packed(std::initializer_list<const Tensor *> sr
       g_dense.pop_back();
       continue;
     }
-    if (g_dense[i].ids == ids) return g_dense[i].made;
+    if (g_dense[i].ids == ids) return g_dense[i];
     i++;
   }
   DenseEntry e;
@@ -153,7 +155,18 @@ const std::vector<Tensor> &dense_packed(std::initializer_list<const Tensor *> sr
   e.ids = std::move(ids);
   e.made = make();
   g_dense.push_back(std::move(e));
-  return g_dense.back().made;
+  return g_dense.back();
+}
+
+// Workspace of a call on M rows: asked for again only when a batch is larger than every one before it (the query looks at
+// all smaller batches), so that a layer's later, smaller calls never grow the scratch
+template <typename Query>
+size_t dense_workspace(DenseEntry &e, int64_t M, Query query) {
+  if (M > e.rows) {
+    e.workspace_bytes = query();
+    e.rows = M;
+  }
+  return e.workspace_bytes;
 }
 
 // what the common forms of the dense ops ask of their tensors; any other form takes the general road
@@ -345,10 +358,11 @@ Tensor mm_w8a16_dq_forward(const Tensor &input, const Tensor &weight, const Tens
     return call_general("my_ops::_mm_general", {input, weight, scale, output, blocksize});
   }
   void *st = stream_of(input);
-  const auto &w = dense_packed({&weight, &scale}, [&]() -> std::vector<Tensor> {
+  DenseEntry &entry = dense_packed({&weight, &scale}, [&]() -> std::vector<Tensor> {
     return {tile_block(weight.contiguous()), scale.to(at::kFloat).contiguous()};
   });
-  const size_t need = moe_mm_fp8_workspace_bytes((int)M, (int)K, (int)N);
+  const auto &w = entry.made;
+  const size_t need = dense_workspace(entry, M, [&] { return moe_mm_fp8_workspace_bytes((int)M, (int)K, (int)N); });
   Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
   check_rc(moe_mm_fp8(st, input.data_ptr(), (int)M, (int)K, (const uint8_t *)w[0].data_ptr(), w[1].data_ptr<float>(), (int)N,
                       output.data_ptr(), ws.data_ptr(), (size_t)ws.numel()),
@@ -371,11 +385,12 @@ Tensor mlp_w8a16_dq_forward(const Tensor &input, const Tensor &gate, const Tenso
     return call_general("my_ops::_mlp_general", {input, gate, up, down, gs, us, ds, output, blocksize});
   }
   void *st = stream_of(input);
-  const auto &w = dense_packed({&gate, &up, &down, &gs, &us, &ds}, [&]() -> std::vector<Tensor> {
+  DenseEntry &entry = dense_packed({&gate, &up, &down, &gs, &us, &ds}, [&]() -> std::vector<Tensor> {
     return {tile_block(at::cat({gate, up}, 0).contiguous()), at::cat({gs, us}, 0).to(at::kFloat).contiguous(),
             tile_block(down.t().contiguous()), ds.t().to(at::kFloat).contiguous()};
   });
-  const size_t need = moe_mlp_fp8_workspace_bytes((int)M, (int)H, (int)I);
+  const auto &w = entry.made;
+  const size_t need = dense_workspace(entry, M, [&] { return moe_mlp_fp8_workspace_bytes((int)M, (int)H, (int)I); });
   Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
   check_rc(moe_mlp_fp8(st, input.data_ptr(), (int)M, (int)H, (const uint8_t *)w[0].data_ptr(), w[1].data_ptr<float>(),
                        (const uint8_t *)w[2].data_ptr(), w[3].data_ptr<float>(), (int)I, output.data_ptr(), ws.data_ptr(),

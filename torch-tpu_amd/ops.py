@@ -9,6 +9,7 @@ non-zero return, as the reference's ops raise through TORCH_CHECK
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -337,7 +338,9 @@ def fused_experts_bf16_workspace_bytes(T, H, I, E, K) -> int:
     return lib.moe_fused_experts_bf16_workspace_bytes(T, H, I, E, K)
 
 
+@functools.lru_cache(maxsize=4096)
 def mm_workspace_bytes(M, K, N) -> int:
+    """Bytes of workspace for mm_fp8 on up to M rows (kept: the size looks at every smaller batch)."""
     return lib.moe_mm_fp8_workspace_bytes(M, K, N)
 
 
@@ -349,7 +352,9 @@ def mm_plan(M, K, N):
     return ("grouped", "sliced", "wavefront", "narrow")[plan[0]], plan[1], plan[2], plan[3]
 
 
+@functools.lru_cache(maxsize=4096)
 def mlp_workspace_bytes(M, H, I) -> int:
+    """Bytes of workspace for mlp_fp8 on up to M rows (kept: the size looks at every smaller batch)."""
     return lib.moe_mlp_fp8_workspace_bytes(M, H, I)
 
 
@@ -435,7 +440,7 @@ def mm_fp8(x, w, w_scale, out=None, workspace=None):
     if out is None:
         out = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
     _need(tuple(out.shape) == (M, N), "out must be [M,N]")
-    need = lib.moe_mm_fp8_workspace_bytes(M, K, N)
+    need = mm_workspace_bytes(M, K, N)
     if workspace is None:
         workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
     _need(workspace.numel() * workspace.element_size() >= need, "workspace too small")
@@ -490,7 +495,7 @@ def mlp_fp8(x, w13, w13_scale, w2, w2_scale, out=None, workspace=None):
     if out is None:
         out = torch.empty(M, H, dtype=torch.bfloat16, device=x.device)
     _need(tuple(out.shape) == (M, H), "out must be [M,H]")
-    need = lib.moe_mlp_fp8_workspace_bytes(M, H, I)
+    need = mlp_workspace_bytes(M, H, I)
     if workspace is None:
         workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
     _need(workspace.numel() * workspace.element_size() >= need, "workspace too small")
