@@ -1,7 +1,10 @@
 """The dense ops' native path against the general one: the same bits for every form both accept, and packed copies that
 follow their weights."""
+import gc
+
 import pytest
 import torch
+from torch.multiprocessing.reductions import StorageWeakRef
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +66,46 @@ def test_what_was_refused_stays_refused(pkg, dev):
     for bad in [(x.float(), w, s, out, 128), (x, w.to(torch.bfloat16), s, out, 128), (x, w, s, out.float(), 128), (x, w, s, out, 0)]:
         with pytest.raises((RuntimeError, TypeError, ValueError)):
             torch.ops.my_ops.mm_w8a16_dq_forward(*bad)
+
+
+def flat_views(dev, *parts):
+    """The parts as views of one storage, each 512-byte aligned."""
+    sizes = [(p.numel() * p.element_size() + 511) // 512 * 512 for p in parts]
+    flat = torch.zeros(sum(sizes), dtype=torch.uint8, device=dev)
+    views, at = [], 0
+    for p, n in zip(parts, sizes):
+        v = flat[at:at + p.numel() * p.element_size()].view(p.dtype).view(p.shape)
+        v.copy_(p)
+        views.append(v)
+        at += n
+    return views
+
+
+@pytest.mark.parametrize("form", ["one flat buffer", "parameters"])
+@pytest.mark.parametrize("op", ["mm", "mlp", "experts"])
+def test_packed_copy_does_not_keep_its_sources_alive(pkg, dev, op, form):
+    E, I, H = 4, 128, 256
+    x = torch.randn(3, H, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(dev)
+    lead = (E,) if op == "experts" else ()
+    tensors = []
+    for i in range(1 if op == "mm" else 3):
+        w, s = weights(dev, I * max(1, *lead, 1), H, i, torch.float32)
+        tensors += [w.view(*lead, I, H), s.view(*lead, I // 128, H // 128)]
+    if form == "parameters":
+        tensors = [torch.nn.Parameter(t, requires_grad=t.dtype == torch.float32) for t in tensors]
+    else:
+        tensors = flat_views(dev, *tensors)
+    alive = [StorageWeakRef(t.untyped_storage()) for t in tensors]
+    my_ops = torch.ops.my_ops
+    ids = torch.zeros(3, 1, dtype=torch.int32, device=dev)
+    if op == "mm":
+        my_ops.mm_w8a16_dq_forward(x, *tensors, torch.empty(3, I, dtype=torch.bfloat16, device=dev), 128)
+    elif op == "mlp":
+        my_ops.mlp_w8a16_dq_forward(x, *tensors[::2], *tensors[1::2], torch.empty_like(x), 128)
+    else:
+        my_ops.fused_moe_fused_experts(torch.empty_like(x), x, None, None, *tensors[::2], *tensors[1::2], ids, ids.float(), None,
+                                       None, None, 128, E, 1, False, 1, 1, None, None, None, False)
+    torch.cuda.synchronize()
+    del tensors, w, s
+    gc.collect()
+    assert all(a.expired() for a in alive)

@@ -94,6 +94,19 @@ Tensor tile_block(const Tensor &w) {
   return out;
 }
 
+// Block scales as fp32, contiguous, in memory of their own: `to` and `contiguous` hand an fp32 tensor through as it is, and
+// an entry that holds its source's storage never sees it die
+Tensor own_scales(const Tensor &s) {
+  return at::empty(s.sizes(), s.options().dtype(at::kFloat)).copy_(s);
+}
+
+// Packed copies are plain data: made outside autograd (a recorded cat or cast would hold the source parameter) and as normal
+// tensors also inside inference mode
+struct PackGuard {
+  c10::InferenceMode inference{false};
+  at::NoGradGuard no_grad;
+};
+
 // Reference argument layout (gate [E,I,H], up [E,I,H], down pre-transposed [E,I,H], bf16 scales of the same
 // orientation: python/regression/test_llm/test_moe.py:285-288) -> W13 = gate rows then up rows [E,2I,H], W2 = down in
 // checkpoint orientation [E,H,I], scales widened to fp32, weight bytes tile-blocked.  Values are untouched.
@@ -116,10 +129,11 @@ const PackedEntry &packed_weights(const Tensor &gate, const Tensor &up, const Te
   PackedEntry e;
   e.ids = ids;
   for (const Tensor *t : src) e.alive.push_back(t->storage().getWeakStorageImpl());
+  PackGuard guard;
   e.w13 = tile_block(at::cat({gate, up}, 1).contiguous());
-  e.w13s = at::cat({gs, us}, 1).to(at::kFloat).contiguous();
+  e.w13s = own_scales(at::cat({gs, us}, 1));
   e.w2 = tile_block(down.transpose(1, 2).contiguous());
-  e.w2s = ds.transpose(1, 2).to(at::kFloat).contiguous();
+  e.w2s = own_scales(ds.transpose(1, 2));
   g_packed.push_back(std::move(e));
   return g_packed.back();
 }
@@ -153,6 +167,7 @@ DenseEntry &dense_packed(std::initializer_list<const Tensor *> src, Make make) {
   DenseEntry e;
   for (const Tensor *t : src) e.alive.push_back(t->storage().getWeakStorageImpl());
   e.ids = std::move(ids);
+  PackGuard guard;
   e.made = make();
   g_dense.push_back(std::move(e));
   return g_dense.back();
@@ -359,7 +374,7 @@ Tensor mm_w8a16_dq_forward(const Tensor &input, const Tensor &weight, const Tens
   }
   void *st = stream_of(input);
   DenseEntry &entry = dense_packed({&weight, &scale}, [&]() -> std::vector<Tensor> {
-    return {tile_block(weight.contiguous()), scale.to(at::kFloat).contiguous()};
+    return {tile_block(weight.contiguous()), own_scales(scale)};
   });
   const auto &w = entry.made;
   const size_t need = dense_workspace(entry, M, [&] { return moe_mm_fp8_workspace_bytes((int)M, (int)K, (int)N); });
@@ -386,8 +401,8 @@ Tensor mlp_w8a16_dq_forward(const Tensor &input, const Tensor &gate, const Tenso
   }
   void *st = stream_of(input);
   DenseEntry &entry = dense_packed({&gate, &up, &down, &gs, &us, &ds}, [&]() -> std::vector<Tensor> {
-    return {tile_block(at::cat({gate, up}, 0).contiguous()), at::cat({gs, us}, 0).to(at::kFloat).contiguous(),
-            tile_block(down.t().contiguous()), ds.t().to(at::kFloat).contiguous()};
+    return {tile_block(at::cat({gate, up}, 0).contiguous()), own_scales(at::cat({gs, us}, 0)),
+            tile_block(down.t().contiguous()), own_scales(ds.t())};
   });
   const auto &w = entry.made;
   const size_t need = dense_workspace(entry, M, [&] { return moe_mlp_fp8_workspace_bytes((int)M, (int)H, (int)I); });
