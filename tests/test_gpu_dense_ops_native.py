@@ -109,3 +109,41 @@ def test_packed_copy_does_not_keep_its_sources_alive(pkg, dev, op, form):
     del tensors, w, s
     gc.collect()
     assert all(a.expired() for a in alive)
+
+
+@pytest.mark.parametrize("op", ["mm", "mlp", "experts"])
+def test_updates_of_a_live_weight_leave_one_packed_copy(pkg, dev, op):
+    E, I, H = 4, 512, 1024
+    lead = (E,) if op == "experts" else ()
+    my_ops = torch.ops.my_ops
+    x = torch.randn(5, H, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(dev)
+    ids = torch.randint(0, E, (5, 1), generator=torch.Generator().manual_seed(2), dtype=torch.int32).to(dev)
+    tensors = []
+    for i in range(1 if op == "mm" else 3):
+        w, s = weights(dev, I * max(1, *lead, 1), H, i)
+        tensors += [w.view(*lead, I, H), s.view(*lead, I // 128, H // 128)]
+    fresh = [[weights(dev, t.numel() // H, H, 10 * k + i)[0].view(t.shape) for i, t in enumerate(tensors[::2])] for k in range(6)]
+
+    def run(ts):
+        out = torch.empty(5, I if op == "mm" else H, dtype=torch.bfloat16, device=dev)
+        if op == "mm":
+            return my_ops.mm_w8a16_dq_forward(x, *ts, out, 128)
+        if op == "mlp":
+            return my_ops.mlp_w8a16_dq_forward(x, *ts[::2], *ts[1::2], out, 128)
+        return my_ops.fused_moe_fused_experts(out, x, None, None, *ts[::2], *ts[1::2], ids, ids.float() + 1, None, None, None,
+                                              128, E, 1, False, 1, 1, None, None, None, False)
+
+    run(tensors)
+    gc.collect()
+    before = torch.cuda.memory_allocated()
+    for new in fresh:                                     # a weight sync: the same tensors, written again
+        for t, n in zip(tensors[::2], new):
+            t.copy_(n)
+        tensors[1].mul_(0.5)
+        got = run(tensors)
+        clones = [t.clone() for t in tensors]
+        assert torch.equal(got, run(clones))
+        del got, clones
+        run(tensors)                                      # (a call drops the entries of freed tensors)
+    gc.collect()
+    assert torch.cuda.memory_allocated() <= before + 4096

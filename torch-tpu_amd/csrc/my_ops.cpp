@@ -20,6 +20,7 @@
 
 #include <array>
 #include <cstdio>
+#include <list>
 #include <map>
 #include <mutex>
 #include <optional>
@@ -38,66 +39,82 @@ void check_rc(int rc, const char *what) { TORCH_CHECK(rc == 0, what, ": ", moe_h
 
 void *stream_of(const Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
-// ---- identity of a weight set ---------------------------------------------------------------------------------
+// ---- packed copies of weights -----------------------------------------------------------------------------------
 // A packed copy belongs to the STORAGES of the tensors it was made from (not to the Python or C++ wrapper objects,
-// which callers re-create freely: `param.data`, views made per call): storage, offset, shape, strides, dtype and the
-// version counter.  The entry keeps weak references to the storages; once one of them has been freed the entry is
-// dead and is dropped the next time the table is walked, so new weights that land on a recycled address never meet
-// an old copy.  An in-place write that does not move the version counter cannot be seen from here
-// (my_ops::_invalidate_weight_cache after such an update).
+// which callers re-create freely: `param.data`, views made per call): storage, offset, shape, strides and dtype.  The entry
+// keeps weak references to the storages; once one of them has been freed the entry is dead and is dropped the next time the
+// table is walked, so new weights that land on a recycled address never meet an old copy.  When the version counter of a
+// source has moved the copy is made again, in the same memory: an update costs no memory, and a HIP graph that reads the
+// copy goes on with the new weights (an update through the sources has to be ordered against their readers on other streams
+// by whoever makes it, and the copy's readers are theirs).  An in-place write that does not move the version counter cannot
+// be seen from here (my_ops::_invalidate_weight_cache after such an update).
 // (two or three dimensions: the callers of identify() have checked that)
 struct SourceId {
   const c10::StorageImpl *storage;
   const void *data;
   int64_t offset;
-  uint32_t version;
   c10::ScalarType dtype;
   int64_t sizes[3], strides[3];
   bool operator==(const SourceId &o) const {
-    bool same = storage == o.storage && data == o.data && offset == o.offset && version == o.version && dtype == o.dtype;
+    bool same = storage == o.storage && data == o.data && offset == o.offset && dtype == o.dtype;
     for (int i = 0; i < 3; i++) same = same && sizes[i] == o.sizes[i] && strides[i] == o.strides[i];
     return same;
   }
 };
 
 SourceId identify(const Tensor &t) {
-  SourceId s;
+  SourceId s{};
   s.storage = t.unsafeGetTensorImpl()->unsafe_storage().unsafeGetStorageImpl();
   s.data = t.data_ptr();
   s.offset = t.storage_offset();
-  s.version = t.is_inference() ? 0u : (uint32_t)t._version();
   s.dtype = t.scalar_type();
-  for (int i = 0; i < 3; i++) {
-    s.sizes[i] = i < t.dim() ? t.size(i) : 0;
-    s.strides[i] = i < t.dim() ? t.stride(i) : 0;
+  for (int i = 0; i < 3 && i < t.dim(); i++) {
+    s.sizes[i] = t.size(i);
+    s.strides[i] = t.stride(i);
   }
   return s;
 }
 
+uint32_t version_of(const Tensor &t) { return t.is_inference() ? 0u : (uint32_t)t._version(); }
+
+enum PackedForm { kFormExperts, kFormMm, kFormMlp };
+constexpr int kMaxSources = 6, kMaxMade = 4;
+
 struct PackedEntry {
-  std::array<SourceId, 6> ids;
+  PackedForm form;
+  std::array<SourceId, kMaxSources> ids{};
+  std::array<uint32_t, kMaxSources> versions{};
   std::vector<c10::weak_intrusive_ptr<c10::StorageImpl>> alive;
-  Tensor w13, w13s, w2, w2s;
+  std::array<Tensor, kMaxMade> made;      // tile-blocked weights and fp32 scales, one pair (a product) or two
+  int64_t packings = 0;
+  int64_t rows = 0;                       // dense: the largest batch seen and the workspace that covers it and all smaller ones
+  size_t workspace_bytes = 0;
+  bool dead() const {
+    for (auto &w : alive)
+      if (w.expired()) return true;
+    return false;
+  }
 };
 
 std::mutex g_mutex;
-std::vector<PackedEntry> g_packed;
+std::list<PackedEntry> g_packed;
 std::map<std::pair<int, void *>, Tensor> g_workspace, g_rw;
 int g_numerics = 0;     // 0 = w8a8 (this file), 1 = w8a16 (general path)
 
-// row-major weight bytes -> tile-blocked (moe_pack_weights), out of place
-Tensor tile_block(const Tensor &w) {
-  Tensor out = at::empty_like(w);
-  const int64_t rows = w.numel() / w.size(-1);
-  check_rc(moe_pack_weights(stream_of(w), w.data_ptr(), rows, (int)(w.size(-1) * w.element_size()), out.data_ptr()),
+// row-major weight bytes -> tile-blocked (moe_pack_weights), into the copy that is there or a new one
+void put_weights(Tensor &dst, const Tensor &rowmajor) {
+  const Tensor w = rowmajor.contiguous();
+  if (!dst.defined()) dst = at::empty_like(w);
+  check_rc(moe_pack_weights(stream_of(w), w.data_ptr(), w.numel() / w.size(-1), (int)(w.size(-1) * w.element_size()),
+                            dst.data_ptr()),
            "moe_pack_weights");
-  return out;
 }
 
 // Block scales as fp32, contiguous, in memory of their own: `to` and `contiguous` hand an fp32 tensor through as it is, and
 // an entry that holds its source's storage never sees it die
-Tensor own_scales(const Tensor &s) {
-  return at::empty(s.sizes(), s.options().dtype(at::kFloat)).copy_(s);
+void put_scales(Tensor &dst, const Tensor &s) {
+  if (!dst.defined()) dst = at::empty(s.sizes(), s.options().dtype(at::kFloat));
+  dst.copy_(s);
 }
 
 // Packed copies are plain data: made outside autograd (a recorded cat or cast would hold the source parameter) and as normal
@@ -107,76 +124,72 @@ struct PackGuard {
   at::NoGradGuard no_grad;
 };
 
-// Reference argument layout (gate [E,I,H], up [E,I,H], down pre-transposed [E,I,H], bf16 scales of the same
-// orientation: python/regression/test_llm/test_moe.py:285-288) -> W13 = gate rows then up rows [E,2I,H], W2 = down in
-// checkpoint orientation [E,H,I], scales widened to fp32, weight bytes tile-blocked.  Values are untouched.
-const PackedEntry &packed_weights(const Tensor &gate, const Tensor &up, const Tensor &down, const Tensor &gs,
-                                  const Tensor &us, const Tensor &ds) {
-  const Tensor *src[6] = {&gate, &up, &down, &gs, &us, &ds};
-  std::array<SourceId, 6> ids;
-  for (int i = 0; i < 6; i++) ids[i] = identify(*src[i]);
-  for (size_t i = 0; i < g_packed.size();) {
-    bool dead = false;
-    for (auto &w : g_packed[i].alive) dead = dead || w.expired();
-    if (dead) {
-      g_packed[i] = std::move(g_packed.back());
-      g_packed.pop_back();
+// call with g_mutex held; make(made) fills or refills the copies
+template <typename Make>
+PackedEntry &packed(PackedForm form, std::initializer_list<const Tensor *> src, Make make) {
+  std::array<SourceId, kMaxSources> ids{};
+  std::array<uint32_t, kMaxSources> versions{};
+  int n = 0;
+  for (const Tensor *t : src) {
+    ids[n] = identify(*t);
+    versions[n++] = version_of(*t);
+  }
+  auto found = g_packed.end();
+  for (auto e = g_packed.begin(); e != g_packed.end();) {
+    if (e->dead()) {
+      e = g_packed.erase(e);
       continue;
     }
-    if (g_packed[i].ids == ids) return g_packed[i];
-    i++;
+    if (e->form == form && e->ids == ids) found = e;
+    ++e;
   }
-  PackedEntry e;
-  e.ids = ids;
-  for (const Tensor *t : src) e.alive.push_back(t->storage().getWeakStorageImpl());
-  PackGuard guard;
-  e.w13 = tile_block(at::cat({gate, up}, 1).contiguous());
-  e.w13s = own_scales(at::cat({gs, us}, 1));
-  e.w2 = tile_block(down.transpose(1, 2).contiguous());
-  e.w2s = own_scales(ds.transpose(1, 2));
-  g_packed.push_back(std::move(e));
-  return g_packed.back();
+  if (found != g_packed.end()) {
+    if (found->versions == versions) return *found;
+  } else {
+    PackedEntry e;
+    e.form = form;
+    e.ids = ids;
+    for (const Tensor *t : src) e.alive.push_back(t->storage().getWeakStorageImpl());
+    g_packed.push_back(std::move(e));
+    found = std::prev(g_packed.end());
+  }
+  try {
+    PackGuard guard;
+    make(found->made);
+  } catch (...) {
+    g_packed.erase(found);
+    throw;
+  }
+  found->versions = versions;
+  found->packings++;
+  return *found;
 }
 
-// The packed copies of the dense ops' weights, under the same rules: `made` is tile-blocked weights and fp32 scales, one
-// pair (a product) or two (the MLP).
-struct DenseEntry {
-  std::vector<SourceId> ids;
-  std::vector<c10::weak_intrusive_ptr<c10::StorageImpl>> alive;
-  std::vector<Tensor> made;
-  int64_t rows = 0;             // the largest batch seen and the workspace that covers it and every smaller one
-  size_t workspace_bytes = 0;
-};
-std::vector<DenseEntry> g_dense;
+// Reference argument layout (gate [E,I,H], up [E,I,H], down pre-transposed [E,I,H], bf16 scales of the same
+// orientation: python/regression/test_llm/test_moe.py:285-288) -> W13 = gate rows then up rows [E,2I,H], its scales, W2 =
+// down in checkpoint orientation [E,H,I], its scales; scales widened to fp32, weight bytes tile-blocked.  Values are
+// untouched.  The gated MLP's weights are the same without the expert dimension.
+PackedEntry &packed_gated(PackedForm form, const Tensor &gate, const Tensor &up, const Tensor &down, const Tensor &gs,
+                          const Tensor &us, const Tensor &ds) {
+  return packed(form, {&gate, &up, &down, &gs, &us, &ds}, [&](std::array<Tensor, kMaxMade> &made) {
+    put_weights(made[0], at::cat({gate, up}, -2));
+    put_scales(made[1], at::cat({gs, us}, -2));
+    put_weights(made[2], down.transpose(-2, -1));
+    put_scales(made[3], ds.transpose(-2, -1));
+  });
+}
 
-template <typename Make>
-DenseEntry &dense_packed(std::initializer_list<const Tensor *> src, Make make) {
-  std::vector<SourceId> ids;
-  for (const Tensor *t : src) ids.push_back(identify(*t));
-  for (size_t i = 0; i < g_dense.size();) {
-    bool dead = false;
-    for (auto &w : g_dense[i].alive) dead = dead || w.expired();
-    if (dead) {
-      g_dense[i] = std::move(g_dense.back());
-      g_dense.pop_back();
-      continue;
-    }
-    if (g_dense[i].ids == ids) return g_dense[i];
-    i++;
-  }
-  DenseEntry e;
-  for (const Tensor *t : src) e.alive.push_back(t->storage().getWeakStorageImpl());
-  e.ids = std::move(ids);
-  PackGuard guard;
-  e.made = make();
-  g_dense.push_back(std::move(e));
-  return g_dense.back();
+PackedEntry &packed_mm(const Tensor &weight, const Tensor &scale) {
+  return packed(kFormMm, {&weight, &scale}, [&](std::array<Tensor, kMaxMade> &made) {
+    put_weights(made[0], weight);
+    put_scales(made[1], scale);
+  });
 }
 
 // Workspace of a call on M rows: asked for again only when a batch is larger than every one before it (the query looks at
 // all smaller batches), so that a layer's later, smaller calls never grow the scratch
 template <typename Query>
-size_t dense_workspace(DenseEntry &e, int64_t M, Query query) {
+size_t dense_workspace(PackedEntry &e, int64_t M, Query query) {
   if (M > e.rows) {
     e.workspace_bytes = query();
     e.rows = M;
@@ -309,7 +322,7 @@ Tensor fused_moe_fused_experts(const Tensor &output, const Tensor &input, const 
   std::lock_guard<std::mutex> lock(g_mutex);
   void *st = stream_of(input);
   ProfileScope prof("fused_moe_fused_experts", st);
-  const PackedEntry &w = packed_weights(gate_weights, up_weights, down_weights, *gate_scales, *up_scales, *down_scales);
+  const auto &w = packed_gated(kFormExperts, gate_weights, up_weights, down_weights, *gate_scales, *up_scales, *down_scales).made;
   const void *rw = nullptr;
   int rw_dtype = MOE_DTYPE_F32;
   if (out_mode) {
@@ -331,8 +344,8 @@ Tensor fused_moe_fused_experts(const Tensor &output, const Tensor &input, const 
   }
   const size_t need = moe_fused_experts_workspace_bytes((int)T, (int)H, (int)I, (int)E, (int)K, 0);
   Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
-  check_rc(moe_fused_experts_fp8_rw(st, input.data_ptr(), (int)T, (int)H, (const uint8_t *)w.w13.data_ptr(),
-                                    w.w13s.data_ptr<float>(), (const uint8_t *)w.w2.data_ptr(), w.w2s.data_ptr<float>(),
+  check_rc(moe_fused_experts_fp8_rw(st, input.data_ptr(), (int)T, (int)H, (const uint8_t *)w[0].data_ptr(),
+                                    w[1].data_ptr<float>(), (const uint8_t *)w[2].data_ptr(), w[3].data_ptr<float>(),
                                     (int)I, (int)E, select_experts.data_ptr<int32_t>(), rw, rw_dtype, (int)K, nullptr,
                                     nullptr, nullptr, nullptr, 0, output.data_ptr(), out_mode, ws.data_ptr(),
                                     (size_t)ws.numel()),
@@ -373,9 +386,7 @@ Tensor mm_w8a16_dq_forward(const Tensor &input, const Tensor &weight, const Tens
     return call_general("my_ops::_mm_general", {input, weight, scale, output, blocksize});
   }
   void *st = stream_of(input);
-  DenseEntry &entry = dense_packed({&weight, &scale}, [&]() -> std::vector<Tensor> {
-    return {tile_block(weight.contiguous()), own_scales(scale)};
-  });
+  PackedEntry &entry = packed_mm(weight, scale);
   const auto &w = entry.made;
   const size_t need = dense_workspace(entry, M, [&] { return moe_mm_fp8_workspace_bytes((int)M, (int)K, (int)N); });
   Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
@@ -400,10 +411,7 @@ Tensor mlp_w8a16_dq_forward(const Tensor &input, const Tensor &gate, const Tenso
     return call_general("my_ops::_mlp_general", {input, gate, up, down, gs, us, ds, output, blocksize});
   }
   void *st = stream_of(input);
-  DenseEntry &entry = dense_packed({&gate, &up, &down, &gs, &us, &ds}, [&]() -> std::vector<Tensor> {
-    return {tile_block(at::cat({gate, up}, 0).contiguous()), own_scales(at::cat({gs, us}, 0)),
-            tile_block(down.t().contiguous()), own_scales(ds.t())};
-  });
+  PackedEntry &entry = packed_gated(kFormMlp, gate, up, down, gs, us, ds);
   const auto &w = entry.made;
   const size_t need = dense_workspace(entry, M, [&] { return moe_mlp_fp8_workspace_bytes((int)M, (int)H, (int)I); });
   Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
@@ -505,12 +513,26 @@ void _set_expert_numerics(int64_t mode) {
 void _invalidate_weight_cache() {
   std::lock_guard<std::mutex> lock(g_mutex);
   g_packed.clear();
-  g_dense.clear();
 }
 
+// weight sets packed for tensors that are alive, every update of one counted again
 int64_t _packed_weight_sets() {
   std::lock_guard<std::mutex> lock(g_mutex);
-  return (int64_t)g_packed.size();
+  int64_t n = 0;
+  g_packed.remove_if([](const PackedEntry &e) { return e.dead(); });
+  for (auto &e : g_packed) n += e.packings;
+  return n;
+}
+
+// memory that the packed copies hold
+int64_t _packed_weight_bytes() {
+  std::lock_guard<std::mutex> lock(g_mutex);
+  int64_t n = 0;
+  g_packed.remove_if([](const PackedEntry &e) { return e.dead(); });
+  for (auto &e : g_packed)
+    for (auto &t : e.made)
+      if (t.defined()) n += (int64_t)t.nbytes();
+  return n;
 }
 
 TORCH_LIBRARY(my_ops, m) {
@@ -527,6 +549,7 @@ TORCH_LIBRARY(my_ops, m) {
   m.def("_set_expert_numerics", _set_expert_numerics);
   m.def("_invalidate_weight_cache", _invalidate_weight_cache);
   m.def("_packed_weight_sets", _packed_weight_sets);
+  m.def("_packed_weight_bytes", _packed_weight_bytes);
 }
 
 TORCH_LIBRARY_IMPL(my_ops, CompositeExplicitAutograd, m) {
