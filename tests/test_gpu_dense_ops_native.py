@@ -147,3 +147,92 @@ def test_updates_of_a_live_weight_leave_one_packed_copy(pkg, dev, op):
         run(tensors)                                      # (a call drops the entries of freed tensors)
     gc.collect()
     assert torch.cuda.memory_allocated() <= before + 4096
+
+
+def one_mm(dev, seed, M=8, K=1024, N=512):
+    w, s = weights(dev, N, K, seed)
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16).to(dev)
+    return x, w, s, torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+
+
+def test_a_call_on_another_stream_waits_for_the_packing(pkg, dev):
+    my_ops = torch.ops.my_ops
+    x, w, s, out = one_mm(dev, 1, K=4096, N=4096)
+    want = my_ops.mm_w8a16_dq_forward(x, w.clone(), s.clone(), torch.empty_like(out), 128)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        torch.cuda._sleep(20_000_000)                     # the packing lies behind some milliseconds of other work
+        first = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), 128)
+    with torch.cuda.stream(b):
+        second = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), 128)
+    w.record_stream(a)
+    torch.cuda.synchronize()
+    assert torch.equal(first, want) and torch.equal(second, want)
+    # an update made and packed on one stream is seen by a call on the other
+    with torch.cuda.stream(b):
+        torch.cuda._sleep(20_000_000)
+        s.mul_(2)
+        my_ops.mm_w8a16_dq_forward(x, w, s, out, 128)
+        done = torch.cuda.Event()
+        done.record()
+    with torch.cuda.stream(a):
+        a.wait_event(done)
+        second = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), 128)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want * 2) and torch.equal(second, want * 2)
+
+
+def test_captured_calls_with_packed_known_and_new_weights(pkg, dev):
+    """A weight packed before the capture is used as it is, one that is new to the capture is packed inside the graph and
+    left alone by eager calls, and an eager refill after an update reaches the graph's copy."""
+    my_ops = torch.ops.my_ops
+    known, new = one_mm(dev, 3), one_mm(dev, 4)
+    run = lambda t, out=None: my_ops.mm_w8a16_dq_forward(*t[:3], t[3] if out is None else out, 128)
+    want = [run((t[0], t[1].clone(), t[2].clone(), torch.empty_like(t[3]))) for t in (known, new)]
+    run(known)
+    torch.cuda.synchronize()
+    held = my_ops._packed_weight_bytes()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(known)
+        run(new)
+    assert my_ops._packed_weight_bytes() <= held          # (less, if the clones' entries went)
+    eager = run(new, torch.empty_like(new[3]))            # before the graph has run at all
+    torch.cuda.synchronize()
+    assert torch.equal(eager, want[1])
+    for _ in range(3):
+        known[3].zero_()
+        new[3].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(known[3], want[0]) and torch.equal(new[3], want[1])
+        assert torch.equal(run(known, torch.empty_like(known[3])), want[0])
+    for t in (known, new):
+        t[2].mul_(2)
+        run(t, torch.empty_like(t[3]))
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(known[3], want[0] * 2) and torch.equal(new[3], want[1] * 2)
+
+
+def test_capture_begun_while_the_packing_still_runs(pkg, dev):
+    my_ops = torch.ops.my_ops
+    x, w, s, out = one_mm(dev, 5)
+    want = my_ops.mm_w8a16_dq_forward(x, w.clone(), s.clone(), torch.empty_like(out), 128)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)
+    my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), 128)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        graph.capture_begin()
+        my_ops.mm_w8a16_dq_forward(x, w, s, out, 128)
+        graph.capture_end()
+    out.zero_()
+    torch.cuda.synchronize()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        out.zero_()

@@ -14,10 +14,14 @@
 // at 32 rows) than its two launches take on the GPU (11 us).
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <array>
 #include <cstdio>
 #include <list>
@@ -37,7 +41,8 @@ using OptTensor = std::optional<Tensor>;
 
 void check_rc(int rc, const char *what) { TORCH_CHECK(rc == 0, what, ": ", moe_hip_strerror(rc), " (code ", rc, ")"); }
 
-void *stream_of(const Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+c10::hip::HIPStream hip_stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()); }
+void *stream_of(const Tensor &t) { return (void *)hip_stream_of(t).stream(); }
 
 // ---- packed copies of weights -----------------------------------------------------------------------------------
 // A packed copy belongs to the STORAGES of the tensors it was made from (not to the Python or C++ wrapper objects,
@@ -80,12 +85,44 @@ uint32_t version_of(const Tensor &t) { return t.is_inference() ? 0u : (uint32_t)
 enum PackedForm { kFormExperts, kFormMm, kFormMlp };
 constexpr int kMaxSources = 6, kMaxMade = 4;
 
+// An event behind the work that makes a copy, until that work has been seen complete
+struct ReadyEvent {
+  hipEvent_t event = nullptr;
+  ReadyEvent() = default;
+  ReadyEvent(ReadyEvent &&o) noexcept : event(o.event) { o.event = nullptr; }
+  ReadyEvent &operator=(ReadyEvent &&) = delete;
+  ~ReadyEvent() { drop(); }
+  void drop() {
+    if (event) (void)hipEventDestroy(event);
+    event = nullptr;
+  }
+  void record(hipStream_t st) {
+    if (!event) C10_HIP_CHECK(hipEventCreateWithFlags(&event, hipEventDisableTiming));
+    C10_HIP_CHECK(hipEventRecord(event, st));
+  }
+  // whether the work is known to be complete (asked in a way that a capture, this thread's or another's, allows)
+  bool complete() {
+    if (!event) return true;
+    c10::hip::HIPStreamCaptureModeGuard relaxed(hipStreamCaptureModeRelaxed);
+    const hipError_t rc = hipEventQuery(event);
+    if (rc == hipSuccess) {
+      drop();
+      return true;
+    }
+    (void)hipGetLastError();
+    if (rc != hipErrorNotReady) C10_HIP_CHECK(rc);
+    return false;
+  }
+};
+
 struct PackedEntry {
   PackedForm form;
   std::array<SourceId, kMaxSources> ids{};
   std::array<uint32_t, kMaxSources> versions{};
   std::vector<c10::weak_intrusive_ptr<c10::StorageImpl>> alive;
   std::array<Tensor, kMaxMade> made;      // tile-blocked weights and fp32 scales, one pair (a product) or two
+  ReadyEvent ready;                       // behind the launches that filled `made`
+  std::vector<c10::hip::HIPStream> known_to_allocator;    // streams whose work the copies' memory waits for when it is freed
   int64_t packings = 0;
   int64_t rows = 0;                       // dense: the largest batch seen and the workspace that covers it and all smaller ones
   size_t workspace_bytes = 0;
@@ -97,7 +134,7 @@ struct PackedEntry {
 };
 
 std::mutex g_mutex;
-std::list<PackedEntry> g_packed;
+std::list<PackedEntry> &g_packed = *new std::list<PackedEntry>;      // (no events destroyed after the runtime at exit)
 std::map<std::pair<int, void *>, Tensor> g_workspace, g_rw;
 int g_numerics = 0;     // 0 = w8a8 (this file), 1 = w8a16 (general path)
 
@@ -124,9 +161,18 @@ struct PackGuard {
   at::NoGradGuard no_grad;
 };
 
-// call with g_mutex held; make(made) fills or refills the copies
+// What a call multiplies with: an entry's copies, or some of its own
+struct Packed {
+  std::array<Tensor, kMaxMade> made;
+  PackedEntry *entry;           // null: a copy that lives in a captured graph
+};
+
+// Call with g_mutex held; make(made) fills or refills the copies.  The copies are made on the caller's stream; a call on
+// another stream waits for that on its own stream, without holding up the host, and the allocator is told of it once.  Work
+// under capture runs with every replay and not now, so nothing that it makes is left for other calls to find: a weight set
+// that has no finished copy then (warm up first) is packed inside the graph.
 template <typename Make>
-PackedEntry &packed(PackedForm form, std::initializer_list<const Tensor *> src, Make make) {
+Packed packed(PackedForm form, std::initializer_list<const Tensor *> src, Make make) {
   std::array<SourceId, kMaxSources> ids{};
   std::array<uint32_t, kMaxSources> versions{};
   int n = 0;
@@ -134,6 +180,12 @@ PackedEntry &packed(PackedForm form, std::initializer_list<const Tensor *> src, 
     ids[n] = identify(*t);
     versions[n++] = version_of(*t);
   }
+  const c10::hip::HIPStream stream = hip_stream_of(**src.begin());
+  const auto capturing = [&] {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    C10_HIP_CHECK(hipStreamIsCapturing(stream.stream(), &status));
+    return status != hipStreamCaptureStatusNone;
+  };
   auto found = g_packed.end();
   for (auto e = g_packed.begin(); e != g_packed.end();) {
     if (e->dead()) {
@@ -143,34 +195,52 @@ PackedEntry &packed(PackedForm form, std::initializer_list<const Tensor *> src, 
     if (e->form == form && e->ids == ids) found = e;
     ++e;
   }
-  if (found != g_packed.end()) {
-    if (found->versions == versions) return *found;
-  } else {
+  const bool current = found != g_packed.end() && found->versions == versions;
+  if (!(current && found->ready.complete()) && capturing()) {
+    PackGuard guard;
+    Packed own{{}, nullptr};
+    make(own.made);
+    return own;
+  }
+  if (found == g_packed.end()) {
     PackedEntry e;
     e.form = form;
     e.ids = ids;
     for (const Tensor *t : src) e.alive.push_back(t->storage().getWeakStorageImpl());
+    e.known_to_allocator.push_back(stream);
     g_packed.push_back(std::move(e));
     found = std::prev(g_packed.end());
+  } else if (found->ready.event) {
+    C10_HIP_CHECK(hipStreamWaitEvent(stream.stream(), found->ready.event, 0));
   }
-  try {
-    PackGuard guard;
-    make(found->made);
-  } catch (...) {
-    g_packed.erase(found);
-    throw;
+  if (!current) {
+    try {
+      PackGuard guard;
+      c10::DeviceGuard device((*src.begin())->device());
+      make(found->made);
+      found->ready.record(stream.stream());
+    } catch (...) {
+      g_packed.erase(found);
+      throw;
+    }
+    found->versions = versions;
+    found->packings++;
   }
-  found->versions = versions;
-  found->packings++;
-  return *found;
+  auto &known = found->known_to_allocator;
+  if (std::find(known.begin(), known.end(), stream) == known.end()) {
+    for (const Tensor &t : found->made)
+      if (t.defined()) c10::hip::HIPCachingAllocator::recordStream(t.storage().data_ptr(), stream);
+    known.push_back(stream);
+  }
+  return {found->made, &*found};
 }
 
 // Reference argument layout (gate [E,I,H], up [E,I,H], down pre-transposed [E,I,H], bf16 scales of the same
 // orientation: python/regression/test_llm/test_moe.py:285-288) -> W13 = gate rows then up rows [E,2I,H], its scales, W2 =
 // down in checkpoint orientation [E,H,I], its scales; scales widened to fp32, weight bytes tile-blocked.  Values are
 // untouched.  The gated MLP's weights are the same without the expert dimension.
-PackedEntry &packed_gated(PackedForm form, const Tensor &gate, const Tensor &up, const Tensor &down, const Tensor &gs,
-                          const Tensor &us, const Tensor &ds) {
+Packed packed_gated(PackedForm form, const Tensor &gate, const Tensor &up, const Tensor &down, const Tensor &gs,
+                    const Tensor &us, const Tensor &ds) {
   return packed(form, {&gate, &up, &down, &gs, &us, &ds}, [&](std::array<Tensor, kMaxMade> &made) {
     put_weights(made[0], at::cat({gate, up}, -2));
     put_scales(made[1], at::cat({gs, us}, -2));
@@ -179,7 +249,7 @@ PackedEntry &packed_gated(PackedForm form, const Tensor &gate, const Tensor &up,
   });
 }
 
-PackedEntry &packed_mm(const Tensor &weight, const Tensor &scale) {
+Packed packed_mm(const Tensor &weight, const Tensor &scale) {
   return packed(kFormMm, {&weight, &scale}, [&](std::array<Tensor, kMaxMade> &made) {
     put_weights(made[0], weight);
     put_scales(made[1], scale);
@@ -189,12 +259,13 @@ PackedEntry &packed_mm(const Tensor &weight, const Tensor &scale) {
 // Workspace of a call on M rows: asked for again only when a batch is larger than every one before it (the query looks at
 // all smaller batches), so that a layer's later, smaller calls never grow the scratch
 template <typename Query>
-size_t dense_workspace(PackedEntry &e, int64_t M, Query query) {
-  if (M > e.rows) {
-    e.workspace_bytes = query();
-    e.rows = M;
+size_t dense_workspace(PackedEntry *e, int64_t M, Query query) {
+  if (!e) return query();
+  if (M > e->rows) {
+    e->workspace_bytes = query();
+    e->rows = M;
   }
-  return e.workspace_bytes;
+  return e->workspace_bytes;
 }
 
 // what the common forms of the dense ops ask of their tensors; any other form takes the general road
@@ -322,7 +393,7 @@ Tensor fused_moe_fused_experts(const Tensor &output, const Tensor &input, const 
   std::lock_guard<std::mutex> lock(g_mutex);
   void *st = stream_of(input);
   ProfileScope prof("fused_moe_fused_experts", st);
-  const auto &w = packed_gated(kFormExperts, gate_weights, up_weights, down_weights, *gate_scales, *up_scales, *down_scales).made;
+  const auto w = packed_gated(kFormExperts, gate_weights, up_weights, down_weights, *gate_scales, *up_scales, *down_scales).made;
   const void *rw = nullptr;
   int rw_dtype = MOE_DTYPE_F32;
   if (out_mode) {
@@ -386,9 +457,9 @@ Tensor mm_w8a16_dq_forward(const Tensor &input, const Tensor &weight, const Tens
     return call_general("my_ops::_mm_general", {input, weight, scale, output, blocksize});
   }
   void *st = stream_of(input);
-  PackedEntry &entry = packed_mm(weight, scale);
-  const auto &w = entry.made;
-  const size_t need = dense_workspace(entry, M, [&] { return moe_mm_fp8_workspace_bytes((int)M, (int)K, (int)N); });
+  const Packed p = packed_mm(weight, scale);
+  const auto &w = p.made;
+  const size_t need = dense_workspace(p.entry, M, [&] { return moe_mm_fp8_workspace_bytes((int)M, (int)K, (int)N); });
   Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
   check_rc(moe_mm_fp8(st, input.data_ptr(), (int)M, (int)K, (const uint8_t *)w[0].data_ptr(), w[1].data_ptr<float>(), (int)N,
                       output.data_ptr(), ws.data_ptr(), (size_t)ws.numel()),
@@ -411,9 +482,9 @@ Tensor mlp_w8a16_dq_forward(const Tensor &input, const Tensor &gate, const Tenso
     return call_general("my_ops::_mlp_general", {input, gate, up, down, gs, us, ds, output, blocksize});
   }
   void *st = stream_of(input);
-  PackedEntry &entry = packed_gated(kFormMlp, gate, up, down, gs, us, ds);
-  const auto &w = entry.made;
-  const size_t need = dense_workspace(entry, M, [&] { return moe_mlp_fp8_workspace_bytes((int)M, (int)H, (int)I); });
+  const Packed p = packed_gated(kFormMlp, gate, up, down, gs, us, ds);
+  const auto &w = p.made;
+  const size_t need = dense_workspace(p.entry, M, [&] { return moe_mlp_fp8_workspace_bytes((int)M, (int)H, (int)I); });
   Tensor &ws = scratch(g_workspace, input, st, need, (size_t)1 << 20);
   check_rc(moe_mlp_fp8(st, input.data_ptr(), (int)M, (int)H, (const uint8_t *)w[0].data_ptr(), w[1].data_ptr<float>(),
                        (const uint8_t *)w[2].data_ptr(), w[3].data_ptr<float>(), (int)I, output.data_ptr(), ws.data_ptr(),
