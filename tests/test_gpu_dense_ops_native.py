@@ -236,3 +236,32 @@ def test_capture_begun_while_the_packing_still_runs(pkg, dev):
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         out.zero_()
+
+
+@pytest.mark.parametrize("op", ["mm", "mlp"])
+def test_a_weight_is_packed_once_whatever_form_its_calls_take(pkg, dev, op):
+    my_ops = torch.ops.my_ops
+    I, H, M = 256, 512, 6
+    ts = []
+    for i in range(1 if op == "mm" else 3):
+        ts += weights(dev, I, H, i)
+    x = torch.randn(M, H, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16).to(dev)
+    fn = my_ops.mm_w8a16_dq_forward if op == "mm" else my_ops.mlp_w8a16_dq_forward
+    args = tuple(ts) if op == "mm" else (*ts[::2], *ts[1::2])
+    width = I if op == "mm" else H
+    call = lambda f, x: f(x, *args, torch.empty(M, 2 * width, dtype=torch.bfloat16, device=dev)[:, :width], 128)
+    pkg.invalidate_weight_cache()
+    want = fn(x, *args, torch.empty(M, width, dtype=torch.bfloat16, device=dev), 128).clone()
+    held = my_ops._packed_weight_bytes()
+    assert held == sum(t.nbytes for t in ts[::2]) + 4 * sum(t.numel() for t in ts[1::2])
+    assert torch.equal(call(fn, x), want)                                         # strided output
+    assert torch.equal(call(fn, torch.cat([x, x], 1)[:, :H]), want)               # strided input
+    if op == "mlp":
+        assert torch.equal(call(my_ops.mlp_w8a8_quant_forward, x), want)
+    pkg.set_expert_numerics("w8a16")
+    try:
+        other = call(fn, x)
+    finally:
+        pkg.set_expert_numerics("w8a8")
+    assert (other.float() - want.float()).norm() < 0.1 * want.float().norm()
+    assert my_ops._packed_weight_bytes() == held and len(pkg._my_ops._weights) == 0

@@ -493,6 +493,29 @@ Tensor mlp_w8a16_dq_forward(const Tensor &input, const Tensor &gate, const Tenso
   return output;
 }
 
+// The packed copies for the other roads of the dense ops (strided tensors, the W8A16 arithmetic, mlp_w8a8_quant_forward):
+// a weight is packed once, whatever form its calls take.  Empty: not the form of weights that this file packs.
+std::vector<Tensor> _mm_weights(const Tensor &weight, const Tensor &scale) {
+  if (weight.dim() != 2 || weight.size(0) % 16 || weight.size(1) % 128 ||
+      !plain_weight(weight, scale, weight.size(0), weight.size(1), weight))
+    return {};
+  std::lock_guard<std::mutex> lock(g_mutex);
+  const Packed p = packed_mm(weight, scale);
+  return {p.made[0].detach(), p.made[1].detach()};
+}
+
+std::vector<Tensor> _mlp_weights(const Tensor &gate, const Tensor &up, const Tensor &down, const Tensor &gs, const Tensor &us,
+                                 const Tensor &ds) {
+  if (gate.dim() != 2) return {};
+  const int64_t I = gate.size(0), H = gate.size(1);
+  if (I % 128 || H % 128 || !plain_weight(gate, gs, I, H, gate) || !plain_weight(up, us, I, H, gate) ||
+      !plain_weight(down, ds, I, H, gate) || gs.scalar_type() != us.scalar_type())
+    return {};
+  std::lock_guard<std::mutex> lock(g_mutex);
+  const Packed p = packed_gated(kFormMlp, gate, up, down, gs, us, ds);
+  return {p.made[0].detach(), p.made[1].detach(), p.made[2].detach(), p.made[3].detach()};
+}
+
 // torch_tpu/csrc/ops/my_ops/NoauxTcTopk.cpp:9-67: group-limited top-k into caller-allocated values / indices
 Tensor noaux_tc_topk(const Tensor &values, const Tensor &indices, const Tensor &scores, int64_t n_groups,
                      int64_t topk_groups, int64_t top_k) {
@@ -619,6 +642,9 @@ TORCH_LIBRARY(my_ops, m) {
   m.def("_profile_report", _profile_report);
   m.def("_set_expert_numerics", _set_expert_numerics);
   m.def("_invalidate_weight_cache", _invalidate_weight_cache);
+  m.def("_mm_weights(Tensor weight, Tensor scale) -> Tensor[]");
+  m.def("_mlp_weights(Tensor gate_weight, Tensor up_weight, Tensor down_weight, Tensor gate_scale, Tensor up_scale, "
+        "Tensor down_scale) -> Tensor[]");
   m.def("_packed_weight_sets", _packed_weight_sets);
   m.def("_packed_weight_bytes", _packed_weight_bytes);
 }
@@ -626,6 +652,8 @@ TORCH_LIBRARY(my_ops, m) {
 TORCH_LIBRARY_IMPL(my_ops, CompositeExplicitAutograd, m) {
   m.impl("mm_w8a16_dq_forward", mm_w8a16_dq_forward);
   m.impl("mlp_w8a16_dq_forward", mlp_w8a16_dq_forward);
+  m.impl("_mm_weights", _mm_weights);
+  m.impl("_mlp_weights", _mlp_weights);
 }
 
 }  // namespace at

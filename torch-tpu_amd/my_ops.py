@@ -411,8 +411,10 @@ def _mlp_forward(input, gate_weight, up_weight, down_weight, gate_scale, up_scal
         ws = _workspace(input.device, ops.fused_experts_bf16_workspace_bytes(M, Hp, Ip, 1, 1))
         ops.fused_experts_bf16(x, w13, w2, _zero_ids(input.device, M), None, out=out.view(M, 1, Hp), workspace=ws)
         return done()
-    w13, w13s, w2, w2s = _dense_packed(
-        (gate_weight, up_weight, down_weight, gate_scale, up_scale, down_scale),
+    weights = (gate_weight, up_weight, down_weight, gate_scale, up_scale, down_scale)
+    shared = torch.ops.my_ops._mlp_weights(*weights) if blocksize == 128 and down_t else None      # the C++ op's own copy
+    w13, w13s, w2, w2s = shared or _dense_packed(
+        weights,
         lambda: (ops.pack_weights(torch.cat([_pad_to(gate_weight, Ip, Hp), _pad_to(up_weight, Ip, Hp)], 0).contiguous()),
                  torch.cat([_scales_128(gate_scale, blocksize, I, H), _scales_128(up_scale, blocksize, I, H)], 0).contiguous(),
                  ops.pack_weights(_pad_to(as_t(down_weight), Ip, Hp).t().contiguous()),
@@ -455,8 +457,9 @@ def _mm_w8a16_dq_forward(input, weight, scale, output, blocksize):
                              f"mm-dequant{blocksize}")
         ops.mm_bf16(x, w, out=out)
         return done()
-    w, ws = _dense_packed((weight, scale), lambda: (ops.pack_weights(_pad_to(weight, Np, Kp).contiguous()),
-                                                     _scales_128(scale, blocksize, N, K)), f"mm{blocksize}")
+    shared = torch.ops.my_ops._mm_weights(weight, scale) if blocksize == 128 else None             # the C++ op's own copy
+    w, ws = shared or _dense_packed((weight, scale), lambda: (ops.pack_weights(_pad_to(weight, Np, Kp).contiguous()),
+                                                              _scales_128(scale, blocksize, N, K)), f"mm{blocksize}")
     if _numerics == "w8a16":
         _w8a16_in_range(Kp)
         ops.mm_w8a16(x, w, ws, out=out)
