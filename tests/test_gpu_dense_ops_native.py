@@ -155,17 +155,18 @@ def one_mm(dev, seed, M=8, K=1024, N=512):
     return x, w, s, torch.empty(M, N, dtype=torch.bfloat16, device=dev)
 
 
-def test_a_call_on_another_stream_waits_for_the_packing(pkg, dev):
+@pytest.mark.parametrize("block", [128, 256])            # the C++ table, the Python one
+def test_a_call_on_another_stream_waits_for_the_packing(pkg, dev, block):
     my_ops = torch.ops.my_ops
     x, w, s, out = one_mm(dev, 1, K=4096, N=4096)
-    want = my_ops.mm_w8a16_dq_forward(x, w.clone(), s.clone(), torch.empty_like(out), 128)
+    want = my_ops.mm_w8a16_dq_forward(x, w.clone(), s.clone(), torch.empty_like(out), block)
     a, b = torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
     with torch.cuda.stream(a):
         torch.cuda._sleep(20_000_000)                     # the packing lies behind some milliseconds of other work
-        first = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), 128)
+        first = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), block)
     with torch.cuda.stream(b):
-        second = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), 128)
+        second = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), block)
     w.record_stream(a)
     torch.cuda.synchronize()
     assert torch.equal(first, want) and torch.equal(second, want)
@@ -173,22 +174,23 @@ def test_a_call_on_another_stream_waits_for_the_packing(pkg, dev):
     with torch.cuda.stream(b):
         torch.cuda._sleep(20_000_000)
         s.mul_(2)
-        my_ops.mm_w8a16_dq_forward(x, w, s, out, 128)
+        my_ops.mm_w8a16_dq_forward(x, w, s, out, block)
         done = torch.cuda.Event()
         done.record()
     with torch.cuda.stream(a):
         a.wait_event(done)
-        second = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), 128)
+        second = my_ops.mm_w8a16_dq_forward(x, w, s, torch.empty_like(out), block)
     torch.cuda.synchronize()
     assert torch.equal(out, want * 2) and torch.equal(second, want * 2)
 
 
-def test_captured_calls_with_packed_known_and_new_weights(pkg, dev):
+@pytest.mark.parametrize("block", [128, 256])
+def test_captured_calls_with_packed_known_and_new_weights(pkg, dev, block):
     """A weight packed before the capture is used as it is, one that is new to the capture is packed inside the graph and
     left alone by eager calls, and an eager refill after an update reaches the graph's copy."""
     my_ops = torch.ops.my_ops
     known, new = one_mm(dev, 3), one_mm(dev, 4)
-    run = lambda t, out=None: my_ops.mm_w8a16_dq_forward(*t[:3], t[3] if out is None else out, 128)
+    run = lambda t, out=None: my_ops.mm_w8a16_dq_forward(*t[:3], t[3] if out is None else out, block)
     want = [run((t[0], t[1].clone(), t[2].clone(), torch.empty_like(t[3]))) for t in (known, new)]
     run(known)
     torch.cuda.synchronize()
@@ -208,6 +210,8 @@ def test_captured_calls_with_packed_known_and_new_weights(pkg, dev):
         torch.cuda.synchronize()
         assert torch.equal(known[3], want[0]) and torch.equal(new[3], want[1])
         assert torch.equal(run(known, torch.empty_like(known[3])), want[0])
+    if block != 128:                                      # (the Python table replaces the copy of an updated weight)
+        return
     for t in (known, new):
         t[2].mul_(2)
         run(t, torch.empty_like(t[3]))

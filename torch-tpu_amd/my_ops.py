@@ -105,7 +105,7 @@ class _DerivedCache:
         return (t.untyped_storage()._cdata, t.storage_offset(), tuple(t.shape), tuple(t.stride()), t.dtype, t.device)
 
     def _purge(self):
-        dead = [k for k, (refs, _, _) in self._entries.items() if any(r.expired() for r in refs)]
+        dead = [k for k, (refs, *_) in self._entries.items() if any(r.expired() for r in refs)]
         for k in dead:
             del self._entries[k]
 
@@ -114,13 +114,33 @@ class _DerivedCache:
         versions = tuple(t._version for t in tensors)
         entry = self._entries.get(key)
         if entry is not None:
-            refs, seen, value = entry
+            refs, seen, value, streams = entry
             if seen == versions and not any(r.expired() for r in refs):
+                self._used(value, streams)
                 return value
         self._purge()
         value = make()
-        self._entries[key] = ([StorageWeakRef(t.untyped_storage()) for t in tensors], versions, value)
+        streams = set()
+        if value[0].is_cuda:
+            # Other calls may come on other streams: the copy is finished before they can find it.  What a capture
+            # records has not run, so nothing of it is kept (the graph makes its copy with every replay).
+            if torch.cuda.is_current_stream_capturing():
+                return value
+            stream = torch.cuda.current_stream(value[0].device)
+            stream.synchronize()
+            streams.add(stream)
+        self._entries[key] = ([StorageWeakRef(t.untyped_storage()) for t in tensors], versions, value, streams)
         return value
+
+    @staticmethod
+    def _used(value, streams):
+        """The allocator learns of every stream that reads a copy: its memory waits for their work when it is freed."""
+        if value[0].is_cuda:
+            stream = torch.cuda.current_stream(value[0].device)
+            if stream not in streams:
+                for t in value:
+                    t.record_stream(stream)
+                streams.add(stream)
 
     def clear(self):
         self._entries.clear()
