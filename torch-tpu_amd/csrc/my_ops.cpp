@@ -24,8 +24,8 @@
 #include <algorithm>
 #include <array>
 #include <cstdio>
-#include <list>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <optional>
 #include <sstream>
@@ -47,8 +47,8 @@ void *stream_of(const Tensor &t) { return (void *)hip_stream_of(t).stream(); }
 // ---- packed copies of weights -----------------------------------------------------------------------------------
 // A packed copy belongs to the STORAGES of the tensors it was made from (not to the Python or C++ wrapper objects,
 // which callers re-create freely: `param.data`, views made per call): storage, offset, shape, strides and dtype.  The entry
-// keeps weak references to the storages; once one of them has been freed the entry is dead and is dropped the next time the
-// table is walked, so new weights that land on a recycled address never meet an old copy.  When the version counter of a
+// keeps weak references to the storages; once one of them has been freed the entry is dead and is dropped by one of the next
+// calls, and the storage's address is not given to another storage before that, so new weights never meet an old copy.  When the version counter of a
 // source has moved the copy is made again, in the same memory: an update costs no memory, and a HIP graph that reads the
 // copy goes on with the new weights (an update through the sources has to be ordered against their readers on other streams
 // by whoever makes it, and the copy's readers are theirs).  An in-place write that does not move the version counter cannot
@@ -134,7 +134,50 @@ struct PackedEntry {
 };
 
 std::mutex g_mutex;
-std::list<PackedEntry> &g_packed = *new std::list<PackedEntry>;      // (no events destroyed after the runtime at exit)
+// The entries, and a hash of each one's form and sources beside them: a call compares hashes, one cache line for eight
+// entries, and looks closer at a match.  (Reading every entry and its weak references instead: 8.5 us a call against 8.3 with 610
+// weights, 8.2 against 8.1 with 305.)
+struct PackedTable {
+  std::vector<std::unique_ptr<PackedEntry>> entries;
+  std::vector<size_t> hashes;
+  size_t next_look = 0;
+
+  static size_t hash_of(PackedForm form, const std::array<SourceId, kMaxSources> &ids) {
+    size_t h = form;
+    for (const SourceId &s : ids) h = (h ^ (size_t)s.data ^ ((size_t)s.storage >> 4)) * 0x9e3779b97f4a7c15ull + (size_t)s.sizes[0];
+    return h;
+  }
+  PackedEntry *find(PackedForm form, const std::array<SourceId, kMaxSources> &ids, size_t hash) {
+    for (size_t i = 0; i < hashes.size(); i++)
+      if (hashes[i] == hash && entries[i]->form == form && entries[i]->ids == ids) return entries[i].get();
+    return nullptr;
+  }
+  PackedEntry *add(size_t hash) {
+    entries.push_back(std::make_unique<PackedEntry>());
+    hashes.push_back(hash);
+    return entries.back().get();
+  }
+  void drop(size_t i) {
+    entries[i] = std::move(entries.back());
+    entries.pop_back();
+    hashes[i] = hashes.back();
+    hashes.pop_back();
+  }
+  void drop(const PackedEntry *e) {
+    for (size_t i = 0; i < entries.size(); i++)
+      if (entries[i].get() == e) return drop(i);
+  }
+  // every call looks at a few entries in turn for dead ones, one that packs at all of them
+  void drop_dead(size_t looks) {
+    for (; looks && !entries.empty(); looks--) {
+      if (next_look >= entries.size()) next_look = 0;
+      if (entries[next_look]->dead()) drop(next_look);
+      else next_look++;
+    }
+  }
+  void drop_all_dead() { drop_dead(entries.size()); }
+};
+PackedTable &g_packed = *new PackedTable;      // (no events destroyed after the runtime at exit)
 std::map<std::pair<int, void *>, Tensor> g_workspace, g_rw;
 int g_numerics = 0;     // 0 = w8a8 (this file), 1 = w8a16 (general path)
 
@@ -186,30 +229,23 @@ Packed packed(PackedForm form, std::initializer_list<const Tensor *> src, Make m
     C10_HIP_CHECK(hipStreamIsCapturing(stream.stream(), &status));
     return status != hipStreamCaptureStatusNone;
   };
-  auto found = g_packed.end();
-  for (auto e = g_packed.begin(); e != g_packed.end();) {
-    if (e->dead()) {
-      e = g_packed.erase(e);
-      continue;
-    }
-    if (e->form == form && e->ids == ids) found = e;
-    ++e;
-  }
-  const bool current = found != g_packed.end() && found->versions == versions;
+  const size_t hash = PackedTable::hash_of(form, ids);
+  g_packed.drop_dead(4);
+  PackedEntry *found = g_packed.find(form, ids, hash);
+  const bool current = found && found->versions == versions;
   if (!(current && found->ready.complete()) && capturing()) {
     PackGuard guard;
     Packed own{{}, nullptr};
     make(own.made);
     return own;
   }
-  if (found == g_packed.end()) {
-    PackedEntry e;
-    e.form = form;
-    e.ids = ids;
-    for (const Tensor *t : src) e.alive.push_back(t->storage().getWeakStorageImpl());
-    e.known_to_allocator.push_back(stream);
-    g_packed.push_back(std::move(e));
-    found = std::prev(g_packed.end());
+  if (!found) {
+    g_packed.drop_all_dead();
+    found = g_packed.add(hash);
+    found->form = form;
+    found->ids = ids;
+    for (const Tensor *t : src) found->alive.push_back(t->storage().getWeakStorageImpl());
+    found->known_to_allocator.push_back(stream);
   } else if (found->ready.event) {
     C10_HIP_CHECK(hipStreamWaitEvent(stream.stream(), found->ready.event, 0));
   }
@@ -220,7 +256,7 @@ Packed packed(PackedForm form, std::initializer_list<const Tensor *> src, Make m
       make(found->made);
       found->ready.record(stream.stream());
     } catch (...) {
-      g_packed.erase(found);
+      g_packed.drop(found);
       throw;
     }
     found->versions = versions;
@@ -232,7 +268,7 @@ Packed packed(PackedForm form, std::initializer_list<const Tensor *> src, Make m
       if (t.defined()) c10::hip::HIPCachingAllocator::recordStream(t.storage().data_ptr(), stream);
     known.push_back(stream);
   }
-  return {found->made, &*found};
+  return {found->made, found};
 }
 
 // Reference argument layout (gate [E,I,H], up [E,I,H], down pre-transposed [E,I,H], bf16 scales of the same
@@ -606,15 +642,16 @@ void _set_expert_numerics(int64_t mode) {
 
 void _invalidate_weight_cache() {
   std::lock_guard<std::mutex> lock(g_mutex);
-  g_packed.clear();
+  g_packed.entries.clear();
+  g_packed.hashes.clear();
 }
 
 // weight sets packed for tensors that are alive, every update of one counted again
 int64_t _packed_weight_sets() {
   std::lock_guard<std::mutex> lock(g_mutex);
   int64_t n = 0;
-  g_packed.remove_if([](const PackedEntry &e) { return e.dead(); });
-  for (auto &e : g_packed) n += e.packings;
+  g_packed.drop_all_dead();
+  for (auto &e : g_packed.entries) n += e->packings;
   return n;
 }
 
@@ -622,9 +659,9 @@ int64_t _packed_weight_sets() {
 int64_t _packed_weight_bytes() {
   std::lock_guard<std::mutex> lock(g_mutex);
   int64_t n = 0;
-  g_packed.remove_if([](const PackedEntry &e) { return e.dead(); });
-  for (auto &e : g_packed)
-    for (auto &t : e.made)
+  g_packed.drop_all_dead();
+  for (auto &e : g_packed.entries)
+    for (auto &t : e->made)
       if (t.defined()) n += (int64_t)t.nbytes();
   return n;
 }
