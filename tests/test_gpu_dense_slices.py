@@ -1,19 +1,30 @@
-"""Dense FP8 products whose reduction is cut into slices on the grouped kernel: the last slice shorter than the others,
-ragged row and column tiles, against the quantised operands' product in 64 bits."""
+"""Dense FP8 products whose reduction is cut into slices, on the grouped kernel (every tile height, the last slice as long as
+the others, shorter, a single step) and on the kernels of few rows, against the quantised operands' product in 64 bits."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 
-# 64-, 128- and 192-row tiles; 144, 128, 37 and 65 steps of 128; N that ends inside a 256-column strip
-@pytest.mark.parametrize("M,K,N", [(129, 18432, 7168), (300, 18432, 7168), (150, 14336, 4096), (520, 16384, 1024),
-                                   (33, 18432, 7168), (64, 16384, 1024), (128, 18432, 272), (32, 18432, 1024),
-                                   # a workgroup per 16 columns: 1, 2 and 4 row tiles, columns past the last eight
-                                   (1, 7168, 1536), (16, 2176, 1040), (32, 7168, 2048), (33, 4096, 2064), (64, 7168, 4096),
-                                   (17, 16384, 16), (31, 2304, 4096), (64, 7168, 4112),
-                                   (1501, 16384, 1008), (385, 4736, 272), (417, 8320, 16), (700, 16384, 1040)])
-def test_sliced_product(pkg, dev, M, K, N):
+# what the shape is to run: kernel, token rows of a work item, slices, steps of the last slice
+@pytest.mark.parametrize("M,K,N,plan", [
+    (33, 18432, 7168, ("sliced", 64, 9, 16)), (64, 16512, 4096, ("sliced", 64, 9, 1)), (50, 18560, 7168, ("sliced", 64, 5, 17)),
+    (64, 32768, 1024, ("sliced", 64, 16, 16)),
+    (150, 14336, 4096, ("sliced", 128, 7, 16)), (300, 18432, 7168, ("sliced", 128, 3, 48)), (520, 16512, 1024, ("sliced", 128, 9, 1)),
+    (300, 18560, 7168, ("sliced", 128, 3, 17)), (1000, 16640, 1040, ("sliced", 128, 5, 2)), (200, 16896, 4096, ("sliced", 128, 5, 4)),
+    (1501, 16384, 1008, ("sliced", 128, 4, 32)), (128, 18432, 272, ("sliced", 128, 9, 16)), (600, 8320, 272, ("sliced", 128, 5, 1)),
+    (520, 16384, 1024, ("sliced", 128, 8, 16)), (700, 16384, 1040, ("sliced", 128, 8, 16)),
+    (129, 18432, 7168, ("sliced", 192, 9, 16)), (150, 18560, 4096, ("sliced", 192, 10, 1)),
+    # a workgroup per 16 columns: 1, 2 and 4 row tiles, columns past the last eight, slices that end inside a batch of steps
+    (1, 7168, 1536, ("narrow", 16, 1, 56)), (16, 2176, 1040, ("narrow", 16, 1, 17)), (32, 7168, 2048, ("narrow", 16, 1, 56)),
+    (64, 16384, 1024, ("narrow", 16, 1, 128)), (32, 18432, 1024, ("narrow", 16, 1, 144)), (17, 16384, 16, ("narrow", 16, 1, 128)),
+    (31, 2304, 4096, ("narrow", 32, 1, 18)), (17, 4736, 4096, ("narrow", 32, 1, 37)), (33, 4096, 2064, ("narrow", 64, 1, 32)),
+    # a wavefront per work item
+    (17, 18432, 16, ("wavefront", 32, 36, 4)), (64, 7168, 4096, ("wavefront", 64, 14, 4)), (64, 7168, 4112, ("wavefront", 64, 7, 8)),
+    (385, 4736, 272, ("wavefront", 64, 10, 1)), (417, 8320, 16, ("wavefront", 64, 17, 1))])
+def test_sliced_product(pkg, dev, M, K, N, plan):
+    kernel, rows, slices, steps = pkg.ops.mm_plan(M, K, N)
+    assert (kernel, rows, slices, K // 128 - (slices - 1) * steps) == plan
     g = torch.Generator().manual_seed(M + K + N)
     x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(dev)
     w = (torch.randn(N, K, generator=g) * 100).clamp(-448, 448).to(torch.float8_e4m3fn).to(dev)

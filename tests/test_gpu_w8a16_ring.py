@@ -1,15 +1,18 @@
-"""The large-tile W8A16 kernels convert a step's weight codes during the step before, out of a register ring of four
-steps: reductions shorter than the ring, reductions that end inside it, and experts whose rows fill a part of the tile."""
+"""The large-tile W8A16 kernels convert a step's weight codes during the step before, out of a register ring of two steps, or
+of four under a long reduction: reductions shorter than the ring, reductions that end inside it, both sides of the rule
+between the two, and experts whose rows fill a part of the tile."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 
-# tokens x (H, I, E, K): 128- and 192-row tiles; a step is 64 elements, so H and I give 2, 4, 6, 10 and 16 steps
+# tokens x (H, I, E, K): 128- and 192-row tiles; a step is 64 elements, so H and I give 2, 4, 6, 10 and 16 steps, all in a
+# ring of two, and 36, 38, 40, 42, 44 and 48: a ring of four from 40 on where it divides the steps and a tile holds more than
+# 32 rows
 @pytest.mark.parametrize("T,H,I,E,K", [
     (200, 128, 128, 4, 1), (200, 384, 128, 4, 1), (160, 640, 384, 4, 2), (330, 128, 640, 4, 2), (700, 384, 256, 4, 2),
-    (333, 1024, 640, 8, 2),
+    (333, 1024, 640, 8, 2), (200, 2560, 2688, 4, 1), (330, 2816, 2304, 4, 2), (700, 2432, 3072, 4, 2),
 ])
 def test_codes_converted_a_step_ahead(pkg, dev, T, H, I, E, K):
     assert pkg.tile_rows(T, K, E) in (128, 192)
