@@ -252,8 +252,11 @@ int moe_fused_experts_w8a16(void *stream, const void *x_bf16, int T, int H, cons
  * multiple of 16.  Layers of few rows run on per-wavefront kernels that slice the reduction over the chip (the
  * slices are added in a fixed order; for the MLP the SwiGLU and re-quantisation ride in that reduction), the others
  * on the grouped kernel with one expert, whose reduction is sliced too where it is long and the output narrow.
- * Which of them runs is a function of (M, K, N), or (M, H, I), that decides the order of the sums, not the
- * arithmetic: a result is reproducible for a given shape.
+ * Which of them runs is a function of (M, K, N), or (M, H, I): a result is reproducible for a given shape.  It decides
+ * the order of the sums and, in the MLP, how the SwiGLU is formed in fp32 before its e4m3 rounding - with expf and
+ * divisions in the sliced reduction, with the hardware's exp2 and reciprocal on the grouped kernel, as in the expert path
+ * (33 to 128 rows, measured both ways: 0.159 % of the codes differ from 64-bit arithmetic's, the error of the values is
+ * the same to seven digits; the matrix instruction's own summation error decides).
  * moe_mlp_fp8 replaces at::mlp_w8a16_dq_forward -> tpudnnMlpW8A16DqAsync
  * (torch_tpu/csrc/ops/my_ops/MlpW8A16Dq.cpp:189-241): out [M, H] bf16 =
  * (silu(x Wg^T) * (x Wu^T)) Wd^T with w13 [2I, H] = gate rows then up rows, w2 [H, I].

@@ -54,7 +54,8 @@ int swiglu_quant_reduce_launch(hipStream_t st, const float *partial, int n_split
 // second product's reduction is then sliced (dense_split).  Small / grouped in us, gated width 18432 at 17 / 33 / 64 / 100 /
 // 128 rows 90 / 120 / 142 / 196 / 215 against 87 / 92 / 100 / 118 / 121; 14336: 55 / 61 / 72 / 90 / 102 against 54 / 57 / 63 / 57 /
 // 60; 12288 at 32 / 128 rows 77 / 144 against 81 / 94; 10240 at 64 / 128: 60 / 80 against 57 / 60; 8192: 54 / 67 against 55 / 59;
-// 2048 at 64 / 128: 38 / 46 against 60 / 68.
+// 2048 at 64 / 128: 38 / 46 against 60 / 68.  (Those with H = 4096 and 7168.  H decides little: at 128 rows under 8192 39 / 39 /
+// 49 / 106 against 35 / 39 / 46 / 81 with H = 512 / 1024 / 2048 / 8192; at 64 rows under 10240 95 against 86 with H = 8192.)
 static inline bool mlp_uses_small_kernel(int M, int I) {
   if (M > 128) return false;
   return M > 64 ? I < 8192 : M <= 32 || I < 12288;

@@ -611,9 +611,9 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
       // the conversions run beside matrix instructions; codes are asked for a step earlier to match.  A step's codes
       // sit in ring slot (step % R), its operands in wdq[step % 2].
       // A wavefront's 64 conversion instructions at the top of the step held up its matrix instructions; with that, the
-      // banks of tok_chunk0 and the longer ring the Mixtral-shaped layer at 333 tokens takes 437 -> 420 us (476 -> 453 on
-      // another card; the conversions and banks alone 451 -> 430), at 1500 tokens 1199 -> 1160, whose first product then
-      // runs at 1.07 PFLOP/s of the 1.24 that a large library product in bf16 reaches here.
+      // banks of tok_chunk0 and the longer ring the Mixtral-shaped layer at 333 tokens takes 3 to 5 % less (437 -> 420, 449 ->
+      // 435 and 476 -> 453 us on three cards), at 1500 tokens 1199 -> 1160, whose first product then runs at 1.07 PFLOP/s of
+      // the 1.24 that a large library product in bf16 reaches here.
       v8i wdq[DQ ? 2 : 1][WT];
       if constexpr (DQ) {
 #pragma unroll

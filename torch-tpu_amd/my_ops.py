@@ -5,10 +5,11 @@ The reference's own MoE ops - fused_moe_fused_experts, fused_moe_fused_experts_v
 fused_moe_grouped_topk - are registered from C++ as the reference registers them (`TORCH_LIBRARY(my_ops, m)` with
 function pointers, torch_tpu/csrc/ops/my_ops/myOps.cpp:29-80; signatures torch_tpu/csrc/ops/my_ops/ops.hpp:610-676,
 716-722): csrc/my_ops.cpp -> libmy_ops_torch.so, which forwards the common call straight to the C ABI.  This module
-loads that library, adds the ops the reference keeps elsewhere or leaves to its callers (the dense W8A16 / W8A8
-layers, the router recipe, the index building, the weight re-layout) as a fragment of the same namespace, and
-implements the rarer forms of the expert op (bf16 weights, other block sizes, ragged sizes, the W8A16 arithmetic)
-that the C++ op hands over to `my_ops::_fused_experts_general`.
+loads that library, adds the ops the reference keeps elsewhere or leaves to its callers (the dense W8A8 layer, the
+router recipe, the index building, the weight re-layout) as a fragment of the same namespace, and implements the rarer
+forms (bf16 weights, other block sizes, ragged sizes, the W8A16 arithmetic, strided tensors) of the expert op and of the
+dense ops mm_w8a16_dq_forward and mlp_w8a16_dq_forward, which the C++ ops hand over to `my_ops::_fused_experts_general`,
+`_mm_general` and `_mlp_general`.
 """
 from __future__ import annotations
 
