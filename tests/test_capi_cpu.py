@@ -341,3 +341,13 @@ def test_dense_workspace_of_a_batch_serves_every_smaller_one(pkg, K, N):
         if slices > 1:
             most = max(most, up(slices * m * N * 4))
         assert size >= up(m * K) + up(m * lib.moe_scale_pitch(K // 128) * 4) + most, (m, kernel, slices)
+
+
+@pytest.mark.parametrize("M", [1, 100, 200, 5000, 2**31 - 1])
+@pytest.mark.parametrize("H,I", [(64, 64), (8, 128), (128, 8), (16, 4096), (1 << 20, 256), (256, 1 << 30), (2**31 - 128, 2**31 - 128)])
+def test_dense_workspace_sizes_of_shapes_that_the_calls_refuse(pkg, M, H, I):
+    """The size functions are asked before the call: any positive sizes get a number, at once."""
+    lib = pkg._lib.lib
+    assert lib.moe_mlp_fp8_workspace_bytes(M, H, I) > 0
+    if H % 128 == 0 and I % 16 == 0:
+        assert lib.moe_mm_fp8_workspace_bytes(M, H, I) > 0

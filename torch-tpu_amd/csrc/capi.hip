@@ -565,7 +565,9 @@ struct DenseWs {
 // Bytes of the slices for M rows: of the only or second product, and of an MLP's first (MLP: K = H, N = H; first product
 // [M, 2I] over H, second [M, H] over I).
 static void dense_partial_bytes(int M, int K, int I, int N, size_t *first, size_t *last) {
-  *first = 0;
+  *first = *last = 0;
+  // (sizes that the calls refuse, but a size function may be asked about)
+  if (K < kBlock || N < 16 || (I > 0 && I < kBlock) || K > 32768 || I > 32768 || N > (1 << 20)) return;
   if (I > 0 ? mlp_uses_small_kernel(M, I) : mm_uses_small_kernel(M, K, N)) {
     if (I > 0) *first = dense_small_partial_bytes(M, K, 2 * I, true);
     *last = dense_small_partial_bytes(M, I > 0 ? I : K, N, false);
