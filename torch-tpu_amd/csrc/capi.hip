@@ -69,10 +69,10 @@ static inline bool mlp_uses_small_kernel(int M, int I) {
 // the sliced kernel up to 384 rows, one of at most 1024 up to 512: the grouped kernel has a handful of strips there
 // (7168 -> 1536 at 129 / 256 / 384 rows: 24 / 27 / 29 us against 34 / 35 / 36 us; 16384 -> 1024: 27 / 31 / 40 against
 // 67 / 69 / 70 us; 4096 -> 4096 is already the grouped kernel's).  From 33 rows on a reduction of 16384 or more is the
-// grouped kernel's, in slices (dense_split): 18432 -> 7168 at 64 / 128 rows 55 / 71 -> 40 / 44 us, 16384 -> 1024 at 128 / 300 /
+// grouped kernel's, in slices (dense_split): 18432 -> 7168 at 64 / 128 rows 54 / 71 -> 39 / 39 us, 16384 -> 1024 at 128 / 300 /
 // 500 rows 28.7 / 36 / 43.5 -> 27.6 / 31.5 / 33.6 us; at 17 rows nothing is gained.  Not where the narrow kernel takes the
-// layer whole (up to 64 rows; sliced / narrow in us at 64 rows: 16384 -> 1024 23.0 / 18.4, 24576 -> 1024 26.3 / 23.4, 32768 ->
-// 1024 27.5 / 31.5), and not for a layer of one strip, whose slices are too few for the units (16384 -> 256 at 100 / 200 / 500
+// layer whole (up to 64 rows; sliced / narrow in us at 64 rows: 16384 -> 1024 23.5 / 16.6, 24576 -> 1024 25.8 / 23.1, 32768 ->
+// 1024 27.0 / 28.5), and not for a layer of one strip, whose slices are too few for the units (16384 -> 256 at 100 / 200 / 500
 // rows sliced 24.3 / 27.3 / 32.5, on this kernel 22.7 / 26.7 / 31; 18432: 25.5 / 28.8 / 32.0 and 25.0 / 29.7 / 31.4, 24576: 26.8 /
 // 29.9 / 33.5 and 29.1 / 31.5 / 34.5).
 static inline bool mm_uses_small_kernel(int M, int K, int N) {
