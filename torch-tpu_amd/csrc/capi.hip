@@ -331,7 +331,7 @@ extern "C" int moe_fused_experts_fp8_rw(void *stream, const void *x_bf16, int T,
                                     w.slot_to_row, pw, zero_rows, H, (const uint16_t *)x_bf16, H, w.xq, w.xs);
     if (rc) return rc;
   } else {
-    // the activations are quantised by extra workgroups of the permutation's scan launch
+    // the activations are quantised by extra workgroups of the permutation's launch (of its scan, if there are three)
     const QuantJob job{(const uint16_t *)x_bf16, w.xq, w.xs, (size_t)T * (H / kBlock), H / kBlock, scale_pitch(H / kBlock)};
     rc = permute_launch(st, ids, T, K, E, choose_tile_m(T, K, E), w.sorted_slot, w.expert_offsets, w.slot_to_row, pw,
                         zero_rows, H, false, &job);
@@ -395,11 +395,11 @@ static int layer_fp8_run(void *stream, const void *x_bf16, int T, int H, const v
     if (may_use_side_stream && has_shared && I_sh == I && T >= kOverlapMinTokens && g_overlap_enabled.load())
       lane = side_lane(st);
     // the router product on the matrix cores, its reduction cut into slices; the routing kernel adds the slices.
-    // More than kChunk slots: the routing kernel also counts the slots per (chunk, expert) - the permutation's first
+    // More than kDirectSlots slots: the routing kernel also counts the slots per (chunk, expert) - the permutation's first
     // pass - into a table the router product's launch has cleared (table, per-expert totals and arrival counter are
     // one run of integers).
     int n_slices = 0;
-    const bool counted = (long)T * K > kChunk && (size_t)pw.n_chunks * E < ((size_t)1 << 30);
+    const bool counted = (long)T * K > kDirectSlots && (size_t)pw.n_chunks * E < ((size_t)1 << 30);
     int32_t *const zero = counted ? pw.chunk_counts : nullptr;
     const int n_zero = counted ? (int)(pw.arrivals + 1 - pw.chunk_counts) : 0;
     if (lane) {
@@ -427,7 +427,7 @@ static int layer_fp8_run(void *stream, const void *x_bf16, int T, int H, const v
       rc = router_front_launch(st, x_bf16, T, H, router_w_bf16, E, d.partial, &n_slices, zero, n_zero);
     }
     if (rc == MOE_OK && logits_out_bf16) rc = sum_slices_launch(st, d.partial, n_slices, T, E, (uint16_t *)logits_out_bf16);
-    // Unless the side stream quantises the activations, extra workgroups do: of the permutation's scan launch (a
+    // Unless the side stream quantises the activations, extra workgroups do: of the permutation's launch (a
     // few dozen workgroups of its own), or - up to kChunk slots, where the permutation is one workgroup - of the
     // routing launch.
     const bool ride_in_scan = !lane && (long)T * K > kChunk;

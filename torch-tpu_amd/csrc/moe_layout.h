@@ -6,7 +6,9 @@
 
 namespace moe {
 
-constexpr int kChunk = 256;   // slots ranked by one wavefront in the permutation kernels
+constexpr int kChunk = 256;   // slots ranked by one workgroup in the permutation kernels
+// Slots up to which the permutation is one launch that counts every id itself (permute_direct_kernel).
+constexpr int kDirectSlots = 64 * kChunk;
 
 // What the grouped GEMMs multiply: FP8 activations x FP8 weights with scales (the path proper), bf16 x bf16
 // (un-quantised experts), or bf16 activations x FP8 weights de-quantised to bf16 in registers (the reference's arithmetic)

@@ -1,7 +1,8 @@
 // Token permutation: a stable counting sort of the flattened [T*K] expert ids.
 //
-// Three small kernels, no host round trip (the grouped GEMMs that follow read the expert
-// offsets and the tile list from device memory):
+// No host round trip: the grouped GEMMs that follow read the expert offsets and the tile list from device memory.
+// Up to kChunk slots are done by one workgroup, up to kDirectSlots by one launch of a workgroup per chunk that counts all
+// ids for itself (permute_direct_kernel); larger problems by three small kernels:
 //   count    one wavefront per chunk of kChunk consecutive slots: per-chunk histogram in LDS.
 //   scan     one wavefront per expert: running sum over the chunks (turns the histogram into
 //            the chunk's starting rank inside its expert); the workgroup that finishes last adds
@@ -10,7 +11,6 @@
 //   scatter  one workgroup per chunk, one wavefront per 64 slots: ranks its slots in slot order
 //            with a ballot "match-any" loop, so equal experts keep their original order (stable),
 //            and writes sorted_slot / slot_to_row.
-// A problem of at most kChunk slots is done by one workgroup in a single launch.
 #include "moe_common.h"
 #include "moe_layout.h"
 #include "permute_small.h"
@@ -21,22 +21,21 @@ namespace moe {
 
 // rank of each lane among the lanes holding the same expert id, in lane order; also the
 // size of that set and whether the lane is the last of it.
-__device__ __forceinline__ void match_rank(int v, bool valid, int lane, int &rank, int &cnt, bool &is_last) {
-  uint64_t todo = __ballot(valid);
-  rank = 0; cnt = 0; is_last = false;
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  while (todo) {
-    int leader = __ffsll((unsigned long long)todo) - 1;
-    int lv = __shfl(v, leader, 64);
-    uint64_t m = __ballot(valid && v == lv);
-    if (valid && v == lv) {
-      rank = __popcll(m & lt);
-      cnt = __popcll(m);
-      is_last = (lane == 63 - __clzll((long long)m));
-    }
-    todo &= ~m;
+// One ballot per bit of the id: a lane's set is where all bits agree with its own.  (A loop over the distinct ids, each
+// fetched from its first lane, is up to 64 dependent rounds where the bits of 256 experts are 8.)
+__device__ __forceinline__ void match_rank(int v, bool valid, int lane, int n_bits, int &rank, int &cnt, bool &is_last) {
+  uint64_t m = __ballot(valid);
+  for (int b = 0; b < n_bits; b++) {
+    const bool one = (v >> b) & 1;
+    const uint64_t ones = __ballot(one);
+    m &= one ? ones : ~ones;
   }
+  if (!valid) m = 0;
+  rank = __popcll(m & ((1ull << lane) - 1));
+  cnt = __popcll(m);
+  is_last = valid && lane == 63 - __clzll((long long)m);
 }
+__device__ __forceinline__ int id_bits(int E) { return 32 - __clz(E - 1 | 1); }
 
 // The per-slot output row of a slot without an expert is zero: its one thread clears it (such slots are rare - a rank of
 // an expert-parallel group sees them for the experts it does not hold).  rows null: nothing to clear.
@@ -83,6 +82,64 @@ __device__ __forceinline__ int block_exclusive_scan(int x, int *lds_wave_sums, i
   __syncthreads();
   total = tot;
   return base + inc - x;
+}
+
+// What the GEMMs read, from the experts' totals (thread t of 256 holds those of experts 4 t .. 4 t + 3): the exclusive scan
+// over the experts -> expert_offsets, and the list of row tiles.
+struct ListSmem {
+  int wave_sums[16];
+  int t_first[MOE_MAX_EXPERTS + 1], t_count[MOE_MAX_EXPERTS], t_off[MOE_MAX_EXPERTS];
+};
+__device__ __forceinline__ void write_lists(ListSmem &sm, const int (&count)[4], int E, int tile_m, int max_tiles,
+                                            int32_t *__restrict__ expert_offsets, int32_t *__restrict__ tile_prefix,
+                                            int32_t *__restrict__ tile_expert, int32_t *__restrict__ tile_desc) {
+  int tiles[4], rows_mine = 0, tiles_mine = 0;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    tiles[j] = (count[j] + tile_m - 1) / tile_m;
+    rows_mine += count[j];
+    tiles_mine += tiles[j];
+  }
+  int total, total_tiles;
+  int off = block_exclusive_scan(rows_mine, sm.wave_sums, total);
+  int first_tile = block_exclusive_scan(tiles_mine, sm.wave_sums, total_tiles);
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int e = 4 * threadIdx.x + j;
+    if (e < E) {
+      expert_offsets[e] = off;
+      tile_prefix[e] = first_tile;
+    }
+    if (e < MOE_MAX_EXPERTS) {
+      sm.t_first[e] = e < E ? first_tile : total_tiles;
+      sm.t_count[e] = count[j];
+      sm.t_off[e] = off;
+    }
+    off += count[j];
+    first_tile += tiles[j];
+  }
+  if (threadIdx.x == 0) {
+    expert_offsets[E] = total;
+    tile_prefix[E] = total_tiles;
+    sm.t_first[MOE_MAX_EXPERTS] = total_tiles;
+  }
+  __syncthreads();
+  // The tile list, one thread per tile: under a skewed load one expert holds hundreds of row tiles, and a loop over
+  // them in that expert's thread would be the longest chain of the kernel.  A tile finds its expert by bisection of
+  // the first-tile table (experts without a tile share their successor's entry and are never the answer).
+  const int n_tiles = min(total_tiles, max_tiles);
+  for (int j = threadIdx.x; j < n_tiles; j += 256) {
+    int lo = 0, hi = E;                                 // sm.t_first[lo] <= j < sm.t_first[hi]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (sm.t_first[mid] <= j) lo = mid; else hi = mid;
+    }
+    const int c = sm.t_count[lo];
+    tile_expert[j] = lo;
+    v4i *d = (v4i *)(tile_desc + (size_t)j * 8);
+    d[0] = (v4i){lo, sm.t_first[lo], (c + tile_m - 1) / tile_m, sm.t_off[lo]};
+    d[1] = (v4i){c, 0, 0, 0};
+  }
 }
 
 // Scan.  First half, one wavefront per expert: a running sum over the chunks turns each chunk's histogram entry into
@@ -150,59 +207,16 @@ __global__ __launch_bounds__(64 * kScanWaves) void permute_scan_kernel(int32_t *
   if (!is_last) return;
   __threadfence();
 
-  __shared__ int wave_sums[16];
-  __shared__ int t_first[MOE_MAX_EXPERTS + 1], t_count[MOE_MAX_EXPERTS], t_off[MOE_MAX_EXPERTS];
   // thread t owns experts 4 t .. 4 t + 3 (MOE_MAX_EXPERTS = 4 x 256 threads)
   static_assert(MOE_MAX_EXPERTS <= 4 * 64 * kScanWaves, "four experts per thread");
-  int count[4], tiles[4], rows_mine = 0, tiles_mine = 0;
+  __shared__ ListSmem lists;
+  int count[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int e = 4 * threadIdx.x + j;
     count[j] = e < E ? __hip_atomic_load(expert_count + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
-    tiles[j] = (count[j] + tile_m - 1) / tile_m;
-    rows_mine += count[j];
-    tiles_mine += tiles[j];
   }
-  int total, total_tiles;
-  int off = block_exclusive_scan(rows_mine, wave_sums, total);
-  int first_tile = block_exclusive_scan(tiles_mine, wave_sums, total_tiles);
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const int e = 4 * threadIdx.x + j;
-    if (e < E) {
-      expert_offsets[e] = off;
-      tile_prefix[e] = first_tile;
-    }
-    if (e < MOE_MAX_EXPERTS) {
-      t_first[e] = e < E ? first_tile : total_tiles;
-      t_count[e] = count[j];
-      t_off[e] = off;
-    }
-    off += count[j];
-    first_tile += tiles[j];
-  }
-  if (threadIdx.x == 0) {
-    expert_offsets[E] = total;
-    tile_prefix[E] = total_tiles;
-    t_first[MOE_MAX_EXPERTS] = total_tiles;
-  }
-  __syncthreads();
-  // The tile list, one thread per tile: under a skewed load one expert holds hundreds of row tiles, and a loop over
-  // them in that expert's thread would be the longest chain of the kernel.  A tile finds its expert by bisection of
-  // the first-tile table (experts without a tile share their successor's entry and are never the answer).
-  const int n_tiles = min(total_tiles, max_tiles);
-  for (int j = threadIdx.x; j < n_tiles; j += 64 * kScanWaves) {
-    int lo = 0, hi = E;                                 // t_first[lo] <= j < t_first[hi]
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (t_first[mid] <= j) lo = mid; else hi = mid;
-    }
-    const int c = t_count[lo];
-    tile_expert[j] = lo;
-    v4i *d = (v4i *)(tile_desc + (size_t)j * 8);
-    d[0] = (v4i){lo, t_first[lo], (c + tile_m - 1) / tile_m, t_off[lo]};
-    d[1] = (v4i){c, 0, 0, 0};
-  }
+  write_lists(lists, count, E, tile_m, max_tiles, expert_offsets, tile_prefix, tile_expert, tile_desc);
 }
 
 // One workgroup per chunk, one wavefront per 64 consecutive slots of it: every wavefront ranks its
@@ -228,7 +242,7 @@ __global__ __launch_bounds__(kChunk) void permute_scatter_kernel(const int32_t *
   const bool valid = s < TK && v >= 0 && v < E;
   int rank, cnt;
   bool is_last;
-  match_rank(v, valid, lane, rank, cnt, is_last);
+  match_rank(v, valid, lane, id_bits(E), rank, cnt, is_last);
   __syncthreads();
   if (valid && is_last) wcount[wave][v] = cnt;
   __syncthreads();
@@ -240,6 +254,96 @@ __global__ __launch_bounds__(kChunk) void permute_scatter_kernel(const int32_t *
   if (valid && row < TK) sorted_slot[row] = s;
   if (s < TK) slot_to_row[s] = row;
   if (s < TK && row < 0) zero_slot_row(zero_rows, row_len, s);
+}
+
+// The whole permutation in one launch, up to kDirectSlots: a workgroup per chunk reads every id - the 64 KB come from L2 -
+// and counts those before its chunk apart from the rest, so that it knows the offsets of its own slots without waiting for
+// anybody; one more workgroup leaves the offsets and the tile list, and those after it quantise the activations.  Three (with
+// counts from the routing launch two) short dependent launches of 5 to 8 us each, a few dozen workgroups, become one.  Whole
+// calls, before -> after in us: Qwen3 shape at 300 / 1500 tokens 148.5 -> 137.4 / 198.8 -> 189.3, its un-quantised experts at 2048
+// tokens (64 chunks) 329 -> 320, the per-slot op at 470 tokens 149.6 -> 137.4, 81 experts of 1152 x 384 at 1143 tokens 65.9 ->
+// 55.1, Mixtral shape at 256 tokens 326 -> 318, 8 experts of 256 x 512 at 516 tokens 46.2 -> 38.8.
+// Reading everything grows with the square of the chunks: above kDirectSlots the three kernels take over.
+__global__ __launch_bounds__(kChunk) void permute_direct_kernel(
+    const int32_t *__restrict__ ids, int TK, int E, int n_chunks, int tile_m, int max_tiles,
+    int32_t *__restrict__ sorted_slot, int32_t *__restrict__ expert_offsets, int32_t *__restrict__ slot_to_row,
+    int32_t *__restrict__ tile_prefix, int32_t *__restrict__ tile_expert, int32_t *__restrict__ tile_desc,
+    uint16_t *__restrict__ zero_rows, int row_len, const QuantJob ride) {
+  if ((int)blockIdx.x > n_chunks) {
+    act_quant_thread(ride.x, ride.n_groups, ride.groups_per_row, ride.pitch, ride.q, ride.s,
+                     (size_t)(blockIdx.x - n_chunks - 1) * kChunk + threadIdx.x);
+    return;
+  }
+  constexpr int NWV = kChunk / 64;
+  struct Place {
+    int wave_sums[16];
+    int wcount[NWV][MOE_MAX_EXPERTS];
+  };
+  __shared__ int before[MOE_MAX_EXPERTS], rest[MOE_MAX_EXPERTS];
+  __shared__ union { Place place; ListSmem lists; } sm;
+  // the workgroup of the lists goes first: its chain is the longer one
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = blockIdx.x == 0 ? n_chunks : (int)blockIdx.x - 1;
+  for (int e = tid; e < E; e += kChunk) {
+    before[e] = 0;
+    rest[e] = 0;
+    if (c < n_chunks) {
+#pragma unroll
+      for (int w = 0; w < NWV; w++) sm.place.wcount[w][e] = 0;
+    }
+  }
+  __syncthreads();
+  constexpr int B = 16;                                  // chunks asked for at a time
+  int v = -1;
+  for (int i0 = 0; i0 < n_chunks; i0 += B) {
+    int id[B];
+#pragma unroll
+    for (int i = 0; i < B; i++) {
+      const int s = (i0 + i) * kChunk + tid;
+      id[i] = s < TK ? ids[s] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < B; i++) {
+      if (i0 + i == c) v = id[i];
+      if (id[i] >= 0 && id[i] < E) atomicAdd(i0 + i < c ? &before[id[i]] : &rest[id[i]], 1);
+    }
+  }
+  __syncthreads();
+  static_assert(MOE_MAX_EXPERTS <= 4 * kChunk, "four experts per thread");
+  int first[4], count[4], mine = 0;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const int e = 4 * tid + j;
+    first[j] = e < E ? before[e] : 0;
+    count[j] = e < E ? first[j] + rest[e] : 0;
+    mine += count[j];
+  }
+  if (c == n_chunks) {
+    write_lists(sm.lists, count, E, tile_m, max_tiles, expert_offsets, tile_prefix, tile_expert, tile_desc);
+    return;
+  }
+  const int s = c * kChunk + tid;
+  const bool valid = v >= 0 && v < E;
+  int rank, cnt, total;
+  bool is_last;
+  match_rank(v, valid, lane, id_bits(E), rank, cnt, is_last);
+  if (is_last) sm.place.wcount[wave][v] = cnt;
+  int off = block_exclusive_scan(mine, sm.place.wave_sums, total);
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    if (4 * tid + j < E) before[4 * tid + j] = off + first[j];       // where the expert's slots of this chunk begin
+    off += count[j];
+  }
+  __syncthreads();
+  int row = -1;
+  if (valid) {
+    row = before[v] + rank;
+    for (int w = 0; w < wave; w++) row += sm.place.wcount[w][v];
+    sorted_slot[row] = s;
+  }
+  if (s < TK) {
+    slot_to_row[s] = row;
+    if (row < 0) zero_slot_row(zero_rows, row_len, s);
+  }
 }
 
 __global__ __launch_bounds__(kChunk) void permute_small_kernel(const int32_t *__restrict__ ids, int TK, int E, int tile_m,
@@ -295,7 +399,7 @@ int permute_quant_small_launch(hipStream_t st, const int32_t *ids, int T, int K,
 // zero_rows (may be null): a [T*K, row_len] bf16 tensor in slot order whose rows of slots WITHOUT an expert (id outside
 // [0, E)) are cleared here - the per-slot output form: nothing else ever writes those rows
 // counted: the routing launch has filled ws.chunk_counts and ws.arrivals is zero (more than kChunk slots only)
-// ride (may be null; more than kChunk slots only): activations quantised by extra workgroups of the scan launch
+// ride (may be null; more than kChunk slots only): activations quantised by extra workgroups of the launch (of the scan, if there are three)
 int permute_launch(hipStream_t st, const int32_t *ids, int T, int K, int E, int tile_m, int32_t *sorted_slot,
                    int32_t *expert_offsets, int32_t *slot_to_row, const PermuteWs &ws, uint16_t *zero_rows, int row_len,
                    bool counted, const QuantJob *ride) {
@@ -305,10 +409,16 @@ int permute_launch(hipStream_t st, const int32_t *ids, int T, int K, int E, int 
                                            ws.tile_prefix, ws.tile_expert, ws.tile_desc, zero_rows, row_len);
     return (int)hipGetLastError();
   }
-  if (!counted) permute_count_kernel<<<ws.n_chunks, 64, 0, st>>>(ids, TK, E, ws.chunk_counts, ws.arrivals);
-  static_assert(64 * kScanWaves == 256, "a quantising workgroup has 256 threads");
-  const int n_scan = (E + kScanWaves - 1) / kScanWaves;
   const QuantJob job = ride ? *ride : QuantJob{};
+  if (!counted && TK <= kDirectSlots) {
+    permute_direct_kernel<<<ws.n_chunks + 1 + job.blocks(), kChunk, 0, st>>>(
+        ids, TK, E, ws.n_chunks, tile_m, ws.max_tiles, sorted_slot, expert_offsets, slot_to_row, ws.tile_prefix, ws.tile_expert,
+        ws.tile_desc, zero_rows, row_len, job);
+    return (int)hipGetLastError();
+  }
+  if (!counted) permute_count_kernel<<<ws.n_chunks, 64, 0, st>>>(ids, TK, E, ws.chunk_counts, ws.arrivals);
+  static_assert(64 * kScanWaves == 256 && kChunk == 256, "a quantising workgroup has 256 threads");
+  const int n_scan = (E + kScanWaves - 1) / kScanWaves;
   permute_scan_kernel<<<n_scan + job.blocks(), 64 * kScanWaves, 0, st>>>(
       ws.chunk_counts, ws.n_chunks, E, tile_m, ws.max_tiles, expert_offsets, ws.tile_prefix, ws.tile_expert, ws.tile_desc,
       ws.expert_count, ws.arrivals, n_scan, job);
