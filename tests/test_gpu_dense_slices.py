@@ -41,6 +41,31 @@ def test_sliced_product(pkg, dev, M, K, N, plan):
     assert torch.equal(out.view(torch.int16), pkg.mm_fp8(x, pkg.pack_weights(w), ws).view(torch.int16))
 
 
+# strips of 128 columns: whole under 128- and 192-row tiles, and slices; a last row tile of one m-tile (its second wavefront
+# of a pair has none), of one row, whole; columns that end inside a strip; an odd number of steps; exactly one round of items
+@pytest.mark.parametrize("M,K,N,plan", [
+    (300, 7168, 7168, ("grouped", 128, 1, 56)), (385, 2176, 7152, ("grouped", 128, 1, 17)), (1040, 2048, 2000, ("grouped", 128, 1, 16)),
+    (2048, 4096, 2048, ("grouped", 128, 1, 32)), (140, 4096, 28672, ("grouped", 192, 1, 32)), (1155, 4224, 4096, ("grouped", 192, 1, 33)),
+    (400, 7168, 1536, ("sliced", 128, 4, 8)), (560, 7296, 1520, ("sliced", 128, 4, 9)), (200, 7168, 2112, ("sliced", 128, 4, 8))])
+def test_strips_of_128_columns(pkg, dev, M, K, N, plan):
+    test_sliced_product(pkg, dev, M, K, N, plan)
+
+
+@pytest.mark.parametrize("M,K,N", [(300, 7168, 7168), (385, 2176, 7152), (1155, 4224, 4096)])
+def test_whole_products_in_strips_of_128_columns_keep_every_sum(pkg, dev, M, K, N):
+    """The rows' bits are those of a batch that takes the wide strips; an infinity in the last step adds no NaN."""
+    g = torch.Generator().manual_seed(M + K)
+    w, ws = (t[0] for t in pkg.synthetic_weights(1, -(-N // 128) * 128, K, dev, 5))
+    w, n = w[:N].contiguous(), -(-N // 128)
+    x = torch.randn(4096, K, generator=g).to(torch.bfloat16).to(dev)
+    got = pkg.mm_fp8(x[:M].contiguous(), w, ws[:n])
+    assert torch.equal(got, pkg.mm_fp8(x, w, ws[:n])[:M])
+    xi = x[:M].clone()
+    xi[M - 1, K - 1] = float("inf")
+    inf = pkg.mm_fp8(xi, w, ws[:n])
+    assert torch.equal(inf[:M - 1], got[:M - 1]) and not inf[M - 1].isnan().all()
+
+
 @pytest.mark.parametrize("M,H,I", [(33, 1024, 12288), (64, 256, 12416), (65, 512, 8192), (128, 1024, 18432), (257, 512, 9216)])
 def test_gated_mlp_of_few_rows_on_the_grouped_kernels(pkg, dev, M, H, I):
     """Against the same layer run row block by row block on the per-wavefront kernels (at most 32 rows)."""

@@ -175,14 +175,22 @@ __device__ __forceinline__ void mma_bf16(v4f (&acc)[WT], const v8i (&w)[WT], con
 //        v_mfma_f32_16x16x32_bf16 accumulating in place), no scales, bf16 intermediate
 // SLICED a dense second product cut along its reduction: a work item is a slice of a tile's steps, its fp32 sums go to
 //        a.partial (an instantiation of its own, so that the whole products carry nothing of it)
-template <int MT, int NW, int DEPTH, bool GATED, bool WREG, bool BF16 = false, int TPS = 16, bool DQ = false, bool SLICED = false>
+// PAIR   strips of 128 columns under a large tile (dense products whose strips of 256 are too few for the units): two
+//        wavefronts share a column group of the strip, each with half of the tile's live m-tiles.  Both load the group's
+//        weights, the second time from the unit's own cache, and each reads half of the token tile from LDS.  Alone in the
+//        chip's one round, a step takes about three quarters of what the wide strip's takes (7168 -> 1536 at 3072 / 2048 rows,
+//        144 / 192 items: 58 / 44 us for the op); a chip full of wide items is better off with those (4001 rows 62 and 68 us).
+template <int MT, int NW, int DEPTH, bool GATED, bool WREG, bool BF16 = false, int TPS = 16, bool DQ = false, bool SLICED = false,
+          bool PAIR = false>
 // Four wavefronts with the weights in registers: two such workgroups share a compute unit (256 registers a lane each)
 __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_gemm_kernel(const GemmArgs a) {
   static_assert(!DQ || BF16, "de-quantised weights feed the bf16 matrix instructions");
-  static_assert(TPS % NW == 0 && (TPS == 16 || (!GATED && !WREG && TPS <= 8)), "narrow strips: second GEMM, operands through LDS");
+  static_assert(PAIR || (TPS % NW == 0 && (TPS == 16 || (!GATED && !WREG && TPS <= 8))), "narrow strips: second GEMM, operands through LDS");
+  static_assert(!PAIR || (!GATED && WREG && !BF16 && NW == 8 && TPS == 8 && MT % 4 == 0), "paired wavefronts: dense products, FP8");
   constexpr int BM = 16 * MT;
   constexpr int NT = 64 * NW;                         // threads
-  constexpr int WT = TPS / NW;                        // weight tiles per wavefront
+  constexpr int WT = PAIR ? 2 * TPS / NW : TPS / NW;  // weight tiles per wavefront
+  constexpr int MTW = PAIR ? MT / 2 : MT;             // m-tiles per wavefront, at most
   constexpr int STAGES = WREG ? 4 : DEPTH + 1;        // token tiles staged in LDS
   constexpr int WLDS = DQ ? 1024 : 2048;              // bytes of a weight tile's step in LDS (DQ: one half of a block)
   using Smem = GemmSmem<MT, NW, STAGES, WREG ? 1 : STAGES, WREG ? 64 : WLDS, TPS, WREG || !BF16>;
@@ -192,6 +200,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wcol = PAIR ? wave >> 1 : wave;           // which of the strip's column groups
   const int li = lane & 15, lg = lane >> 4;
 
   // ---- which tile -------------------------------------------------------------------------
@@ -205,7 +214,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   const int n_mtiles = n_routed + (a.sh_rows + BM - 1) / BM;
   // Each XCD takes an equal share of the shared expert's work items (full tiles: the heaviest, so
   // they go first) and then an equal, contiguous share of the routed ones.
-  static_assert(!SLICED || (!GATED && !BF16 && TPS == 16), "slices: second product on FP8 operands, wide strips");
+  static_assert(!SLICED || (!GATED && !BF16 && (TPS == 16 || PAIR)), "slices: second product on FP8 operands, tall tiles");
   const int n_slice_work = n_routed * a.n_strips;      // work items of one slice
   const int n_routed_work = SLICED ? n_slice_work * a.n_slices : n_slice_work;
   const int n_shared_work = (n_mtiles - n_routed) * a.n_strips;
@@ -282,6 +291,12 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   const int rows_a = shared ? a.sh_rows : a.rows_a;
   if (rows <= 0) return;
   const int mt_live = (rows + 15) >> 4;               // m-tiles that hold at least one row
+  // PAIR: the even wavefront of a pair takes the lower half of the live m-tiles, the odd one the rest (of a single m-tile
+  // none: it then walks the empty one above it, whose rows are copies of a live one, and stores nothing)
+  const int mt_low = (mt_live + 1) >> 1;
+  const int mt_first = PAIR && (wave & 1) ? mt_low : 0;
+  const int mt_mine = PAIR ? ((wave & 1) ? mt_live - mt_low : mt_low) : mt_live;
+  const int mt_run = PAIR ? max(mt_mine, 1) : mt_live;
   const bool stream_weights = n_mt == 1;              // the expert's rows fit this one row tile
 
   const int n_kb = a.Kd >> 7;                         // 128-steps of the whole reduction
@@ -297,7 +312,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   for (int j = 0; j < WT; j++) {
     int wrow;
     if (GATED) wrow = (j < WT / 2 ? 0 : a.N) + strip * 128 + wave * (8 * WT) + (j % (WT / 2)) * 16;
-    else wrow = strip * (16 * TPS) + wave * (16 * WT) + j * 16;
+    else wrow = strip * (16 * TPS) + wcol * (16 * WT) + j * 16;
     wrow = min(wrow, a.n_rows_w - 16);                 // tiles past the matrix re-read its last rows
     wtile[j] = wq + ((size_t)e * a.n_rows_w + wrow) * (DQ ? a.Kd >> 1 : a.Kd) + (SLICED ? (size_t)kb_first * 2048 : 0);
   }
@@ -339,7 +354,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     if (tid < 8) sm.sb[tid >> 2][NKB + (tid & 3)] = 0.f;
   }
   __syncthreads();
-  const int sb_row0 = GATED ? 0 : (wave * WT) / 8;      // which of the two rows this wavefront's tiles use
+  const int sb_row0 = GATED ? 0 : (wcol * WT) / 8;      // which of the two rows this wavefront's tiles use
   const int sb_row1 = GATED ? 1 : sb_row0;
   // Token tile -> LDS by direct loads: one instruction moves 64 x 16 bytes = 8 rows x 128 bytes to
   // LDS bytes [M0 + 16*lane); the XOR swizzle is applied on the source side (lane l fetches the
@@ -380,9 +395,9 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   constexpr uint32_t kTokStage = BM * 128, kSacBuf = MT * 1024;
   const int n_chunks = (NKB + 15) >> 4;
 
-  v4f acc[MT][WT];
+  v4f acc[MTW][WT];
 #pragma unroll
-  for (int mt = 0; mt < MT; mt++)
+  for (int mt = 0; mt < MTW; mt++)
 #pragma unroll
     for (int j = 0; j < WT; j++) acc[mt][j] = (v4f){0.f, 0.f, 0.f, 0.f};
 
@@ -600,9 +615,9 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
       constexpr int LIVE = decltype(live_c)::value;
       constexpr int R = decltype(ring_c)::value;         // ring slots in use = steps per pass of the unrolled loop
       constexpr int L_WAIT = NTOK + LPT * WT * (R / 2);  // loads younger than the ones a step boundary needs
-      static_assert(LIVE % 2 == 0 && LIVE >= 2 && LIVE <= MT, "live m-tiles come in pairs");
+      static_assert(LIVE % 2 == 0 && LIVE >= 2 && LIVE <= MTW, "live m-tiles come in pairs");
       constexpr int PD = 2;                              // m-tiles between an LDS read and its use
-      const bool top_empty = mt_live < LIVE;             // uniform: the top m-tile of the top pair holds no row
+      const bool top_empty = mt_run < LIVE;              // uniform: the top m-tile of the top pair holds no row
       // the first requests go out inside the instantiation: no branch may sit between a register
       // load's request and its wait (the compiler would copy the registers while the load is in flight)
       request(0, 0);
@@ -645,9 +660,9 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
         if (tid < BM) {
           const int kc = min(k, last);                   // past the end: a finite scale times the zero behind the table
           float sa = sm.sac[(kc >> 4) & 1][(tid >> 4) * 256 + ((kc & 12) << 4) + (tid & 15) * 4 + (kc & 3)];
-          // (an infinite scale would make NaN of the zero.  The whole products leave it at that: the select costs 1 % of a
-          // prefill layer, and a register that the 96-row kernel does not have)
-          if (SLICED && k > last) sa = 0.f;
+          // (an infinite scale would make NaN of the zero.  The whole products of wide strips leave it at that: the select costs
+          // 1 % of a prefill layer, and a register that the 96-row kernel does not have)
+          if ((SLICED || PAIR) && k > last) sa = 0.f;
           sm.fsc[k & 3][tid] = make_float2(sa * sm.sb[0][k], sa * sm.sb[1][k]);
         }
       };
@@ -656,14 +671,14 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
       produce_f(2);
       __syncthreads();
       auto read_x = [&](int kb, int mt) {
-        const uint8_t *t = sm.tok[kb & 3] + li * 128 + mt * 2048;
+        const uint8_t *t = sm.tok[kb & 3] + li * 128 + (mt_first + mt) * 2048;
         return concat8(*(const v4i *)(t + o0), *(const v4i *)(t + o1));
       };
       // GATED: both products (gate tiles use .x, up tiles .y); second GEMM: the one of this wavefront's column block
       auto read_f = [&](int kb, int mt) {
         if (BF16) return make_float2(0.f, 0.f);
         if (GATED) return sm.fsc[kb & 3][mt * 16 + li];
-        const float f = ((const float *)&sm.fsc[kb & 3][mt * 16 + li])[sb_row0];
+        const float f = ((const float *)&sm.fsc[kb & 3][(mt_first + mt) * 16 + li])[sb_row0];
         return make_float2(f, f);
       };
       v8i x[XB];
@@ -785,8 +800,8 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
     };
     auto pick = [&](auto self, auto live_c, auto ring_c) -> void {
       constexpr int LIVE = decltype(live_c)::value;
-      if constexpr (LIVE >= MT) run(std::integral_constant<int, MT>{}, ring_c);
-      else if (mt_live <= LIVE) run(live_c, ring_c);
+      if constexpr (LIVE >= MTW) run(std::integral_constant<int, MTW>{}, ring_c);
+      else if (mt_run <= LIVE) run(live_c, ring_c);
       else self(self, std::integral_constant<int, LIVE + 2>{}, ring_c);
     };
     using short_ring = std::integral_constant<int, 2>;
@@ -884,26 +899,26 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
   } else if constexpr (SLICED) {
     // a slice of the product: fp32, straight from the registers (16 bytes per lane, 64 per row and tile)
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-      const int r = mt * 16 + li;
+    for (int mt = 0; mt < MTW; mt++) {
+      const int r = (mt_first + mt) * 16 + li;
 #pragma unroll
       for (int j = 0; j < WT; j++) {
-        const int col = strip * (16 * TPS) + (wave * WT + j) * 16 + lg * 4;
-        if (r < rows && col < a.N)
+        const int col = strip * (16 * TPS) + (wcol * WT + j) * 16 + lg * 4;
+        if (mt < mt_mine && r < rows && col < a.N)
           *(v4f *)(a.partial + ((size_t)slice * a.rows_a + row0 + r) * a.N + col) = acc[mt][j];
       }
     }
     return;
   } else {
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-      if (mt < mt_live) {
+    for (int mt = 0; mt < MTW; mt++) {
+      if (mt < mt_mine) {
 #pragma unroll
         for (int j = 0; j < WT; j++) {
           v2i o;
           o[0] = (int)pack2_bf16(acc[mt][j][0], acc[mt][j][1]);
           o[1] = (int)pack2_bf16(acc[mt][j][2], acc[mt][j][3]);
-          *(v2i *)(stage + (mt * 16 + li) * RS + (wave * (16 * WT) + j * 16 + lg * 4) * 2) = o;
+          *(v2i *)(stage + ((mt_first + mt) * 16 + li) * RS + (wcol * (16 * WT) + j * 16 + lg * 4) * 2) = o;
         }
       }
     }
@@ -930,7 +945,7 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
 // tile_m: row tile of the tile list (grouped mode) or of this launch (dense mode); routed_tiles: entries of the list
 // (an upper bound known on the host) or row tiles of the dense matrix; mean_rows: rows per expert on average.
 template <bool GATED, bool BF16 = false, bool DQ = false>
-static int launch_gemm(hipStream_t st, GemmArgs &a, int tile_m, int routed_tiles, double mean_rows) {
+static int launch_gemm(hipStream_t st, GemmArgs &a, int tile_m, int routed_tiles, double mean_rows, bool pair = false) {
   // the kernel keeps one weight-block scale per 128-step in LDS and forms per-lane operand offsets in 32 bits
   if (a.Kd < 128 || a.Kd % 128 || (a.Kd >> 7) > kMaxKB) return MOE_E_SHAPE;
   if ((double)a.rows_a * a.Kd >= 2147483648.0 || (double)a.sh_rows * a.Kd >= 2147483648.0) return MOE_E_SHAPE;
@@ -957,8 +972,8 @@ static int launch_gemm(hipStream_t st, GemmArgs &a, int tile_m, int routed_tiles
   // round (a dense 7168 -> 7168 product at 288-384 rows, 140-168 wide items: 64 us in narrow strips, 46 us in wide ones).
   // (a dense layer knows its row tiles; the tile list's entries are an upper bound, a few more than the real ones -
   // Mixtral shape at 48-96 tokens: 9-11 entries for 8 real tiles of 16 strips each - hence the wider margin there)
-  const bool narrow = !GATED && !a.partial && (km <= 32 || (km == 64 && row_tiles * ((a.N + 255) / 256) < (a.fixed_expert >= 0 ? 129 : 193)));
-  a.n_strips = GATED ? a.N / 128 : narrow ? (a.N + 63) / 64 : (a.N + 255) / 256;
+  const bool narrow = !GATED && !pair && !a.partial && (km <= 32 || (km == 64 && row_tiles * ((a.N + 255) / 256) < (a.fixed_expert >= 0 ? 129 : 193)));
+  a.n_strips = GATED ? a.N / 128 : pair ? (a.N + 127) / 128 : narrow ? (a.N + 63) / 64 : (a.N + 255) / 256;
   a.max_mtiles = routed_tiles;
   long total = row_tiles * a.n_strips * (a.partial ? a.n_slices : 1);
   total = (total + 7) / 8 * 8 + 16;                  // the per-XCD split rounds two shares up
@@ -981,6 +996,15 @@ static int launch_gemm(hipStream_t st, GemmArgs &a, int tile_m, int routed_tiles
     }
   }
   if constexpr (!GATED && !BF16) {
+    if (pair) {
+#define MOE_GEMM_PAIR(MT, SLICED) grouped_gemm_kernel<MT, 8, 2, false, true, false, 8, false, SLICED, true><<<grid, dim3(512), 0, st>>>(a)
+      if (km == 128 && a.partial) MOE_GEMM_PAIR(8, true);
+      else if (km == 128) MOE_GEMM_PAIR(8, false);
+      else if (km == 192 && !a.partial) MOE_GEMM_PAIR(12, false);
+      else return MOE_E_SHAPE;
+#undef MOE_GEMM_PAIR
+      return (int)hipGetLastError();
+    }
     if (a.partial) {
 #define MOE_GEMM_SLICED(MT, WREG) grouped_gemm_kernel<MT, 8, 2, false, WREG, false, 16, false, true><<<grid, dim3(512), 0, st>>>(a)
       switch (km) {
@@ -1068,16 +1092,16 @@ int gemm2_launch(hipStream_t st, const uint8_t *hq, const float *hs, int rows_a,
 int dense_product_launch(hipStream_t st, const uint8_t *xq, const float *xs, int M, int K, const uint8_t *w, const float *ws,
                          int N, uint16_t *out, float *partial) {
   const DenseSplit sp = dense_split(M, K, N);
-  if (sp.slices == 1)
+  if (sp.slices == 1 && sp.cols == 256)
     return gemm2_launch(st, xq, xs, M, M, N, w, ws, K, 1, 1, nullptr, nullptr, nullptr, 0, out, nullptr, nullptr, 0, nullptr,
                         nullptr, nullptr, kNumericsFp8);
   GemmArgs a{};
   a.aq = xq; a.as = xs; a.w = w; a.ws = ws; a.y = out;
   a.as_pitch = scale_pitch(K / kBlock);
   a.Kd = K; a.N = N; a.n_rows_w = N; a.rows_a = M; a.topk = 1; a.E = 1; a.fixed_expert = 0;
-  a.k_steps = sp.k_steps; a.n_slices = sp.slices; a.partial = partial;
-  const int rc = launch_gemm<false>(st, a, sp.tile_m, (M + sp.tile_m - 1) / sp.tile_m, (double)M);
-  if (rc) return rc;
+  a.k_steps = sp.k_steps; a.n_slices = sp.slices; a.partial = sp.slices > 1 ? partial : nullptr;
+  const int rc = launch_gemm<false>(st, a, sp.tile_m, (M + sp.tile_m - 1) / sp.tile_m, (double)M, sp.cols == 128);
+  if (rc || sp.slices == 1) return rc;
   return splitk_reduce_launch(st, partial, sp.slices, (size_t)M * N, out);
 }
 

@@ -84,12 +84,22 @@ static inline int choose_dense_tile_m(long rows, int items_per_row_tile, int ste
 // Measured, whole op, before -> after: 16384 -> 1024 at 520 / 700 / 1500 / 4000 rows 70 / 72 / 83 / 126 -> 34 / 36 / 53 / 105 us;
 // gated MLP 7168 / 18432 at 129 / 300 / 400 rows 165 / 209 / 245 -> 130 / 174 / 219 us (the second product 115 -> 57 + 6 us at 300
 // rows, 2.3 TB/s of weights), 4096 / 14336 at 129 / 300 / 600 rows 99 / 107 / 167 -> 71 / 85 / 146 us.
+//
+// Strips of 128 columns (paired wavefronts, more than 128 rows and 256 columns) are twice the work items, each with a step of
+// about 1100 cycles under 128 rows.  Whole, they take a layer whose narrow items are more than half a round and no more than one: the
+// wide 64-row tiles that it gets otherwise are one round of 1500-cycle steps.  192 rows likewise, where 128 are too many
+// items.  Sliced, they compete by the model, which lets a layer of few strips have them.  Measured, whole op, before ->
+// after in us: 7168 -> 1536 at 400 / 560 / 1500 / 2000 rows 28.6 / 35.3 / 50.6 / 53.6 -> 24.9 / 26.0 / 41.6 / 44.2, 7168 -> 7168 at
+// 300 / 400 rows 46.3 / 48.0 -> 38.1 / 39.5, 4096 -> 4096 at 560 / 800 rows 30.3 / 31.5 -> 27.2 / 28.9, 16384 -> 1024 at 140 / 400
+// rows 28.5 / 31.1 -> 23.8 / 27.0, 7168 -> 2112 at 200 / 1100 rows 27.8 / 48.7 -> 22.9 / 40.8, 4096 -> 28672 at 140 rows (192-row
+// tile) 39.6 -> 30.9.  Outside the line: fewer items 4096 -> 4096 at 300 rows (96) 24.8 -> 25.4, 2048 -> 7168 at 200 rows (112)
+// 15.6 -> 16.4; more 7168 -> 1536 at 2800 rows (264) 59.5 -> 78.4; short reductions 512 -> 4096 at 800 rows 10.7 -> 11.6.
 struct DenseSplit {
-  int tile_m, slices, k_steps;
+  int tile_m, slices, k_steps, cols;                     // cols: output columns of a strip, 256 or 128
 };
 static inline DenseSplit dense_split(long rows, int K, int N) {
   const int steps = K / 128, strips = (N + 255) / 256;
-  DenseSplit best = {choose_dense_tile_m(rows, strips, steps), 1, steps};
+  DenseSplit best = {choose_dense_tile_m(rows, strips, steps), 1, steps, 256};
   const auto rounds = [](long items) { return (double)((items + 255) / 256); };
   double best_cost;
   {
@@ -105,14 +115,28 @@ static inline DenseSplit dense_split(long rows, int K, int N) {
       const int slices = (steps + len - 1) / len;
       const double cost = rounds(items * slices) * (len * (300.0 + 150.0 * (tm / 16)) + 20000.0) + 10000.0 +
                           8.0 * slices * (double)rows * N / 2000.0;
-      if (cost < best_cost) { best = {tm, slices, len}; best_cost = cost; }
+      if (cost < best_cost) { best = {tm, slices, len, 256}; best_cost = cost; }
     }
+  }
+  if (rows <= 128 || N <= 256) return best;
+  const int pair_strips = (N + 127) / 128;
+  const long pair128 = (rows + 127) / 128 * (long)pair_strips, pair192 = (rows + 191) / 192 * (long)pair_strips;
+  if (best.slices == 1) {
+    if (steps >= 16 && pair128 > 128 && pair128 <= 256) best = {128, 1, steps, 128};
+    else if (steps >= 32 && pair128 > 256 && pair192 > 128 && pair192 <= 224) best = {192, 1, steps, 128};
+  }
+  best_cost *= 0.94;                                     // (where the model sees less, the two measure the same)
+  for (int len = 16; len < steps; len += 16) {
+    const int slices = (steps + len - 1) / len;
+    const double cost = rounds(pair128 * slices) * (len * 1100.0 + 20000.0) + 10000.0 + 8.0 * slices * (double)rows * N / 2000.0;
+    if (cost < best_cost) { best = {128, slices, len, 128}; best_cost = cost; }
   }
   return best;
 }
 // No product of more rows is sliced: with q rounds of whole items of a tall tile the slices cost at least q (steps x step +
 // 40 000) cycles and the whole product at most 0.87 / 0.97 (q + 1)(steps x step + 20 000) - the tile that is chosen is at
-// most 1 / 0.97 dearer than any other, and not the 64-row one from four rounds on - which is less from q = 9 on.  (At least
+// most 1 / 0.97 dearer than any other, and not the 64-row one from four rounds on - which is less from q = 9 on.  (Narrow strips
+// are the dearer slices there: two or more wide strips of N > 256 columns make at least 2 s - 1 narrow ones of 1100 cycles.  At least
 // 512: up to there the per-wavefront kernels have slices of their own.)
 static inline long dense_split_max_rows(int K, int N) {
   return K / 128 > 16 ? 512 + 192 * (9 * 256 / ((N + 255) / 256) + 1l) : 512;
