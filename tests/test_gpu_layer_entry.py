@@ -510,3 +510,40 @@ def test_module_form_holds_its_weights_as_buffers(pkg, oracle, dev):
                                shared=tuple(torch.zeros_like(t) for t in sh))
     other.load_state_dict(state)
     assert torch.equal(other(x).view(torch.int16), out.view(torch.int16))
+
+
+@pytest.mark.parametrize("T", [1, 40, 600])
+@pytest.mark.parametrize("odd", ["none", "out", "bias", "shared", "workspace of words", "strided out", "bf16 scales", "other device's"])
+def test_layer_entry_native_road_and_the_other_agree(pkg, dev, T, odd):
+    """ops.layer_fp8 in the form that is taken natively, against the same call asking for the routing (which is not); what
+    the native road does not take runs or raises as it does there."""
+    E, H, I, K = 16, 256, 256, 2
+    w13, w2 = pkg.synthetic_weights(E, 2 * I, H, dev, 1), pkg.synthetic_weights(E, H, I, dev, 2)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
+    wr = (torch.randn(E, H, generator=g) * 0.1).to(torch.bfloat16).to(dev)
+    kw = dict(mode="sigmoid")
+    if odd == "bias":
+        kw["bias"] = torch.randn(E, generator=g).to(dev)
+    if odd == "shared":
+        kw["shared"] = (*pkg.synthetic_weights(1, 2 * I, H, dev, 3), *pkg.synthetic_weights(1, H, I, dev, 4))
+    need = pkg.layer_workspace_bytes(T, H, I, E, K, I if odd == "shared" else 0)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    want = pkg.layer_fp8(x, wr, *w13, *w2, K, return_routing=True, **kw)[0]
+    if odd == "out":
+        kw["out"] = torch.empty(T, H, dtype=torch.bfloat16, device=dev)
+    if odd == "workspace of words":
+        ws = torch.empty(need // 4, dtype=torch.int32, device=dev)
+    if odd in ("strided out", "bf16 scales", "other device's"):
+        if odd == "strided out":
+            kw["out"] = torch.empty(T, 2 * H, dtype=torch.bfloat16, device=dev)[:, ::2]
+        scale = w13[1].to(torch.bfloat16) if odd == "bf16 scales" else w13[1]
+        with pytest.raises(RuntimeError):
+            pkg.layer_fp8(x.cpu() if odd.startswith("other") else x, wr, w13[0], scale, *w2, K, workspace=ws, **kw)
+        return
+    got = pkg.layer_fp8(x, wr, *w13, *w2, K, workspace=ws, **kw)
+    assert torch.equal(got, want)
+    if odd == "out":
+        assert got is kw["out"]
+    with pytest.raises(RuntimeError):
+        pkg.layer_fp8(x, wr, *w13, *w2, K, workspace=ws[:ws.numel() - 1], **{k: v for k, v in kw.items() if k != "out"})

@@ -16,6 +16,7 @@
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -655,6 +656,52 @@ int64_t _packed_weight_sets() {
   return n;
 }
 
+// ---- the layer's one call ---------------------------------------------------------------------------------------------
+// moe_layer_fp8 for the common form of ops.layer_fp8: every operand plain and on the current device.  The checks and the call
+// took 20 us of Python per layer call, as long as all launches of a small layer (256 x 512, 8 experts, 1 to 100 tokens).
+// Returns the library's code, or kNotPlain for any other form: the caller's own road then says what is wrong, or runs it.
+constexpr int64_t kNotPlain = 1 << 20;
+
+bool plain_tensor(const Tensor &t, c10::ScalarType dtype, at::IntArrayRef sizes, const Tensor &like) {
+  return t.scalar_type() == dtype && t.sizes() == sizes && t.is_cuda() && t.device() == like.device() && t.is_contiguous();
+}
+
+int64_t _layer_fp8(const Tensor &x, const Tensor &router, const Tensor &w13, const Tensor &w13s, const Tensor &w2, const Tensor &w2s,
+                   int64_t top_k, int64_t mode, const OptTensor &bias, int64_t n_groups, int64_t topk_groups, bool renorm,
+                   double scale, const OptTensor &sh13, const OptTensor &sh13s, const OptTensor &sh2, const OptTensor &sh2s,
+                   const Tensor &out, const Tensor &workspace) {
+  if (x.dim() != 2 || w13.dim() != 3 || !x.is_cuda() || x.device().index() != c10::hip::current_device()) return kNotPlain;
+  const int64_t T = x.size(0), H = x.size(1), E = w13.size(0), I = w13.size(1) / 2;
+  const auto fits = [](int64_t v) { return v >= 0 && v < (1ll << 31); };
+  if (!fits(T) || !fits(H) || !fits(I) || E < 1 || E > 1024 || top_k < 1 || top_k > E || H % 128 || I % 128 || !fits(n_groups) ||
+      !fits(topk_groups))
+    return kNotPlain;
+  const auto fp8 = at::kFloat8_e4m3fn;
+  if (!plain_tensor(x, at::kBFloat16, {T, H}, x) || !plain_tensor(router, at::kBFloat16, {E, H}, x) ||
+      !plain_tensor(w13, fp8, {E, 2 * I, H}, x) || !plain_tensor(w13s, at::kFloat, {E, 2 * I / 128, H / 128}, x) ||
+      !plain_tensor(w2, fp8, {E, H, I}, x) || !plain_tensor(w2s, at::kFloat, {E, H / 128, I / 128}, x) ||
+      !plain_tensor(out, at::kBFloat16, {T, H}, x) || !plain_tensor(workspace, at::kByte, {workspace.numel()}, x) ||
+      (bias && !plain_tensor(*bias, at::kFloat, {E}, x)))
+    return kNotPlain;
+  int64_t I_sh = 0;
+  if (sh13) {
+    if (!sh13s || !sh2 || !sh2s || sh13->dim() != 3) return kNotPlain;
+    I_sh = sh13->size(1) / 2;
+    if (I_sh < 128 || I_sh % 128 || !fits(I_sh) || !plain_tensor(*sh13, fp8, {1, 2 * I_sh, H}, x) ||
+        !plain_tensor(*sh13s, at::kFloat, {1, 2 * I_sh / 128, H / 128}, x) || !plain_tensor(*sh2, fp8, {1, H, I_sh}, x) ||
+        !plain_tensor(*sh2s, at::kFloat, {1, H / 128, I_sh / 128}, x))
+      return kNotPlain;
+  }
+  if ((size_t)workspace.numel() < moe_layer_fp8_workspace_bytes((int)T, (int)H, (int)I, (int)E, (int)top_k, (int)I_sh)) return kNotPlain;
+  return moe_layer_fp8(stream_of(x), x.data_ptr(), (int)T, (int)H, router.data_ptr(), bias ? bias->data_ptr<float>() : nullptr,
+                       (int)E, (int)top_k, (int)mode, (int)n_groups, (int)topk_groups, renorm, (float)scale,
+                       (const uint8_t *)w13.data_ptr(), w13s.data_ptr<float>(), (const uint8_t *)w2.data_ptr(),
+                       w2s.data_ptr<float>(), (int)I, sh13 ? (const uint8_t *)sh13->data_ptr() : nullptr,
+                       sh13 ? sh13s->data_ptr<float>() : nullptr, sh13 ? (const uint8_t *)sh2->data_ptr() : nullptr,
+                       sh13 ? sh2s->data_ptr<float>() : nullptr, (int)I_sh, out.data_ptr(), nullptr, nullptr, nullptr,
+                       workspace.data_ptr(), (size_t)workspace.numel());
+}
+
 // memory that the packed copies hold
 int64_t _packed_weight_bytes() {
   std::lock_guard<std::mutex> lock(g_mutex);
@@ -682,6 +729,7 @@ TORCH_LIBRARY(my_ops, m) {
   m.def("_mm_weights(Tensor weight, Tensor scale) -> Tensor[]");
   m.def("_mlp_weights(Tensor gate_weight, Tensor up_weight, Tensor down_weight, Tensor gate_scale, Tensor up_scale, "
         "Tensor down_scale) -> Tensor[]");
+  m.def("_layer_fp8", _layer_fp8);
   m.def("_packed_weight_sets", _packed_weight_sets);
   m.def("_packed_weight_bytes", _packed_weight_bytes);
 }

@@ -275,8 +275,13 @@ def router_logits(x, router_weight, out=None, workspace=None):
     return out
 
 
+@functools.lru_cache(maxsize=4096)
 def layer_workspace_bytes(T, H, I, E, K, I_shared=0) -> int:
     return lib.moe_layer_fp8_workspace_bytes(T, H, I, E, K, I_shared)
+
+
+_LAYER_MODES = {"softmax": ROUTE_SOFTMAX, "sigmoid": ROUTE_SIGMOID, "softmax_logit_bias": ROUTE_SOFTMAX_LOGIT_BIAS}
+_NOT_PLAIN = 1 << 20     # my_ops::_layer_fp8: not the form that it takes
 
 
 def layer_fp8(x, router_weight, w13, w13_scale, w2, w2_scale, top_k: int, mode: str = "softmax", bias=None,
@@ -288,8 +293,17 @@ def layer_fp8(x, router_weight, w13, w13_scale, w2, w2_scale, top_k: int, mode: 
     or (out, logits bf16 [T,E], weights fp32 [T,k], ids int32 [T,k]) with return_routing.
     static_scratch: use the library's built-in scratch array instead of a workspace (moe_layer_fp8_static: no
     device allocation when `out` is given; small batches only, calls on one GPU must not overlap)."""
-    modes = {"softmax": ROUTE_SOFTMAX, "sigmoid": ROUTE_SIGMOID, "softmax_logit_bias": ROUTE_SOFTMAX_LOGIT_BIAS}
+    modes = _LAYER_MODES
     _need(mode in modes, f"unknown routing mode {mode!r}")
+    # The common form natively; any other, and what is wrong with one, below.  A tracer sees the calls below, as ever.
+    if workspace is not None and not (return_routing or static_scratch) and not torch.compiler.is_compiling():
+        result = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if out is None else out
+        sh = (None, None, None, None) if shared is None else shared
+        rc = torch.ops.my_ops._layer_fp8.default(x, router_weight, w13, w13_scale, w2, w2_scale, top_k, modes[mode], bias, n_groups,
+                                                 topk_groups, bool(renorm), float(scale), *sh, result, workspace)
+        if rc != _NOT_PLAIN:
+            check(rc, "layer_fp8")
+            return result
     _need(x.dim() == 2 and w13.dim() == 3 and w2.dim() == 3 and router_weight.dim() == 2, "bad ranks")
     T, H = x.shape
     E, I2, H2 = w13.shape
