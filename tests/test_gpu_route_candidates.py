@@ -32,3 +32,29 @@ def test_picks_of_one_token_equal_the_whole_rows(pkg, dev, E, K, n_groups, topk_
         w, ids = pkg.moe_route(x[t0:t0 + 8].contiguous(), *args)
         assert torch.equal(ids, ids_all[t0:t0 + 8])
         assert torch.equal(w.view(torch.int32), w_all[t0:t0 + 8].view(torch.int32))
+
+
+# every road of the selection: one token to a workgroup, one to a wavefront, groups of 32 and others
+@pytest.mark.parametrize("T", [7, 96])
+@pytest.mark.parametrize("E,K,n_groups,topk_groups", [(8, 2, 1, 1), (128, 8, 1, 1), (256, 8, 8, 4), (60, 7, 12, 5), (249, 8, 3, 2), (300, 8, 1, 1)])
+def test_nan_scores_come_first_whatever_the_batch(pkg, oracle, dev, T, E, K, n_groups, topk_groups):
+    """NaN of either sign before everything else, lower index first, in a row and among the groups' sums: the oracle's order
+    (torch.sort), on every road."""
+    g = torch.Generator().manual_seed(E + T)
+    x = torch.randn(T, E, generator=g)
+    both = torch.tensor([0x7fc00000, 0xffc00000 - 2 ** 32], dtype=torch.int32).view(torch.float32)
+    where = torch.rand(T, E, generator=g) < 0.02
+    x[where] = both[torch.randint(0, 2, (int(where.sum()),), generator=g)]
+    x[1] = both[1]                                        # nothing but NaN
+    x[2, : E // n_groups] = both[0]                       # a whole group (or everything)
+    x[3] = float("-inf")
+    x[3, E // 2] = both[1]
+    x[4, 0], x[4, 1:E // n_groups] = float("inf"), float("-inf")         # a group whose sum is NaN
+    want, want_ids = oracle.select_sigmoid_grouped(x, None, K, n_groups, topk_groups, scale=1.0, renorm=False)
+    w, ids = pkg.moe_route(x.to(dev), K, "scores", None, n_groups, topk_groups, renorm=False)
+    assert torch.equal(ids.cpu(), want_ids)
+    torch.testing.assert_close(w.cpu(), want, rtol=0, atol=0, equal_nan=True)
+    if n_groups > 1:
+        values, idx = torch.empty(T, K, device=dev), torch.empty(T, K, dtype=torch.int32, device=dev)
+        pkg.noaux_tc_topk(values, idx, x.to(dev), n_groups, topk_groups, K)
+        assert torch.equal(idx.cpu(), want_ids)

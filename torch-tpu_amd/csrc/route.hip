@@ -15,7 +15,8 @@ namespace moe {
 
 
 // A candidate is one 64-bit key: the score's bits mapped monotonically onto unsigned integers in the upper half
-// (-0 counts as +0, NaN sorts below -inf: it never wins), the complement of the element index in the lower half.
+// (-0 counts as +0, a NaN of either sign comes before everything, as torch.sort and torch.topk order it), the complement
+// of the element index in the lower half.
 // "Greater value, then lower index" is then a single unsigned comparison, candidates of one row never compare equal,
 // and 0 - below every real candidate - stands for "no candidate".
 typedef unsigned long long cand_t;
@@ -24,7 +25,7 @@ __device__ __forceinline__ uint32_t ordered_bits(float x) {
   uint32_t b = __float_as_uint(x);
   if (x == 0.f) b = 0;
   uint32_t u = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-  if (x != x) u = 1;
+  if (x != x) u = 0xffffffffu;
   return u;
 }
 __device__ __forceinline__ cand_t make_cand(float v, int index) {
@@ -145,9 +146,10 @@ __device__ __forceinline__ void select_row(float (&v)[PER_LANE], int E, int lane
     // the topk_groups best groups: lane g counts the groups that come before its own in
     // "greater score, then lower index" order
     int rank = 0;
+    const uint32_t mine = ordered_bits(gscore);
     for (int g = 0; g < n_groups; g++) {
-      const float s = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, gscore), g));
-      rank += (s > gscore || (s == gscore && g < lane)) ? 1 : 0;
+      const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)mine, g);
+      rank += (s > mine || (s == mine && g < lane)) ? 1 : 0;
     }
     const uint64_t keep = __ballot(lane < n_groups && rank < topk_groups);
 #pragma unroll

@@ -31,10 +31,10 @@ struct RouteBlockSmem {
 };
 
 // (score a, index ai) comes before (b, bi) - greater score, then lower index - exactly when
-// order_key(a, ai) > order_key(b, bi).  Adding +0 first makes -0 and +0 the same key, as they compare equal.
+// order_key(a, ai) > order_key(b, bi).  Adding +0 first makes -0 and +0 the same key, as they compare equal; NaN comes first.
 __device__ __forceinline__ uint64_t order_key(float v, int idx) {
   uint32_t u = __float_as_uint(v + 0.0f);
-  u = (u >> 31) ? ~u : (u | 0x80000000u);
+  u = v != v ? 0xffffffffu : (u >> 31) ? ~u : (u | 0x80000000u);
   return ((uint64_t)u << 32) | (uint32_t)(0x7fffffff - idx);
 }
 
