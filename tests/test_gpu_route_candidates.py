@@ -58,3 +58,18 @@ def test_nan_scores_come_first_whatever_the_batch(pkg, oracle, dev, T, E, K, n_g
         values, idx = torch.empty(T, K, device=dev), torch.empty(T, K, dtype=torch.int32, device=dev)
         pkg.noaux_tc_topk(values, idx, x.to(dev), n_groups, topk_groups, K)
         assert torch.equal(idx.cpu(), want_ids)
+
+
+@pytest.mark.parametrize("E,K,n_groups,topk_groups", [(256, 8, 8, 4), (256, 32, 8, 1), (256, 32, 8, 7), (128, 6, 64, 3), (249, 8, 3, 2), (4, 2, 2, 1)])
+def test_fewer_finite_scores_than_picks_under_a_group_limit(pkg, oracle, dev, E, K, n_groups, topk_groups):
+    """Row t has t finite scores, from none to more than K: the rest of the picks are -inf ones, lowest index first, of kept and
+    dropped groups alike."""
+    g = torch.Generator().manual_seed(E + K)
+    T = min(K + 3, E)
+    x = torch.full((T, E), float("-inf"))
+    for t in range(T):
+        x[t, torch.randperm(E, generator=g)[:t]] = torch.randn(t, generator=g)
+    _, want_ids = oracle.select_sigmoid_grouped(x, None, K, n_groups, topk_groups, renorm=False)
+    for rows in (x, x.repeat(65 // T + 1, 1)):            # a workgroup per token, and more than 64 tokens
+        _, ids = pkg.moe_route(rows.to(dev), K, "scores", None, n_groups, topk_groups, renorm=False)
+        assert torch.equal(ids[:T].cpu(), want_ids) and torch.equal(ids[-T:].cpu(), want_ids)

@@ -27,7 +27,7 @@ struct RouteBlockSmem {
   float wmax[kRouteBlock / 64];
   float wsel[64];              // weight source of pick k
   int isel[64];                // expert of pick k
-  int unsure;                  // the last pick is no better than what the group limit masked
+  int above[kRouteBlock / 64], level[kRouteBlock / 64];   // experts better than -inf under the group limit, and at -inf, per wavefront
 };
 
 // (score a, index ai) comes before (b, bi) - greater score, then lower index - exactly when
@@ -57,7 +57,6 @@ __device__ __forceinline__ void route_block(RouteBlockSmem &sm, const void *logi
   float v = (bias != nullptr && live) ? x + bias[e] : x;  // what the selection looks at
   if (scores_row != nullptr && live && mode != MOE_ROUTE_SOFTMAX) scores_row[e] = x;
   if (e < 64) { sm.isel[e] = -1; sm.wsel[e] = 0.f; }
-  if (e == 0) sm.unsure = 0;
   sm.cand[e] = 0;
   float denom_all = 0.f;
   if (mode == MOE_ROUTE_SOFTMAX) {
@@ -86,10 +85,11 @@ __device__ __forceinline__ void route_block(RouteBlockSmem &sm, const void *logi
 
   // First the position inside a part of the row - the expert's group, or the 64 experts of its wavefront: a pick is among
   // the K best of its part, so only those are compared with one another afterwards.  Against one pass over the whole
-  // table that is 32 + 32 compares instead of 32 + 256 for the DeepSeek-V3 router, 64 + 16 for 128 experts: whole layers at
-  // one token 89.7 -> 87.7 us (DeepSeek shape), 35.4 -> 34.3 (Qwen3 shape), 85.3 -> 83.1 (Mixtral shape, whose eight experts
-  // used to be compared with 256 entries; part of it the 32-bit division of the weighted sum).
-  const bool grouped = n_groups > 1;
+  // table that is 32 + 32 compares instead of 32 + 256 for the DeepSeek-V3 router, 64 + 16 for 128 experts.  A launch of one
+  // token, one pass -> parts, in us: 256 experts in 8 groups, 8 picks 5.8 -> 3.7 (with fewer than 8 finite scores in the kept
+  // groups 5.9 -> 3.8), 32 picks 5.8 -> 4.5; 256 experts without groups, 8 / 32 picks 4.8 -> 3.7 / 4.5; 128 experts 4.6 -> 3.5;
+  // 8 experts 4.7 -> 2.7.
+  const bool grouped = n_groups > 1 && topk_groups < n_groups;       // (a limit that keeps every group is none)
   const int per = grouped ? E / n_groups : 64;
   const int part = live ? (grouped ? e / per : wave) : 0, first = part * per, last = min(first + per, E);
   int pos = 0;                                            // position in the part
@@ -98,6 +98,8 @@ __device__ __forceinline__ void route_block(RouteBlockSmem &sm, const void *logi
     for (int j = first; j < last; j++) pos += sm.key[j] > key;
   }
   int n_parts = (E + 63) / 64, place = part;              // parts still in question, and which of them this one is
+  bool low = false;                                       // -inf, as it came or by the limit
+  uint64_t lows = 0;
   if (grouped) {
     if (live && pos < 2) sm.gtop[part][pos] = v;
     __syncthreads();
@@ -110,36 +112,36 @@ __device__ __forceinline__ void route_block(RouteBlockSmem &sm, const void *logi
       for (int h = 0; h < n_groups; h++) place += sm.gkey[h] > gk;
     }
     n_parts = topk_groups;
+    // Experts of dropped groups stay candidates with -inf, as a masked_fill would leave them.  Nothing sorts below that, so
+    // such an expert's position in the row is the number of better ones plus the number of its like before it.
+    low = live && (place >= topk_groups || key <= order_key(-INFINITY, 0));
+    lows = __ballot(low);
+    const uint64_t better = __ballot(live && !low);
+    if (lane == 0) {
+      sm.above[wave] = __popcll(better);
+      sm.level[wave] = __popcll(lows);
+    }
   }
   const int kept = min(K, per), n_cand = n_parts * kept;  // at least K (the caller has checked topk_groups * per >= K)
-  const bool masked = grouped && topk_groups < n_groups;
-  if (live && place < n_parts && pos < kept) sm.cand[place * kept + pos] = key;
+  if (live && !low && place < n_parts && pos < kept) sm.cand[place * kept + pos] = key;
   __syncthreads();
-  if (e < n_cand && sm.cand[e] != 0) {
-    const uint64_t mine = sm.cand[e];
+  if (low) {
+    int r = __popcll(lows & ((1ull << lane) - 1));
+#pragma unroll
+    for (int w = 0; w < kRouteBlock / 64; w++) r += sm.above[w] + (w < wave ? sm.level[w] : 0);
+    if (r < K) { sm.isel[r] = e; sm.wsel[r] = raw; }
+  }
+  const uint64_t mine = sm.cand[e];
+  if (mine != 0) {
     int r = 0;
-#pragma unroll 8
-    for (int j = 0; j < n_cand; j++) r += sm.cand[j] > mine;
+    for (int j0 = 0; j0 < n_cand; j0 += 16) {             // (0 beyond the candidates: whole batches of reads)
+#pragma unroll
+      for (int j = 0; j < 16; j++) r += sm.cand[j0 + j] > mine;
+    }
     if (r < K) {
       const int who = 0x7fffffff - (int)(uint32_t)mine;
       sm.isel[r] = who;
       sm.wsel[r] = sm.raw[who];
-    }
-    // experts of dropped groups stay candidates with -inf, as a masked_fill would leave them
-    if (masked && r == K - 1 && mine <= order_key(-INFINITY, 0)) sm.unsure = 1;
-  }
-  if (masked) {
-    __syncthreads();
-    if (sm.unsure) {                                      // rare: the whole table, with the dropped groups at -inf
-      if (live && place >= n_parts) key = order_key(-INFINITY, e);
-      sm.key[e] = key;
-      __syncthreads();
-      if (live) {
-        int r = 0;
-#pragma unroll 8
-        for (int j = 0; j < E; j++) r += sm.key[j] > key;
-        if (r < K) { sm.isel[r] = e; sm.wsel[r] = raw; }
-      }
     }
   }
   __syncthreads();
