@@ -28,8 +28,7 @@ __global__ __launch_bounds__(256) void weighted_reduce_kernel(const uint16_t *__
   const int hv = H >> 3;   // 16-byte vectors per row
   const size_t idx = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (size_t)T * hv) return;
-  // (a 64-bit division is a fair part of what the launch of a single token takes)
-  const int t = idx >> 32 ? (int)(idx / hv) : (int)((uint32_t)idx / (uint32_t)hv), c = (int)(idx - (size_t)t * hv) * 8;
+  const int t = (int)(idx / hv), c = (int)(idx % hv) * 8;
   float acc[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) acc[i] = 0.f;
