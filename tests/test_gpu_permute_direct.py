@@ -59,3 +59,24 @@ def test_one_hot_expert_and_empty_ones_reach_the_gemms(pkg, oracle, dev, T):
     big = pkg.fused_experts_fp8(x, *ld, ids)
     for lo in (0, T // 2, T - 40):
         assert torch.equal(big[lo:lo + 40], pkg.fused_experts_fp8(x[lo:lo + 40].contiguous(), *ld, ids[lo:lo + 40].contiguous()))
+
+
+# one and two picks, chunks on either side of the line from which counts are kept in copies, experts at the edges of 8, 4, 2 and 1
+@pytest.mark.parametrize("T,K,E", [(6144, 1, 8), (6145, 1, 8), (DIRECT_SLOTS, 1, 1), (DIRECT_SLOTS, 1, 128), (DIRECT_SLOTS, 1, 129), (16001, 1, 256),
+                                   (DIRECT_SLOTS, 1, 257), (DIRECT_SLOTS, 1, 512), (12345, 1, 513), (DIRECT_SLOTS // 2, 2, 2), (8111, 2, 64),
+                                   (DIRECT_SLOTS // 2, 2, 65)])
+@pytest.mark.parametrize("load", ["even", "collapsed", "half outside"])
+def test_counts_kept_in_copies_add_up(pkg, dev, T, K, E, load):
+    ids = _ids(T, K, E, T + E, 0.5 if load == "half outside" else 0.0)
+    if load == "collapsed":
+        ids[:] = torch.arange(E - K, E, dtype=torch.int32)
+    ss, off, s2r = (t.cpu() for t in pkg.moe_permute(ids.to(dev), E))
+    flat = ids.flatten().long()
+    valid = (flat >= 0) & (flat < E)
+    n = int(valid.sum())
+    want = torch.sort(torch.where(valid, flat, E), stable=True).indices[:n]
+    rows = torch.full((T * K,), -1)
+    rows[want] = torch.arange(n)
+    assert torch.equal(ss[:n].long(), want) and torch.equal(s2r.long(), rows)
+    counts = torch.bincount(flat[valid], minlength=E)
+    assert torch.equal(off.long(), torch.cat([torch.zeros(1, dtype=torch.long), counts.cumsum(0)]))

@@ -264,8 +264,26 @@ __global__ __launch_bounds__(kChunk) void permute_scatter_kernel(const int32_t *
 // tokens (64 chunks) 329 -> 320, the per-slot op at 470 tokens 149.6 -> 137.4, 81 experts of 1152 x 384 at 1143 tokens 65.9 ->
 // 55.1, Mixtral shape at 256 tokens 326 -> 318, 8 experts of 256 x 512 at 516 tokens 46.2 -> 38.8.
 // Reading everything grows with the square of the chunks: above kDirectSlots the three kernels take over.
+//
+// SPREAD: lanes that add to one counter wait for one another, and a wavefront whose 64 slots all ask for one expert takes
+// about ten times as long to count as one whose slots differ.  The experts of a token are distinct, so K picks put at most
+// 64 / K slots of a wavefront on one expert.  For one pick, and for two among few experts, a load that collapsed made the
+// launch as slow as the three that it replaces from 30 chunks on, and slower above.  From there the counts are kept in several
+// copies, neighbouring lanes adding to different ones (at an odd pitch: the copies of a counter sit in different banks), which
+// are added up afterwards.  Three launches / one copy / copies in us, every slot on the first K experts: 16384 x 1 slots, 8
+// experts 10.5 / 18.0 / 9.5, 256 experts 12.6 / 18.2 / 10.1, 512 experts 14.7 / 18.5 / 12.8; 8192 x 2, 8 experts 10.6 / 11.4 / 9.5.
+// Evenly spread: 16384 x 1, 8 experts 11.2 / 8.6 / 9.5, 256 experts 19.4 / 8.4 / 9.8; 8192 x 2, 8 experts 11.3 / 8.5 / 9.5.  Outside
+// the line one copy is no slower than three launches however the load lies: collapsed, 4352 x 1 slots (17 chunks) 10.4 / 8.2, 8192 x 2
+// of 128 experts 11.9 / 11.7, 5461 x 3 of 8 experts 11.4 / 9.9, 2048 x 8 of 128 experts 12.6 / 8.2, 16384 x 1 of 1024 21.5 / 18.7.
+constexpr int kCountTable = MOE_MAX_EXPERTS + 16;        // eight copies of up to 129 counts, four of 257, two of 513
+static int direct_copies(int K, int E, int n_chunks) {
+  if (n_chunks <= 24 || !(K == 1 ? E <= 512 : K == 2 && E <= 64)) return 1;
+  return E <= 128 ? 8 : E <= 256 ? 4 : 2;
+}
+
+template <bool SPREAD>
 __global__ __launch_bounds__(kChunk) void permute_direct_kernel(
-    const int32_t *__restrict__ ids, int TK, int E, int n_chunks, int tile_m, int max_tiles,
+    const int32_t *__restrict__ ids, int TK, int E, int copies, int n_chunks, int tile_m, int max_tiles,
     int32_t *__restrict__ sorted_slot, int32_t *__restrict__ expert_offsets, int32_t *__restrict__ slot_to_row,
     int32_t *__restrict__ tile_prefix, int32_t *__restrict__ tile_expert, int32_t *__restrict__ tile_desc,
     uint16_t *__restrict__ zero_rows, int row_len, const QuantJob ride) {
@@ -279,7 +297,8 @@ __global__ __launch_bounds__(kChunk) void permute_direct_kernel(
     int wave_sums[16];
     int wcount[NWV][MOE_MAX_EXPERTS];
   };
-  __shared__ int before[MOE_MAX_EXPERTS], rest[MOE_MAX_EXPERTS];
+  constexpr int kTable = SPREAD ? kCountTable : MOE_MAX_EXPERTS;
+  __shared__ int before[kTable], rest[kTable];
   __shared__ union { Place place; ListSmem lists; } sm;
   // the workgroup of the lists goes first: its chain is the longer one
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = blockIdx.x == 0 ? n_chunks : (int)blockIdx.x - 1;
@@ -289,6 +308,14 @@ __global__ __launch_bounds__(kChunk) void permute_direct_kernel(
     if (c < n_chunks) {
 #pragma unroll
       for (int w = 0; w < NWV; w++) sm.place.wcount[w][e] = 0;
+    }
+  }
+  const int pitch = E | 1;
+  int *const my_before = before + (lane & (copies - 1)) * pitch, *const my_rest = rest + (lane & (copies - 1)) * pitch;
+  if constexpr (SPREAD) {
+    for (int i = E + tid; i < copies * pitch; i += kChunk) {
+      before[i] = 0;
+      rest[i] = 0;
     }
   }
   __syncthreads();
@@ -304,10 +331,25 @@ __global__ __launch_bounds__(kChunk) void permute_direct_kernel(
 #pragma unroll
     for (int i = 0; i < B; i++) {
       if (i0 + i == c) v = id[i];
-      if (id[i] >= 0 && id[i] < E) atomicAdd(i0 + i < c ? &before[id[i]] : &rest[id[i]], 1);
+      if (id[i] >= 0 && id[i] < E) {
+        if constexpr (SPREAD) atomicAdd((i0 + i < c ? my_before : my_rest) + id[i], 1);
+        else atomicAdd(i0 + i < c ? &before[id[i]] : &rest[id[i]], 1);
+      }
     }
   }
   __syncthreads();
+  if constexpr (SPREAD) {
+    for (int e = tid; e < E; e += kChunk) {
+      int b = before[e], r = rest[e];
+      for (int i = 1; i < copies; i++) {
+        b += before[i * pitch + e];
+        r += rest[i * pitch + e];
+      }
+      before[e] = b;
+      rest[e] = r;
+    }
+    __syncthreads();
+  }
   static_assert(MOE_MAX_EXPERTS <= 4 * kChunk, "four experts per thread");
   int first[4], count[4], mine = 0;
 #pragma unroll
@@ -411,9 +453,11 @@ int permute_launch(hipStream_t st, const int32_t *ids, int T, int K, int E, int 
   }
   const QuantJob job = ride ? *ride : QuantJob{};
   if (!counted && TK <= kDirectSlots) {
-    permute_direct_kernel<<<ws.n_chunks + 1 + job.blocks(), kChunk, 0, st>>>(
-        ids, TK, E, ws.n_chunks, tile_m, ws.max_tiles, sorted_slot, expert_offsets, slot_to_row, ws.tile_prefix, ws.tile_expert,
-        ws.tile_desc, zero_rows, row_len, job);
+    const int copies = direct_copies(K, E, ws.n_chunks);
+    const auto kernel = copies > 1 ? permute_direct_kernel<true> : permute_direct_kernel<false>;
+    kernel<<<ws.n_chunks + 1 + job.blocks(), kChunk, 0, st>>>(
+        ids, TK, E, copies, ws.n_chunks, tile_m, ws.max_tiles, sorted_slot, expert_offsets, slot_to_row, ws.tile_prefix,
+        ws.tile_expert, ws.tile_desc, zero_rows, row_len, job);
     return (int)hipGetLastError();
   }
   if (!counted) permute_count_kernel<<<ws.n_chunks, 64, 0, st>>>(ids, TK, E, ws.chunk_counts, ws.arrivals);
