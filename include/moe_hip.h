@@ -273,6 +273,9 @@ size_t moe_mm_fp8_workspace_bytes(int M, int K, int N);
 #define MOE_PLAN_WAVEFRONT      2   /* a wavefront per work item, slices added by a second launch       */
 #define MOE_PLAN_NARROW         3   /* a workgroup per 16 columns, the reduction sliced over its wavefronts */
 int moe_mm_fp8_plan(int M, int K, int N, int *plan);
+/* Output columns of a work item of that plan: 256 or 64 (grouped kernel), 128 (there, two wavefronts to a column group),
+ * 16 (narrow) or a multiple of 16 (wavefront); 0 for a shape that moe_mm_fp8 refuses. */
+int moe_mm_fp8_plan_columns(int M, int K, int N);
 int moe_mm_fp8(void *stream, const void *x_bf16, int M, int K, const uint8_t *w, const float *w_scale, int N,
                void *out_bf16, void *workspace, size_t workspace_bytes);
 /*

@@ -351,3 +351,25 @@ def test_dense_workspace_sizes_of_shapes_that_the_calls_refuse(pkg, M, H, I):
     assert lib.moe_mlp_fp8_workspace_bytes(M, H, I) > 0
     if H % 128 == 0 and I % 16 == 0:
         assert lib.moe_mm_fp8_workspace_bytes(M, H, I) > 0
+
+
+@pytest.mark.parametrize("M,K,N,columns", [
+    # strips of 128 columns, whole and sliced: the shapes whose results the GPU tests of those strips check
+    (300, 7168, 7168, 128), (385, 2176, 7152, 128), (1040, 2048, 2000, 128), (2048, 4096, 2048, 128), (140, 4096, 28672, 128),
+    (1155, 4224, 4096, 128), (400, 7168, 1536, 128), (560, 7296, 1520, 128), (200, 7168, 2112, 128), (600, 8320, 272, 128),
+    # strips of 256 in the other sliced products that they check: 64, 128 and 192 rows, the last slice whole and short
+    (33, 18432, 7168, 256), (64, 16512, 4096, 256), (150, 14336, 4096, 256), (300, 18560, 7168, 256), (1000, 16640, 1040, 256),
+    (128, 18432, 272, 256), (700, 16384, 1040, 256), (129, 18432, 7168, 256), (150, 18560, 4096, 256),
+    # whole products: wide strips, narrow ones of the 64-row tile and of few rows; the kernels of few rows
+    (4001, 7168, 1536, 256), (700, 512, 4096, 256), (600, 7168, 1536, 64), (20, 2048, 28672, 64),
+    (1, 7168, 1536, 16), (64, 7168, 4096, 64),
+])
+def test_plan_says_the_strip_width_of_a_dense_product(pkg, M, K, N, columns):
+    assert pkg.ops.mm_plan_columns(M, K, N) == columns
+
+
+def test_strip_width_of_a_refused_shape_is_an_error(pkg):
+    lib = pkg._lib.lib
+    assert [lib.moe_mm_fp8_plan_columns(*s) for s in ((-1, 128, 16), (5, 100, 16), (5, 128, 17), (5, 32896, 16))] == [0, 0, 0, 0]
+    with pytest.raises(RuntimeError):
+        pkg.ops.mm_plan_columns(5, 100, 16)

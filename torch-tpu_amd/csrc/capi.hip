@@ -656,6 +656,24 @@ extern "C" int moe_mm_fp8_plan(int M, int K, int N, int *plan) {
   return MOE_OK;
 }
 
+extern "C" int moe_mm_fp8_plan_columns(int M, int K, int N) {
+  using namespace moe;
+  int plan[4];
+  if (moe_mm_fp8_plan(M, K, N, plan) != MOE_OK) return 0;
+  if (plan[0] == MOE_PLAN_NARROW) return 16;
+  if (plan[0] == MOE_PLAN_WAVEFRONT) {
+    int splits, len, rows, chunks, tiles;
+    dense_small_plan(M, K, N, &splits, &len, &rows, &chunks, &tiles);
+    return 16 * tiles;
+  }
+  if (plan[0] == MOE_PLAN_GROUPED_SLICED || M > 128) {
+    const DenseSplit sp = dense_split(M, K, N);
+    if (sp.slices > 1 || sp.cols == 128) return sp.cols;
+  }
+  const long wide = (M + plan[1] - 1) / plan[1] * (long)((N + 255) / 256);
+  return plan[1] <= 32 || (plan[1] == 64 && wide <= kNarrowMaxWideItems) ? 64 : 256;
+}
+
 extern "C" int moe_mm_fp8(void *stream, const void *x_bf16, int M, int K, const uint8_t *w, const float *w_scale,
                           int N, void *out_bf16, void *workspace, size_t workspace_bytes) {
   using namespace moe;

@@ -972,7 +972,7 @@ static int launch_gemm(hipStream_t st, GemmArgs &a, int tile_m, int routed_tiles
   // round (a dense 7168 -> 7168 product at 288-384 rows, 140-168 wide items: 64 us in narrow strips, 46 us in wide ones).
   // (a dense layer knows its row tiles; the tile list's entries are an upper bound, a few more than the real ones -
   // Mixtral shape at 48-96 tokens: 9-11 entries for 8 real tiles of 16 strips each - hence the wider margin there)
-  const bool narrow = !GATED && !pair && !a.partial && (km <= 32 || (km == 64 && row_tiles * ((a.N + 255) / 256) < (a.fixed_expert >= 0 ? 129 : 193)));
+  const bool narrow = !GATED && !pair && !a.partial && (km <= 32 || (km == 64 && row_tiles * ((a.N + 255) / 256) <= (a.fixed_expert >= 0 ? kNarrowMaxWideItems : 192)));
   a.n_strips = GATED ? a.N / 128 : pair ? (a.N + 127) / 128 : narrow ? (a.N + 63) / 64 : (a.N + 255) / 256;
   a.max_mtiles = routed_tiles;
   long total = row_tiles * a.n_strips * (a.partial ? a.n_slices : 1);

@@ -94,6 +94,8 @@ static inline int choose_dense_tile_m(long rows, int items_per_row_tile, int ste
 // rows 28.5 / 31.1 -> 23.8 / 27.0, 7168 -> 2112 at 200 / 1100 rows 27.8 / 48.7 -> 22.9 / 40.8, 4096 -> 28672 at 140 rows (192-row
 // tile) 39.6 -> 30.9.  Outside the line: fewer items 4096 -> 4096 at 300 rows (96) 24.8 -> 25.4, 2048 -> 7168 at 200 rows (112)
 // 15.6 -> 16.4; more 7168 -> 1536 at 2800 rows (264) 59.5 -> 78.4; short reductions 512 -> 4096 at 800 rows 10.7 -> 11.6.
+// Row tiles of 64 rows over at most this many strips of 256 columns are worked on in strips of 64 (launch_gemm).
+constexpr int kNarrowMaxWideItems = 128;
 struct DenseSplit {
   int tile_m, slices, k_steps, cols;                     // cols: output columns of a strip, 256 or 128
 };
@@ -104,7 +106,7 @@ static inline DenseSplit dense_split(long rows, int K, int N) {
   double best_cost;
   {
     const long row_tiles = (rows + best.tile_m - 1) / best.tile_m;
-    const bool narrow = best.tile_m == 64 && row_tiles * strips < 129;
+    const bool narrow = best.tile_m == 64 && row_tiles * strips <= kNarrowMaxWideItems;
     const double step = best.tile_m > 64 ? 300.0 + 150.0 * (best.tile_m / 16) : narrow ? 1000.0 : 1500.0;
     best_cost = 0.87 * rounds(row_tiles * strips) * (steps * step + 20000.0);      // a clear win or none
   }

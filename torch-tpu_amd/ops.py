@@ -366,6 +366,13 @@ def mm_plan(M, K, N):
     return ("grouped", "sliced", "wavefront", "narrow")[plan[0]], plan[1], plan[2], plan[3]
 
 
+def mm_plan_columns(M, K, N) -> int:
+    """Output columns of a work item of mm_plan's kernel: 256, 128 or 64 on the grouped kernel, else a multiple of 16."""
+    columns = lib.moe_mm_fp8_plan_columns(M, K, N)
+    _need(columns > 0, "bad dense shape")
+    return columns
+
+
 @functools.lru_cache(maxsize=4096)
 def mlp_workspace_bytes(M, H, I) -> int:
     """Bytes of workspace for mlp_fp8 on up to M rows (kept: the size looks at every smaller batch)."""
