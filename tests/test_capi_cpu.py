@@ -373,3 +373,10 @@ def test_strip_width_of_a_refused_shape_is_an_error(pkg):
     assert [lib.moe_mm_fp8_plan_columns(*s) for s in ((-1, 128, 16), (5, 100, 16), (5, 128, 17), (5, 32896, 16))] == [0, 0, 0, 0]
     with pytest.raises(RuntimeError):
         pkg.ops.mm_plan_columns(5, 100, 16)
+
+
+@pytest.mark.parametrize("M,K,N,rows,columns", [
+    (257, 4096, 6144, 64, 64), (320, 4096, 6144, 64, 64), (321, 4096, 6144, 128, 128), (300, 2048, 6144, 64, 64), (1344, 7168, 1536, 64, 64),
+    (1345, 7168, 1536, 128, 128), (641, 4096, 3072, 128, 128)])
+def test_narrow_strips_of_the_64_row_tile_stay_where_they_measured_faster(pkg, M, K, N, rows, columns):
+    assert pkg.ops.mm_plan(M, K, N)[:2] == ("grouped", rows) and pkg.ops.mm_plan_columns(M, K, N) == columns

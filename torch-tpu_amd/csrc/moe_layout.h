@@ -86,8 +86,10 @@ static inline int choose_dense_tile_m(long rows, int items_per_row_tile, int ste
 // rows, 2.3 TB/s of weights), 4096 / 14336 at 129 / 300 / 600 rows 99 / 107 / 167 -> 71 / 85 / 146 us.
 //
 // Strips of 128 columns (paired wavefronts, more than 128 rows and 256 columns) are twice the work items, each with a step of
-// about 1100 cycles under 128 rows.  Whole, they take a layer whose narrow items are more than half a round and no more than one: the
-// wide 64-row tiles that it gets otherwise are one round of 1500-cycle steps.  192 rows likewise, where 128 are too many
+// about 1100 cycles under 128 rows.  Whole, they take a layer of which they are more than half a round and no more than one: the wide
+// 64-row tiles that it gets otherwise are one round of 1500-cycle steps.  (Not where that tile is worked on in strips of 64:
+// those against these, 4096 -> 6144 at 257 / 320 / 321 rows 24.6 / 25.3 / 30.2 and 25.6 / 26.2 / 26.3 us, wide from 321 rows on, 2048 ->
+// 6144 at 257 / 320 rows 15.2 / 15.8 and 16.7 / 16.9, 7168 -> 1536 at 1281 / 1344 / 1345 rows 40.8 / 41.1 / 49.4 and 42.1 / 42.0 / 42.2.)  192 rows likewise, where 128 are too many
 // items.  Sliced, they compete by the model, which lets a layer of few strips have them.  Measured, whole op, before ->
 // after in us: 7168 -> 1536 at 400 / 560 / 1500 / 2000 rows 28.6 / 35.3 / 50.6 / 53.6 -> 24.9 / 26.0 / 41.6 / 44.2, 7168 -> 7168 at
 // 300 / 400 rows 46.3 / 48.0 -> 38.1 / 39.5, 4096 -> 4096 at 560 / 800 rows 30.3 / 31.5 -> 27.2 / 28.9, 16384 -> 1024 at 140 / 400
@@ -104,9 +106,9 @@ static inline DenseSplit dense_split(long rows, int K, int N) {
   DenseSplit best = {choose_dense_tile_m(rows, strips, steps), 1, steps, 256};
   const auto rounds = [](long items) { return (double)((items + 255) / 256); };
   double best_cost;
+  const long row_tiles = (rows + best.tile_m - 1) / best.tile_m;
+  const bool narrow = best.tile_m == 64 && row_tiles * strips <= kNarrowMaxWideItems;
   {
-    const long row_tiles = (rows + best.tile_m - 1) / best.tile_m;
-    const bool narrow = best.tile_m == 64 && row_tiles * strips <= kNarrowMaxWideItems;
     const double step = best.tile_m > 64 ? 300.0 + 150.0 * (best.tile_m / 16) : narrow ? 1000.0 : 1500.0;
     best_cost = 0.87 * rounds(row_tiles * strips) * (steps * step + 20000.0);      // a clear win or none
   }
@@ -123,7 +125,7 @@ static inline DenseSplit dense_split(long rows, int K, int N) {
   if (rows <= 128 || N <= 256) return best;
   const int pair_strips = (N + 127) / 128;
   const long pair128 = (rows + 127) / 128 * (long)pair_strips, pair192 = (rows + 191) / 192 * (long)pair_strips;
-  if (best.slices == 1) {
+  if (best.slices == 1 && !narrow) {
     if (steps >= 16 && pair128 > 128 && pair128 <= 256) best = {128, 1, steps, 128};
     else if (steps >= 32 && pair128 > 256 && pair192 > 128 && pair192 <= 224) best = {192, 1, steps, 128};
   }
