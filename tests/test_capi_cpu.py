@@ -356,7 +356,7 @@ def test_dense_workspace_sizes_of_shapes_that_the_calls_refuse(pkg, M, H, I):
 @pytest.mark.parametrize("M,K,N,columns", [
     # strips of 128 columns, whole and sliced: the shapes whose results the GPU tests of those strips check
     (300, 7168, 7168, 128), (385, 2176, 7152, 128), (1040, 2048, 2000, 128), (2048, 4096, 2048, 128), (140, 4096, 28672, 128),
-    (1155, 4224, 4096, 128), (400, 7168, 1536, 128), (560, 7296, 1520, 128), (200, 7168, 2112, 128), (600, 8320, 272, 128),
+    (155, 4224, 28672, 128), (400, 7168, 1536, 128), (560, 7296, 1520, 128), (200, 7168, 2112, 128), (600, 8320, 272, 128),
     # strips of 256 in the other sliced products that they check: 64, 128 and 192 rows, the last slice whole and short
     (33, 18432, 7168, 256), (64, 16512, 4096, 256), (150, 14336, 4096, 256), (300, 18560, 7168, 256), (1000, 16640, 1040, 256),
     (128, 18432, 272, 256), (700, 16384, 1040, 256), (129, 18432, 7168, 256), (150, 18560, 4096, 256),
@@ -379,4 +379,12 @@ def test_strip_width_of_a_refused_shape_is_an_error(pkg):
     (257, 4096, 6144, 64, 64), (320, 4096, 6144, 64, 64), (321, 4096, 6144, 128, 128), (300, 2048, 6144, 64, 64), (1344, 7168, 1536, 64, 64),
     (1345, 7168, 1536, 128, 128), (641, 4096, 3072, 128, 128)])
 def test_narrow_strips_of_the_64_row_tile_stay_where_they_measured_faster(pkg, M, K, N, rows, columns):
+    assert pkg.ops.mm_plan(M, K, N)[:2] == ("grouped", rows) and pkg.ops.mm_plan_columns(M, K, N) == columns
+
+
+@pytest.mark.parametrize("M,K,N,rows,columns", [
+    (129, 4096, 22528, 192, 128), (192, 4096, 32768, 192, 128), (192, 4992, 28672, 192, 128), (193, 4096, 28672, 128, 256),
+    (150, 4096, 22400, 128, 256), (150, 4096, 32784, 192, 256), (150, 5120, 28672, 128, 256), (150, 3968, 28672, 128, 256),
+    (1025, 4096, 4096, 128, 256), (1200, 4096, 4096, 128, 256), (3300, 7168, 1536, 128, 256), (513, 7168, 7168, 64, 256), (768, 18432, 7168, 128, 256)])
+def test_tall_strips_of_128_columns_take_one_row_tile(pkg, M, K, N, rows, columns):
     assert pkg.ops.mm_plan(M, K, N)[:2] == ("grouped", rows) and pkg.ops.mm_plan_columns(M, K, N) == columns

@@ -89,13 +89,24 @@ static inline int choose_dense_tile_m(long rows, int items_per_row_tile, int ste
 // about 1100 cycles under 128 rows.  Whole, they take a layer of which they are more than half a round and no more than one: the wide
 // 64-row tiles that it gets otherwise are one round of 1500-cycle steps.  (Not where that tile is worked on in strips of 64:
 // those against these, 4096 -> 6144 at 257 / 320 / 321 rows 24.6 / 25.3 / 30.2 and 25.6 / 26.2 / 26.3 us, wide from 321 rows on, 2048 ->
-// 6144 at 257 / 320 rows 15.2 / 15.8 and 16.7 / 16.9, 7168 -> 1536 at 1281 / 1344 / 1345 rows 40.8 / 41.1 / 49.4 and 42.1 / 42.0 / 42.2.)  192 rows likewise, where 128 are too many
-// items.  Sliced, they compete by the model, which lets a layer of few strips have them.  Measured, whole op, before ->
+// 6144 at 257 / 320 rows 15.2 / 15.8 and 16.7 / 16.9, 7168 -> 1536 at 1281 / 1344 / 1345 rows 40.8 / 41.1 / 49.4 and 42.1 / 42.0 / 42.2.)  Sliced,
+// they compete by the model, which lets a layer of few strips have them.  Measured, whole op, before ->
 // after in us: 7168 -> 1536 at 400 / 560 / 1500 / 2000 rows 28.6 / 35.3 / 50.6 / 53.6 -> 24.9 / 26.0 / 41.6 / 44.2, 7168 -> 7168 at
 // 300 / 400 rows 46.3 / 48.0 -> 38.1 / 39.5, 4096 -> 4096 at 560 / 800 rows 30.3 / 31.5 -> 27.2 / 28.9, 16384 -> 1024 at 140 / 400
-// rows 28.5 / 31.1 -> 23.8 / 27.0, 7168 -> 2112 at 200 / 1100 rows 27.8 / 48.7 -> 22.9 / 40.8, 4096 -> 28672 at 140 rows (192-row
-// tile) 39.6 -> 30.9.  Outside the line: fewer items 4096 -> 4096 at 300 rows (96) 24.8 -> 25.4, 2048 -> 7168 at 200 rows (112)
-// 15.6 -> 16.4; more 7168 -> 1536 at 2800 rows (264) 59.5 -> 78.4; short reductions 512 -> 4096 at 800 rows 10.7 -> 11.6.
+// rows 28.5 / 31.1 -> 23.8 / 27.0, 7168 -> 2112 at 200 / 1100 rows 27.8 / 48.7 -> 22.9 / 40.8.  Outside the line: fewer items
+// 4096 -> 4096 at 300 rows (96) 24.8 -> 25.4, 2048 -> 7168 at 200 rows (112) 15.6 -> 16.4; more 7168 -> 1536 at 2800 rows (264: two
+// rounds) 59.5 -> 78.4; short reductions 512 -> 4096 at 800 rows 10.7 -> 11.6.
+//
+// 192 rows of 128 columns take wide layers of 129 to 192 rows: one row tile instead of two of 128 rows that each load the
+// weights.  Wide / these strips in us, the weights in the caches and (in brackets) rotated through 500 MB: 4096 -> 22528 at 129 / 192
+// rows 34.2 (34.8) / 32.3 (36.8) and 28.2 (33.7) / 31.4 (36.1), 4096 -> 28672 40.0 (36.7) / 35.6 (39.2) and 29.0 (35.3) / 33.5 (38.4), 4096 ->
+// 32768 (256 strips, the whole round) 44.5 (38.4) / 38.5 (40.9) and 31.3 (36.3) / 35.3 (40.5).  Outside the line they lose where the
+// weights come from memory: fewer strips 4096 -> 18432 at 129 / 192 rows (31.9) / (34.0) and (32.1) / (34.7), longer reductions 5120 ->
+// 24576 (42.9) / (45.7) and (44.3) / (46.6), 7168 -> 24576 (53.3) / (58.0) and (54.7) / (59.0), 12288 -> 28672 94.0 / 100.5 and 97.3 / 102.8; and several row
+// tiles are no gain: 4096 -> 4096 at 1025 / 1200 rows 34.1 / 35.0 and 33.7 / 35.7, 14336 -> 4096 90.9 / 94.4 and 89.0 / 97.6, 7168 -> 1536 at
+// 2800 / 3300 rows 55.7 / 57.6 and 55.5 / 59.1, 7168 -> 7168 at 576 / 768 rows 49.1 / 51.0 and 49.4 / 52.8.  Shorter reductions lose with
+// the weights in memory as well, 3968 -> 28672 (39.7) / (40.6) and (40.2) / (41.6), 3072 -> 28672 (30.4) / (32.3) and (31.1) / (32.9), until 2048, which
+// the line leaves out: 2048 -> 28672 23.7 (23.2) / 22.4 (24.4) and 19.8 (22.2) / 22.0 (24.5).
 // Row tiles of 64 rows over at most this many strips of 256 columns are worked on in strips of 64 (launch_gemm).
 constexpr int kNarrowMaxWideItems = 128;
 struct DenseSplit {
@@ -124,12 +135,15 @@ static inline DenseSplit dense_split(long rows, int K, int N) {
   }
   if (rows <= 128 || N <= 256) return best;
   const int pair_strips = (N + 127) / 128;
-  const long pair128 = (rows + 127) / 128 * (long)pair_strips, pair192 = (rows + 191) / 192 * (long)pair_strips;
+  const long pair128 = (rows + 127) / 128 * (long)pair_strips;
   if (best.slices == 1 && !narrow) {
     if (steps >= 16 && pair128 > 128 && pair128 <= 256) best = {128, 1, steps, 128};
-    else if (steps >= 32 && pair128 > 256 && pair192 > 128 && pair192 <= 224) best = {192, 1, steps, 128};
+    else if (rows <= 192 && steps >= 32 && steps < 40 && pair_strips >= 176 && pair_strips <= 256) best = {192, 1, steps, 128};
   }
-  best_cost *= 0.94;                                     // (where the model sees less, the two measure the same)
+  // Slices of narrow strips have to be 6 % better by the model.  Where it sees less, wide / narrow measure in us: 14336 -> 4096 at
+  // 228 / 256 rows 33.7 / 34.7 and 35.1 / 35.3, 16384 -> 1024 at 700 / 850 / 1280 rows 34.6 / 37.5 / 48.7 and 35.1 / 37.2 / 49.3.  (7168 -> 1536
+  // at 593 to 640 rows falls on the wrong side of it: 35.6 whole, 25.8 in slices of narrow strips.)
+  best_cost *= 0.94;
   for (int len = 16; len < steps; len += 16) {
     const int slices = (steps + len - 1) / len;
     const double cost = rounds(pair128 * slices) * (len * 1100.0 + 20000.0) + 10000.0 + 8.0 * slices * (double)rows * N / 2000.0;
