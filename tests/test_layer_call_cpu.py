@@ -1,0 +1,51 @@
+"""ops.layer_fp8's argument handling where no GPU is: the library's entry point is replaced by one that records its arguments,
+so that a call that the wrapper accepts completes, and one that it refuses raises what it raises with a GPU."""
+import ctypes
+
+import pytest
+import torch
+
+T, H, I, E, K = 3, 256, 128, 4, 2
+
+
+class Lib:
+    def __init__(self, real):
+        self.real, self.calls = real, []
+        kind = ctypes.CFUNCTYPE(ctypes.c_int, *real.moe_layer_fp8.argtypes)
+        self.moe_layer_fp8 = kind(lambda *args: (self.calls.append(args), 0)[1])
+
+    def __getattr__(self, name):
+        return getattr(self.real, name)
+
+
+@pytest.fixture
+def road(pkg, monkeypatch):
+    """(layer call, calls that reached the library)"""
+    ops = pkg.ops
+    lib = Lib(ops.lib)
+
+    def address(t, name, dtype=None):
+        assert isinstance(t, torch.Tensor) and t.is_contiguous() and (dtype is None or t.dtype == dtype), name
+        return t.data_ptr()
+
+    monkeypatch.setattr(ops, "lib", lib)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_dev", address)
+    fp8 = torch.float8_e4m3fn
+    given = dict(x=torch.zeros(T, H, dtype=torch.bfloat16), router_weight=torch.zeros(E, H, dtype=torch.bfloat16),
+                 w13=torch.zeros(E, 2 * I, H, dtype=fp8), w13_scale=torch.ones(E, 2 * I // 128, H // 128),
+                 w2=torch.zeros(E, H, I, dtype=fp8), w2_scale=torch.ones(E, H // 128, I // 128), top_k=K,
+                 workspace=torch.empty(1 << 16, dtype=torch.uint8))
+    return lambda **more: ops.layer_fp8(**{**given, **more}), lib.calls
+
+
+def test_plain_call(road):
+    call, calls = road
+    assert call().shape == (T, H) and len(calls) == 1
+
+
+def test_layer_call_under_the_jit_tracer(road):
+    """A tracer records operators: one with a number as its result is not for it to see."""
+    call, calls = road
+    traced = torch.jit.trace(lambda x: call(x=x), (torch.zeros(T, H, dtype=torch.bfloat16),), check_trace=False)
+    assert len(calls) == 1 and "_layer_fp8" not in str(traced.graph)

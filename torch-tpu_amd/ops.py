@@ -295,8 +295,10 @@ def layer_fp8(x, router_weight, w13, w13_scale, w2, w2_scale, top_k: int, mode: 
     device allocation when `out` is given; small batches only, calls on one GPU must not overlap)."""
     modes = _LAYER_MODES
     _need(mode in modes, f"unknown routing mode {mode!r}")
-    # The common form natively; any other, and what is wrong with one, below.  A tracer sees the calls below, as ever.
-    if workspace is not None and not (return_routing or static_scratch) and not torch.compiler.is_compiling():
+    # The common form natively; any other, and what is wrong with one, below.  So is a call that Dynamo, export or the JIT's
+    # tracer looks at: none of them can take an operator whose result is a status.
+    if (workspace is not None and not (return_routing or static_scratch) and not torch.compiler.is_compiling()
+            and not torch.jit.is_tracing()):
         result = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if out is None else out
         sh = (None, None, None, None) if shared is None else shared
         rc = torch.ops.my_ops._layer_fp8.default(x, router_weight, w13, w13_scale, w2, w2_scale, top_k, modes[mode], bias, n_groups,
