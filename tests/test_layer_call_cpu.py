@@ -49,3 +49,19 @@ def test_layer_call_under_the_jit_tracer(road):
     call, calls = road
     traced = torch.jit.trace(lambda x: call(x=x), (torch.zeros(T, H, dtype=torch.bfloat16),), check_trace=False)
     assert len(calls) == 1 and "_layer_fp8" not in str(traced.graph)
+
+
+class Picky(torch.Tensor):
+    """A subclass that declines operators that it does not know."""
+    @classmethod
+    def __torch_function__(cls, func, types, args=(), kwargs=None):
+        return NotImplemented if "my_ops" in str(func) else super().__torch_function__(func, types, args, kwargs or {})
+
+
+@pytest.mark.parametrize("which", ["x", "w13_scale", "bias", "out"])
+def test_operands_of_a_tensor_subclass(road, which):
+    call, calls = road
+    t = {"x": torch.zeros(T, H, dtype=torch.bfloat16), "w13_scale": torch.ones(E, 2 * I // 128, H // 128), "bias": torch.zeros(E),
+         "out": torch.zeros(T, H, dtype=torch.bfloat16)}[which].as_subclass(Picky)
+    call(**{which: t})
+    assert len(calls) == 1

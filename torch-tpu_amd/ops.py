@@ -284,6 +284,12 @@ _LAYER_MODES = {"softmax": ROUTE_SOFTMAX, "sigmoid": ROUTE_SIGMOID, "softmax_log
 _NOT_PLAIN = 1 << 20     # my_ops::_layer_fp8: not the form that it takes
 
 
+def _plain(*operands) -> bool:
+    """No operand is of a Tensor subclass, which may have its own idea of operators (a mode, e.g. a default device, is fine)."""
+    return (not torch.overrides.has_torch_function(operands)
+            or all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in operands))
+
+
 def layer_fp8(x, router_weight, w13, w13_scale, w2, w2_scale, top_k: int, mode: str = "softmax", bias=None,
                      n_groups: int = 1, topk_groups: int = 1, renorm: bool = True, scale: float = 1.0, shared=None,
                      out=None, workspace=None, return_routing: bool = False, static_scratch: bool = False):
@@ -301,8 +307,10 @@ def layer_fp8(x, router_weight, w13, w13_scale, w2, w2_scale, top_k: int, mode: 
             and not torch.jit.is_tracing()):
         result = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if out is None else out
         sh = (None, None, None, None) if shared is None else shared
-        rc = torch.ops.my_ops._layer_fp8.default(x, router_weight, w13, w13_scale, w2, w2_scale, top_k, modes[mode], bias, n_groups,
-                                                 topk_groups, bool(renorm), float(scale), *sh, result, workspace)
+        rc = _NOT_PLAIN
+        if _plain(x, router_weight, w13, w13_scale, w2, w2_scale, bias, *sh, result, workspace):
+            rc = torch.ops.my_ops._layer_fp8.default(x, router_weight, w13, w13_scale, w2, w2_scale, top_k, modes[mode], bias, n_groups,
+                                                     topk_groups, bool(renorm), float(scale), *sh, result, workspace)
         if rc != _NOT_PLAIN:
             check(rc, "layer_fp8")
             return result
