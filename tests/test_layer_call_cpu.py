@@ -65,3 +65,25 @@ def test_operands_of_a_tensor_subclass(road, which):
          "out": torch.zeros(T, H, dtype=torch.bfloat16)}[which].as_subclass(Picky)
     call(**{which: t})
     assert len(calls) == 1
+
+
+@pytest.mark.parametrize("renorm", [None, "x", [1]])
+def test_renorm_that_is_no_number_is_refused(road, renorm):
+    call, calls = road
+    with pytest.raises((TypeError, ValueError)):
+        call(renorm=renorm)
+    assert not calls
+
+
+def test_native_road_takes_renorm_as_the_other_does(road, monkeypatch):
+    """A whole number's truth: 0.5 is 0, as the C argument has it."""
+    call, calls = road
+    seen = []
+
+    class Op:
+        default = staticmethod(lambda *args: (seen.append(args[11]), 1 << 20)[1])
+
+    monkeypatch.setattr(torch.ops.my_ops, "_layer_fp8", Op)
+    for renorm in (True, False, 2, 0, 0.5, 1.5):
+        call(renorm=renorm)
+    assert seen == [bool(args[11]) for args in calls] == [True, False, True, False, False, True]

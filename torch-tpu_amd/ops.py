@@ -310,7 +310,7 @@ def layer_fp8(x, router_weight, w13, w13_scale, w2, w2_scale, top_k: int, mode: 
         rc = _NOT_PLAIN
         if _plain(x, router_weight, w13, w13_scale, w2, w2_scale, bias, *sh, result, workspace):
             rc = torch.ops.my_ops._layer_fp8.default(x, router_weight, w13, w13_scale, w2, w2_scale, top_k, modes[mode], bias, n_groups,
-                                                     topk_groups, bool(renorm), float(scale), *sh, result, workspace)
+                                                     topk_groups, bool(int(renorm)), float(scale), *sh, result, workspace)
         if rc != _NOT_PLAIN:
             check(rc, "layer_fp8")
             return result
