@@ -87,3 +87,13 @@ def test_native_road_takes_renorm_as_the_other_does(road, monkeypatch):
     for renorm in (True, False, 2, 0, 0.5, 1.5):
         call(renorm=renorm)
     assert seen == [bool(args[11]) for args in calls] == [True, False, True, False, False, True]
+
+
+@pytest.mark.parametrize("size", ["layer_workspace_bytes", "mm_workspace_bytes", "mlp_workspace_bytes"])
+def test_sizes_asked_for_before_do_not_answer_other_types(pkg, size):
+    """The sizes are kept by their arguments: 4.0 is refused, also once the size of 4 is known."""
+    fn = getattr(pkg.ops, size)
+    args = (4, 256, 128, 8, 2) if size.startswith("layer") else (4, 256, 128)
+    assert fn(*args) > 0
+    with pytest.raises(ctypes.ArgumentError):
+        fn(float(args[0]), *args[1:])

@@ -275,7 +275,7 @@ def router_logits(x, router_weight, out=None, workspace=None):
     return out
 
 
-@functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=4096, typed=True)
 def layer_workspace_bytes(T, H, I, E, K, I_shared=0) -> int:
     return lib.moe_layer_fp8_workspace_bytes(T, H, I, E, K, I_shared)
 
@@ -362,7 +362,7 @@ def fused_experts_bf16_workspace_bytes(T, H, I, E, K) -> int:
     return lib.moe_fused_experts_bf16_workspace_bytes(T, H, I, E, K)
 
 
-@functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=4096, typed=True)
 def mm_workspace_bytes(M, K, N) -> int:
     """Bytes of workspace for mm_fp8 on up to M rows (kept: the size looks at every smaller batch)."""
     return lib.moe_mm_fp8_workspace_bytes(M, K, N)
@@ -383,7 +383,7 @@ def mm_plan_columns(M, K, N) -> int:
     return columns
 
 
-@functools.lru_cache(maxsize=4096)
+@functools.lru_cache(maxsize=4096, typed=True)
 def mlp_workspace_bytes(M, H, I) -> int:
     """Bytes of workspace for mlp_fp8 on up to M rows (kept: the size looks at every smaller batch)."""
     return lib.moe_mlp_fp8_workspace_bytes(M, H, I)
