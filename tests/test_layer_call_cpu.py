@@ -97,3 +97,8 @@ def test_sizes_asked_for_before_do_not_answer_other_types(pkg, size):
     assert fn(*args) > 0
     with pytest.raises(ctypes.ArgumentError):
         fn(float(args[0]), *args[1:])
+
+
+def test_native_layer_call_declares_what_it_writes(pkg):
+    schema = torch.ops.my_ops._layer_fp8.default._schema
+    assert [a.name for a in schema.arguments if a.alias_info is not None and a.alias_info.is_write] == ["out", "workspace"]

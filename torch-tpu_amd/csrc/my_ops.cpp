@@ -729,7 +729,9 @@ TORCH_LIBRARY(my_ops, m) {
   m.def("_mm_weights(Tensor weight, Tensor scale) -> Tensor[]");
   m.def("_mlp_weights(Tensor gate_weight, Tensor up_weight, Tensor down_weight, Tensor gate_scale, Tensor up_scale, "
         "Tensor down_scale) -> Tensor[]");
-  m.def("_layer_fp8", _layer_fp8);
+  m.def("_layer_fp8(Tensor x, Tensor router_weight, Tensor w13, Tensor w13_scale, Tensor w2, Tensor w2_scale, int top_k, int mode, "
+        "Tensor? bias, int n_groups, int topk_groups, bool renorm, float scale, Tensor? shared_w13, Tensor? shared_w13_scale, "
+        "Tensor? shared_w2, Tensor? shared_w2_scale, Tensor(a!) out, Tensor(b!) workspace) -> int", _layer_fp8);
   m.def("_packed_weight_sets", _packed_weight_sets);
   m.def("_packed_weight_bytes", _packed_weight_bytes);
 }
