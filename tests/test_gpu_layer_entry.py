@@ -547,3 +547,53 @@ def test_layer_entry_native_road_and_the_other_agree(pkg, dev, T, odd):
         assert got is kw["out"]
     with pytest.raises(RuntimeError):
         pkg.layer_fp8(x, wr, *w13, *w2, K, workspace=ws[:ws.numel() - 1], **{k: v for k, v in kw.items() if k != "out"})
+
+
+@pytest.mark.parametrize("form,native", [("none", True), ("out", True), ("bias", True), ("shared", True), ("parameter", True),
+                                         ("workspace of words", False), ("strided out", False), ("bias of one row", False),
+                                         ("bf16 scales", False), ("host x", False), ("traced", False)])
+def test_which_layer_calls_are_native(pkg, dev, monkeypatch, form, native):
+    """The common forms don't reach the Python road's call of the library, the others do not get past the native checks."""
+    T, E, H, I, K = 40, 16, 256, 256, 2
+    w13, w2 = pkg.synthetic_weights(E, 2 * I, H, dev, 1), pkg.synthetic_weights(E, H, I, dev, 2)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
+    wr = (torch.randn(E, H, generator=g) * 0.1).to(torch.bfloat16).to(dev)
+    sh = (*pkg.synthetic_weights(1, 2 * I, H, dev, 3), *pkg.synthetic_weights(1, H, I, dev, 4)) if form == "shared" else (None,) * 4
+    ws = torch.empty(pkg.layer_workspace_bytes(T, H, I, E, K, I if form == "shared" else 0), dtype=torch.uint8, device=dev)
+    out, bias, s13 = torch.empty(T, H, dtype=torch.bfloat16, device=dev), None, w13[1]
+    if form.startswith("bias"):
+        bias = torch.randn(E, generator=g).to(dev).view((1, E) if form == "bias of one row" else (E,))
+    if form == "parameter":
+        wr = torch.nn.Parameter(wr)
+    if form == "workspace of words":
+        ws = ws[:ws.numel() // 4 * 4].view(torch.int32)
+    if form == "strided out":
+        out = torch.empty(T, 2 * H, dtype=torch.bfloat16, device=dev)[:, ::2]
+    if form == "bf16 scales":
+        s13 = s13.to(torch.bfloat16)
+    if form == "host x":
+        x = x.cpu()
+    if form != "traced":
+        rc = torch.ops.my_ops._layer_fp8.default(x, wr, w13[0], s13, *w2, K, 1, bias, 1, 1, True, 1.0, *sh, out, ws)
+        assert rc == (0 if native else 1 << 20)
+
+    class Lib:
+        calls = 0
+
+        def __getattr__(self, name):
+            Lib.calls += name == "moe_layer_fp8"
+            return getattr(real, name)
+
+    real = pkg.ops.lib
+    monkeypatch.setattr(pkg.ops, "lib", Lib())
+    call = lambda t: pkg.layer_fp8(t, wr, w13[0], s13, *w2, K, mode="sigmoid", bias=bias, workspace=ws,
+                                   shared=sh if form == "shared" else None, out=out if "out" in form else None)
+    if form in ("strided out", "bf16 scales", "host x"):
+        with pytest.raises(RuntimeError):
+            call(x)
+        return
+    got = torch.jit.trace(call, (x,), check_trace=False)(x) if form == "traced" else call(x)
+    assert (Lib.calls == 0) == native
+    if native and form != "out":
+        assert torch.equal(got, out)
