@@ -798,6 +798,11 @@ __global__ __launch_bounds__(64 * NW, (WREG && NW == 4) ? 2 : 1) void grouped_ge
         for (int r = 0; r < 4; r++) acc[0][j][r] = fmaf(p[1][j][r], f, acc[0][j][r]);
       }
     };
+    // PAIR: the wavefronts of a pair may walk different numbers of m-tiles, so wavefronts of one workgroup run different
+    // bodies and meet at different barriers of the text.  The hardware counts arrivals, which makes that sound as long as
+    // every body has the same barriers before its loop and in each step, asks for the same loads in the same order in a step
+    // and takes as many steps - the same ring, that is.  (In all other instantiations the choice is the workgroup's.)
+    static_assert(!PAIR || RING == 2, "wavefronts of a workgroup in different bodies: one ring for all");
     auto pick = [&](auto self, auto live_c, auto ring_c) -> void {
       constexpr int LIVE = decltype(live_c)::value;
       if constexpr (LIVE >= MTW) run(std::integral_constant<int, MTW>{}, ring_c);
