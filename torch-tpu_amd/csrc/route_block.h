@@ -134,9 +134,16 @@ __device__ __forceinline__ void route_block(RouteBlockSmem &sm, const void *logi
   const uint64_t mine = sm.cand[e];
   if (mine != 0) {
     int r = 0;
-    for (int j0 = 0; j0 < n_cand; j0 += 16) {             // (0 beyond the candidates: whole batches of reads)
+    // sixteen at a time (0 beyond the candidates), all reads before the first comparison: left to itself the compiler
+    // waits for every read in turn in some of the kernels
+#pragma unroll 1
+    for (int j0 = 0; j0 < n_cand; j0 += 16) {
+      uint64_t other[16];
 #pragma unroll
-      for (int j = 0; j < 16; j++) r += sm.cand[j0 + j] > mine;
+      for (int j = 0; j < 16; j++) other[j] = sm.cand[j0 + j];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < 16; j++) r += other[j] > mine;
     }
     if (r < K) {
       const int who = 0x7fffffff - (int)(uint32_t)mine;
