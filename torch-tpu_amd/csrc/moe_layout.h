@@ -7,7 +7,12 @@
 namespace moe {
 
 constexpr int kChunk = 256;   // slots ranked by one workgroup in the permutation kernels
-// Slots up to which the permutation is one launch that counts every id itself (permute_direct_kernel).
+// Slots up to which the permutation is one launch that counts every id itself (permute_direct_kernel).  Three launches / one, in
+// us, 20480 / 24576 / 32768 / 65536 / 131072 slots: 8 picks of 128 experts 12.0 / 12.3 / 12.6 / 14.1 / 16.8 and 9.4 / 10.5 / 12.7 / 23.0 / 49.6; at
+// 32768 slots 8 picks of 256 / 1024 experts 14.2 / 26.2 and 12.8 / 15.3, 2 of 8 10.4 and 14.4.  In a layer, where the first of the three
+// rides in the routing launch: 128 experts of 2048 x 768 at 20480 / 24576 / 32768 / 131072 slots 260.8 / 282.0 / 342.9 / 940 and 259.7 / 281.1 /
+// 344.8 / 961, 256 of 1024 x 256 at 32768 144.8 and 149.1, 8 of 256 x 128 at 20480 55.0 and 50.1.  So one launch is the better form up to
+// 24576 slots at least and the worse one from 32768 on in most layers; the line stays below both.
 constexpr int kDirectSlots = 64 * kChunk;
 
 // What the grouped GEMMs multiply: FP8 activations x FP8 weights with scales (the path proper), bf16 x bf16
@@ -93,7 +98,8 @@ static inline int choose_dense_tile_m(long rows, int items_per_row_tile, int ste
 // they compete by the model, which lets a layer of few strips have them.  Measured, whole op, before ->
 // after in us: 7168 -> 1536 at 400 / 560 / 1500 / 2000 rows 28.6 / 35.3 / 50.6 / 53.6 -> 24.9 / 26.0 / 41.6 / 44.2, 7168 -> 7168 at
 // 300 / 400 rows 46.3 / 48.0 -> 38.1 / 39.5, 4096 -> 4096 at 560 / 800 rows 30.3 / 31.5 -> 27.2 / 28.9, 16384 -> 1024 at 140 / 400
-// rows 28.5 / 31.1 -> 23.8 / 27.0, 7168 -> 2112 at 200 / 1100 rows 27.8 / 48.7 -> 22.9 / 40.8.  Outside the line: fewer items
+// rows 28.5 / 31.1 -> 23.8 / 27.0, 7168 -> 2112 at 200 / 1100 rows 27.8 / 48.7 -> 22.9 / 40.8; as the second product of a gated MLP
+// 7168 / 2048 at 257 / 400 / 512 rows (the whole MLP) 64.0 / 65.3 / 65.9 -> 62.5 / 63.6 / 63.9.  Outside the line: fewer items
 // 4096 -> 4096 at 300 rows (96) 24.8 -> 25.4, 2048 -> 7168 at 200 rows (112) 15.6 -> 16.4; more 7168 -> 1536 at 2800 rows (264: two
 // rounds) 59.5 -> 78.4; short reductions 512 -> 4096 at 800 rows 10.7 -> 11.6.
 //
