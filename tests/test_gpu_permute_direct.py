@@ -63,7 +63,7 @@ def test_one_hot_expert_and_empty_ones_reach_the_gemms(pkg, oracle, dev, T):
 
 # one and two picks, chunks on either side of the line from which counts are kept in copies, experts at the edges of 8, 4, 2 and 1
 @pytest.mark.parametrize("T,K,E", [(6144, 1, 8), (6145, 1, 8), (DIRECT_SLOTS, 1, 1), (DIRECT_SLOTS, 1, 128), (DIRECT_SLOTS, 1, 129), (16001, 1, 256),
-                                   (DIRECT_SLOTS, 1, 257), (DIRECT_SLOTS, 1, 512), (12345, 1, 513), (DIRECT_SLOTS // 2, 2, 2), (8111, 2, 64),
+                                   (DIRECT_SLOTS, 1, 257), (DIRECT_SLOTS, 1, 512), (12345, 1, 513), (DIRECT_SLOTS // 2, 2, 2), (8111, 2, 64), (6144, 2, 8), (6145, 2, 8),
                                    (DIRECT_SLOTS // 2, 2, 65)])
 @pytest.mark.parametrize("load", ["even", "collapsed", "half outside"])
 def test_counts_kept_in_copies_add_up(pkg, dev, T, K, E, load):

@@ -267,25 +267,26 @@ __global__ __launch_bounds__(kChunk) void permute_scatter_kernel(const int32_t *
 // 55.1, Mixtral shape at 256 tokens 326 -> 318, 8 experts of 256 x 512 at 516 tokens 46.2 -> 38.8.
 // Reading everything grows with the square of the chunks: above kDirectSlots the three kernels take over.
 //
-// SPREAD: lanes that add to one counter wait for one another, and a wavefront whose 64 slots all ask for one expert takes
+// COPIES: lanes that add to one counter wait for one another, and a wavefront whose 64 slots all ask for one expert takes
 // about ten times as long to count as one whose slots differ.  The experts of a token are distinct, so K picks put at most
 // 64 / K slots of a wavefront on one expert.  For one pick, and for two among few experts, a load that collapsed made the
-// launch as slow as the three that it replaces from 30 chunks on, and slower above.  From there the counts are kept in several
-// copies, neighbouring lanes adding to different ones (at an odd pitch: the copies of a counter sit in different banks), which
-// are added up afterwards.  Three launches / one copy / copies in us, every slot on the first K experts: 16384 x 1 slots, 8
-// experts 10.5 / 18.0 / 9.5, 256 experts 12.6 / 18.2 / 10.1, 512 experts 14.7 / 18.5 / 12.8; 8192 x 2, 8 experts 10.6 / 11.4 / 9.5.
-// Evenly spread: 16384 x 1, 8 experts 11.2 / 8.6 / 9.5, 256 experts 19.4 / 8.4 / 9.8; 8192 x 2, 8 experts 11.3 / 8.5 / 9.5.  Outside
-// the line one copy is no slower than three launches however the load lies: collapsed, 4352 x 1 slots (17 chunks) 10.4 / 8.2, 8192 x 2
-// of 128 experts 11.9 / 11.7, 5461 x 3 of 8 experts 11.4 / 9.9, 2048 x 8 of 128 experts 12.6 / 8.2, 16384 x 1 of 1024 21.5 / 18.7.
+// launch as slow as the three that it replaces from about 30 and 56 chunks on, and slower above.  From 25 and 49 on the counts are
+// kept in several copies, neighbouring lanes adding to different ones (at an odd pitch: the copies of a counter sit in different
+// banks), which are added up afterwards.  Three launches / one copy / copies in us, every slot on the first K experts: 16384 x 1
+// slots, 8 experts 10.5 / 18.0 / 9.1, 256 experts 12.5 / 18.4 / 9.7, 512 experts 14.7 / 18.5 / 12.4; 8192 x 2, 8 experts 10.6 / 11.4 / 9.1.
+// Evenly spread: 16384 x 1, 8 experts 11.3 / 8.6 / 9.1, 256 experts 19.3 / 8.5 / 9.6; 8192 x 2, 8 experts 11.3 / 8.6 / 9.1.  Outside
+// the line one copy is no slower than three launches however the load lies: collapsed, 4352 x 1 slots (17 chunks) 10.4 / 8.2, 6144 x 2 of
+// 8 experts (48 chunks) 10.5 / 9.6, 8192 x 2 of 128 experts 12.0 / 11.6, 5461 x 3 of 8 experts 11.4 / 9.9, 2048 x 8 of 128 experts
+// 12.7 / 8.2, 16384 x 1 of 1024 21.6 / 18.7.
 constexpr int kCountTable = MOE_MAX_EXPERTS + 16;        // eight copies of up to 129 counts, four of 257, two of 513
 static int direct_copies(int K, int E, int n_chunks) {
-  if (n_chunks <= 24 || !(K == 1 ? E <= 512 : K == 2 && E <= 64)) return 1;
+  if (!(K == 1 ? E <= 512 && n_chunks > 24 : K == 2 && E <= 64 && n_chunks > 48)) return 1;
   return E <= 128 ? 8 : E <= 256 ? 4 : 2;
 }
 
-template <bool SPREAD>
+template <int COPIES>
 __global__ __launch_bounds__(kChunk) void permute_direct_kernel(
-    const int32_t *__restrict__ ids, int TK, int E, int copies, int n_chunks, int tile_m, int max_tiles,
+    const int32_t *__restrict__ ids, int TK, int E, int n_chunks, int tile_m, int max_tiles,
     int32_t *__restrict__ sorted_slot, int32_t *__restrict__ expert_offsets, int32_t *__restrict__ slot_to_row,
     int32_t *__restrict__ tile_prefix, int32_t *__restrict__ tile_expert, int32_t *__restrict__ tile_desc,
     uint16_t *__restrict__ zero_rows, int row_len, const QuantJob ride) {
@@ -299,7 +300,7 @@ __global__ __launch_bounds__(kChunk) void permute_direct_kernel(
     int wave_sums[16];
     int wcount[NWV][MOE_MAX_EXPERTS];
   };
-  constexpr int kTable = SPREAD ? kCountTable : MOE_MAX_EXPERTS;
+  constexpr int kTable = COPIES > 1 ? kCountTable : MOE_MAX_EXPERTS;
   __shared__ int before[kTable], rest[kTable];
   __shared__ union { Place place; ListSmem lists; } sm;
   // the workgroup of the lists goes first: its chain is the longer one
@@ -313,9 +314,9 @@ __global__ __launch_bounds__(kChunk) void permute_direct_kernel(
     }
   }
   const int pitch = E | 1;
-  int *const my_before = before + (lane & (copies - 1)) * pitch, *const my_rest = rest + (lane & (copies - 1)) * pitch;
-  if constexpr (SPREAD) {
-    for (int i = E + tid; i < copies * pitch; i += kChunk) {
+  int *const my_before = before + (lane & (COPIES - 1)) * pitch, *const my_rest = rest + (lane & (COPIES - 1)) * pitch;
+  if constexpr (COPIES > 1) {
+    for (int i = E + tid; i < COPIES * pitch; i += kChunk) {
       before[i] = 0;
       rest[i] = 0;
     }
@@ -334,16 +335,17 @@ __global__ __launch_bounds__(kChunk) void permute_direct_kernel(
     for (int i = 0; i < B; i++) {
       if (i0 + i == c) v = id[i];
       if (id[i] >= 0 && id[i] < E) {
-        if constexpr (SPREAD) atomicAdd((i0 + i < c ? my_before : my_rest) + id[i], 1);
+        if constexpr (COPIES > 1) atomicAdd((i0 + i < c ? my_before : my_rest) + id[i], 1);
         else atomicAdd(i0 + i < c ? &before[id[i]] : &rest[id[i]], 1);
       }
     }
   }
   __syncthreads();
-  if constexpr (SPREAD) {
+  if constexpr (COPIES > 1) {
     for (int e = tid; e < E; e += kChunk) {
       int b = before[e], r = rest[e];
-      for (int i = 1; i < copies; i++) {
+#pragma unroll
+      for (int i = 1; i < COPIES; i++) {
         b += before[i * pitch + e];
         r += rest[i * pitch + e];
       }
@@ -442,7 +444,7 @@ int permute_quant_small_launch(hipStream_t st, const int32_t *ids, int T, int K,
 
 // zero_rows (may be null): a [T*K, row_len] bf16 tensor in slot order whose rows of slots WITHOUT an expert (id outside
 // [0, E)) are cleared here - the per-slot output form: nothing else ever writes those rows
-// counted: the routing launch has filled ws.chunk_counts and ws.arrivals is zero (more than kChunk slots only)
+// counted: the routing launch has filled ws.chunk_counts and ws.arrivals is zero (more than kDirectSlots slots only)
 // ride (may be null; more than kChunk slots only): activations quantised by extra workgroups of the launch (of the scan, if there are three)
 int permute_launch(hipStream_t st, const int32_t *ids, int T, int K, int E, int tile_m, int32_t *sorted_slot,
                    int32_t *expert_offsets, int32_t *slot_to_row, const PermuteWs &ws, uint16_t *zero_rows, int row_len,
@@ -456,10 +458,11 @@ int permute_launch(hipStream_t st, const int32_t *ids, int T, int K, int E, int 
   const QuantJob job = ride ? *ride : QuantJob{};
   if (!counted && TK <= kDirectSlots) {
     const int copies = direct_copies(K, E, ws.n_chunks);
-    const auto kernel = copies > 1 ? permute_direct_kernel<true> : permute_direct_kernel<false>;
+    const auto kernel = copies == 8 ? permute_direct_kernel<8> : copies == 4 ? permute_direct_kernel<4>
+                        : copies == 2 ? permute_direct_kernel<2> : permute_direct_kernel<1>;
     kernel<<<ws.n_chunks + 1 + job.blocks(), kChunk, 0, st>>>(
-        ids, TK, E, copies, ws.n_chunks, tile_m, ws.max_tiles, sorted_slot, expert_offsets, slot_to_row, ws.tile_prefix,
-        ws.tile_expert, ws.tile_desc, zero_rows, row_len, job);
+        ids, TK, E, ws.n_chunks, tile_m, ws.max_tiles, sorted_slot, expert_offsets, slot_to_row, ws.tile_prefix, ws.tile_expert,
+        ws.tile_desc, zero_rows, row_len, job);
     return (int)hipGetLastError();
   }
   if (!counted) permute_count_kernel<<<ws.n_chunks, 64, 0, st>>>(ids, TK, E, ws.chunk_counts, ws.arrivals);
