@@ -12,6 +12,8 @@ import ctypes
 import functools
 
 import torch
+from torch.jit import is_tracing
+from torch.overrides import has_torch_function
 
 from ._lib import MoeHipError, check, lib
 
@@ -284,9 +286,9 @@ _LAYER_MODES = {"softmax": ROUTE_SOFTMAX, "sigmoid": ROUTE_SIGMOID, "softmax_log
 _NOT_PLAIN = 1 << 20     # my_ops::_layer_fp8: not the form that it takes
 
 
-def _plain(*operands) -> bool:
+def _plain(operands) -> bool:
     """No operand is of a Tensor subclass, which may have its own idea of operators (a mode, e.g. a default device, is fine)."""
-    return (not torch.overrides.has_torch_function(operands)
+    return (not has_torch_function(operands)
             or all(t is None or type(t) in (torch.Tensor, torch.nn.Parameter) for t in operands))
 
 
@@ -304,11 +306,11 @@ def layer_fp8(x, router_weight, w13, w13_scale, w2, w2_scale, top_k: int, mode: 
     # The common form natively; any other, and what is wrong with one, below.  So is a call that Dynamo, export or the JIT's
     # tracer looks at: none of them can take an operator whose result is a status.
     if (workspace is not None and not (return_routing or static_scratch) and not torch.compiler.is_compiling()
-            and not torch.jit.is_tracing()):
+            and not is_tracing()):
         result = torch.empty(x.shape, dtype=torch.bfloat16, device=x.device) if out is None else out
         sh = (None, None, None, None) if shared is None else shared
         rc = _NOT_PLAIN
-        if _plain(x, router_weight, w13, w13_scale, w2, w2_scale, bias, *sh, result, workspace):
+        if _plain((x, router_weight, w13, w13_scale, w2, w2_scale, bias, *sh, result, workspace)):
             rc = torch.ops.my_ops._layer_fp8.default(x, router_weight, w13, w13_scale, w2, w2_scale, top_k, modes[mode], bias, n_groups,
                                                      topk_groups, bool(int(renorm)), float(scale), *sh, result, workspace)
         if rc != _NOT_PLAIN:
